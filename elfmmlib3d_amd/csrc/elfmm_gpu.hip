@@ -1641,17 +1641,31 @@ __global__ void k_pgather(int n, int nt, const int *__restrict__ iz, const int *
     }
 }
 
-constexpr int PN_THREADS = 256;     // points per workgroup (one per thread)
+constexpr int PN_THREADS = 256;     // lanes per workgroup
 constexpr int PN_TILE = 256;        // source records per LDS tile
-constexpr int PN_REC = 19;          // x y z, q[4], d[4][3]
+constexpr int PN_REC = 14;          // x y z, f[3], D xx xy xz yy yz zz, c2 tr D, pad
 
 // Near field of point sources: each point of a leaf (its sources, then its
 // targets) against the sources of the leaf's near boxes (self + list 1),
 // without the self pair (lfmm3dparthess_direct_self / _direct,
-// src/lfmm3dparthess.f:1150-1470), as potential, gradient and Hessian of
-// the four Laplace problems, phi = q/r + d.(x - y)/r^3, combined like the
-// far field into displacement and strain (9 values per point). Workgroup =
-// (near box, first point); the source records go through LDS in tiles.
+// src/lfmm3dparthess.f:1150-1470). A pair is evaluated as the elastic fields
+// themselves, not as the four Laplace problems the reference splits them
+// into: with R = x - y, f = sigma_sl / (2 mu), D = sym(sigma_dl x sigma_dv),
+// v = D R, c1 + c2 = 1,
+//   u      = R along + (2 - c1) f / r + 2 c2 v / r^3
+//   strain = I along + sym(R P) + 2 c2 D / r^3
+//   along  = (c1 f.R - c2 tr D + 3 c1 R.v / r^2) / r^3
+//   P      = -(3 (c1 f.R - c2 tr D) + 15 c1 R.v / r^2) R / r^5
+//            + (2 c1 - 2) f / r^3 + 6 (c1 - c2) v / r^5
+// about 80 operations a pair (both layers, strain) with 10 sums to hold,
+// against 290 and 40 for the Laplace fields. Bound by FP64 vector issue.
+// A point's sources are dealt to S lanes (a power of two, chosen per leaf by
+// point_chunks), added across them at the end; a workgroup takes PN_THREADS
+// consecutive (point, lane) pairs of one leaf, chunk = (near box, first
+// pair, S), and the source records go through LDS in tiles.
+// 1,000,000 points at iprec 2 (5.8e9 pairs): 53.4 ms as Laplace fields, 19.1
+// in this form (beside the far field); 3,704 points at iprec 1: 0.80 and 0.03.
+template <bool SL, bool DL, bool ST>
 __global__ __launch_bounds__(PN_THREADS) void k_pnear(int n, int src_eval, const int *__restrict__ nfb,
                                                      const int *__restrict__ nfs, const int *__restrict__ nfi,
                                                      const int *__restrict__ ss, const int *__restrict__ sc,
@@ -1661,72 +1675,119 @@ __global__ __launch_bounds__(PN_THREADS) void k_pnear(int n, int src_eval, const
                                                      const double *__restrict__ nodes, double c1,
                                                      double *__restrict__ nf)
 {
-    __shared__ double S[PN_TILE * PN_REC];
-    int q = chunks[2 * blockIdx.x], p0 = chunks[2 * blockIdx.x + 1];
+    __shared__ __align__(16) double S[PN_TILE * PN_REC];
+    int q = chunks[3 * blockIdx.x], l0 = chunks[3 * blockIdx.x + 1], split = chunks[3 * blockIdx.x + 2];
     int b = nfb[q];
     int nsb = src_eval ? sc[b] : 0;
-    int loc = p0 + (int)threadIdx.x;
+    int loc = (l0 + (int)threadIdx.x) / split, sub = (int)threadIdx.x & (split - 1);
     bool has = loc < nsb + tc[b];
     int ip = has ? (loc < nsb ? ss[b] + loc : n + ts[b] + (loc - nsb)) : -1;
     double x = has ? pts[3 * (size_t)ip] : 0.0, y = has ? pts[3 * (size_t)ip + 1] : 0.0,
            z = has ? pts[3 * (size_t)ip + 2] : 0.0;
-    double acc[40];
-#pragma unroll
-    for (int k = 0; k < 40; k++) acc[k] = 0.0;
+    const double c2 = 1.0 - c1;
+    double u0 = 0.0, u1 = 0.0, u2 = 0.0, al = 0.0;
+    double hxx = 0.0, hyy = 0.0, hzz = 0.0, hxy = 0.0, hxz = 0.0, hyz = 0.0;   // off-diagonal sums doubled
+    auto pair = [&](const double *r, bool self) {
+        double Rx = x - r[0], Ry = y - r[1], Rz = z - r[2];
+        double r2 = Rx * Rx + Ry * Ry + Rz * Rz;
+        // 1/sqrt(r2) from the hardware estimate and one third-order step
+        double i1 = __builtin_amdgcn_rsq(r2);
+        double e = fma(-r2 * i1, i1, 1.0);
+        i1 = fma(i1 * e, fma(0.375, e, 0.5), i1);
+        if (self) i1 = 0.0;
+        double i2 = i1 * i1, i3 = i1 * i2, i5 = i3 * i2;
+        double t = 0.0, w = 0.0, vx = 0.0, vy = 0.0, vz = 0.0;
+        if (SL) t = c1 * (r[3] * Rx + r[4] * Ry + r[5] * Rz);
+        if (DL) {
+            vx = r[6] * Rx + r[7] * Ry + r[8] * Rz;
+            vy = r[7] * Rx + r[9] * Ry + r[10] * Rz;
+            vz = r[8] * Rx + r[10] * Ry + r[11] * Rz;
+            w = (vx * Rx + vy * Ry + vz * Rz) * i2;
+            t -= r[12];
+        }
+        double along = i3 * (DL ? fma(3.0 * c1, w, t) : t);
+        u0 = fma(along, Rx, u0);
+        u1 = fma(along, Ry, u1);
+        u2 = fma(along, Rz, u2);
+        double g3 = 2.0 * c2 * i3;
+        if (SL) {
+            double g1 = (2.0 - c1) * i1;
+            u0 = fma(g1, r[3], u0);
+            u1 = fma(g1, r[4], u1);
+            u2 = fma(g1, r[5], u2);
+        }
+        if (DL) {
+            u0 = fma(g3, vx, u0);
+            u1 = fma(g3, vy, u1);
+            u2 = fma(g3, vz, u2);
+        }
+        if (ST) {
+            double ga = i5 * (DL ? fma(-15.0 * c1, w, -3.0 * t) : -3.0 * t);
+            double px = ga * Rx, py = ga * Ry, pz = ga * Rz;
+            if (SL) {
+                double a3 = -g3;                      // 2 c1 - 2 = -2 c2
+                px = fma(a3, r[3], px);
+                py = fma(a3, r[4], py);
+                pz = fma(a3, r[5], pz);
+            }
+            if (DL) {
+                double b5 = 6.0 * (c1 - c2) * i5;
+                px = fma(b5, vx, px);
+                py = fma(b5, vy, py);
+                pz = fma(b5, vz, pz);
+            }
+            al += along;
+            hxx = fma(Rx, px, hxx);
+            hyy = fma(Ry, py, hyy);
+            hzz = fma(Rz, pz, hzz);
+            hxy = fma(Rx, py, fma(Ry, px, hxy));
+            hxz = fma(Rx, pz, fma(Rz, px, hxz));
+            hyz = fma(Ry, pz, fma(Rz, py, hyz));
+            if (DL) {
+                double g6 = 2.0 * g3;
+                hxx = fma(g3, r[6], hxx);
+                hxy = fma(g6, r[7], hxy);
+                hxz = fma(g6, r[8], hxz);
+                hyy = fma(g3, r[9], hyy);
+                hyz = fma(g6, r[10], hyz);
+                hzz = fma(g3, r[11], hzz);
+            }
+        }
+    };
     for (int k = nfs[q]; k < nfs[q + 1]; k++) {
         int jb = nfi[k], j0 = ss[jb], cnt = sc[jb];
         for (int t0 = 0; t0 < cnt; t0 += PN_TILE) {
             int m = min(PN_TILE, cnt - t0);
             __syncthreads();                          // previous tile done
-            for (int e = threadIdx.x; e < m * PN_REC; e += PN_THREADS) {
-                int sj = e / PN_REC, c = e - sj * PN_REC;
-                S[e] = nodes[(size_t)(j0 + t0 + sj) * NODE_STRIDE + c];
+            for (int sj = threadIdx.x; sj < m; sj += PN_THREADS) {
+                const double *o = nodes + (size_t)(j0 + t0 + sj) * NODE_STRIDE;
+                double *d = S + sj * PN_REC;
+                for (int c = 0; c < 6; c++) d[c] = o[c];
+                d[6] = o[7];
+                d[7] = o[8];
+                d[8] = o[9];
+                d[9] = o[11];
+                d[10] = o[12];
+                d[11] = o[15];
+                d[12] = c2 * (o[7] + o[11] + o[15]);
             }
             __syncthreads();
             if (!has) continue;
-            for (int sj = 0; sj < m; sj++) {
-                if (j0 + t0 + sj == ip) continue;     // the self pair
-                const double *r = S + sj * PN_REC;
-                double Rx = x - r[0], Ry = y - r[1], Rz = z - r[2];
-                double ri = 1.0 / sqrt(Rx * Rx + Ry * Ry + Rz * Rz);
-                double ri2 = ri * ri, s3 = ri * ri2, s5 = s3 * ri2, s7 = s5 * ri2;
-                double xx = Rx * Rx, yy = Ry * Ry, zz = Rz * Rz, xy = Rx * Ry, xz = Rx * Rz, yz = Ry * Rz;
-#pragma unroll
-                for (int pr = 0; pr < 4; pr++) {
-                    double qv = r[3 + pr];
-                    const double *dv = r + 7 + 3 * pr;
-                    double dR = dv[0] * Rx + dv[1] * Ry + dv[2] * Rz;
-                    double *a = acc + 10 * pr;
-                    a[0] += qv * ri + dR * s3;
-                    double gr = -qv * s3 - 3.0 * dR * s5;     // coefficient of R in the gradient
-                    a[1] += gr * Rx + dv[0] * s3;
-                    a[2] += gr * Ry + dv[1] * s3;
-                    a[3] += gr * Rz + dv[2] * s3;
-                    double hq = 3.0 * qv * s5 + 15.0 * dR * s7;  // of R_a R_b
-                    double hd = -3.0 * s5;                      // of d_a R_b + d_b R_a
-                    a[4] += hq * xx + gr + 2.0 * hd * dv[0] * Rx;
-                    a[5] += hq * yy + gr + 2.0 * hd * dv[1] * Ry;
-                    a[6] += hq * zz + gr + 2.0 * hd * dv[2] * Rz;
-                    a[7] += hq * xy + hd * (dv[0] * Ry + dv[1] * Rx);
-                    a[8] += hq * xz + hd * (dv[0] * Rz + dv[2] * Rx);
-                    a[9] += hq * yz + hd * (dv[1] * Rz + dv[2] * Ry);
-                }
+            if (jb == b && src_eval) {                // the self pair is in this box
+                for (int sj = sub; sj < m; sj += split) pair(S + sj * PN_REC, j0 + t0 + sj == ip);
+            } else {
+                for (int sj = sub; sj < m; sj += split) pair(S + sj * PN_REC, false);
             }
         }
     }
-    if (!has) return;
-    double X[3] = {x, y, z}, u[3] = {0.0, 0.0, 0.0}, hm[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-    lap_to_elastic(acc, X, c1, u, hm);
-    double *g = nf + (size_t)ip * 9;
-    g[0] = u[0];
-    g[1] = u[1];
-    g[2] = u[2];
-    g[3] = hm[0][0];
-    g[4] = hm[1][1];
-    g[5] = hm[2][2];
-    g[6] = (hm[0][1] + hm[1][0]) / 2;
-    g[7] = (hm[0][2] + hm[2][0]) / 2;
-    g[8] = (hm[1][2] + hm[2][1]) / 2;
+    double g[9] = {u0, u1, u2, hxx + al, hyy + al, hzz + al, 0.5 * hxy, 0.5 * hxz, 0.5 * hyz};
+    for (int off = split >> 1; off > 0; off >>= 1)
+#pragma unroll
+        for (int c = 0; c < 9; c++) g[c] += __shfl_xor(g[c], off);
+    if (!has || sub) return;
+    double *o = nf + (size_t)ip * 9;
+#pragma unroll
+    for (int c = 0; c < 9; c++) o[c] = g[c];
 }
 
 // ------------------------------------------------------------------------
@@ -2788,6 +2849,36 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
     return 0;
 }
 
+// Workgroups of the point near field (k_pnear): (near box, first (point,
+// lane) pair, lanes per point). Lanes per point: at least as many as give
+// the device PN_WAVES waves (a small call has few points: at 3,704 points and
+// one lane each 58 waves would run 256 CUs), then per box up to four times
+// that, the one that leaves the fewest lanes of its last wave idle (195
+// points fill 3.05 waves at one lane each, 12.2 at four).
+std::vector<int> point_chunks(const Tree &T, const Plan &PL, int src_eval)
+{
+    constexpr int64_t PN_WAVES = 4096;               // 256 CUs x 4 SIMDs x 4
+    auto npts = [&](int b) { return (src_eval ? T.src_count[b] : 0) + T.tgt_count[b]; };
+    int64_t total = 0;
+    for (int b : PL.nf_boxes) total += npts(b);
+    int low = 1;
+    while (low < 64 && total * low < PN_WAVES * 64) low *= 2;
+    std::vector<int> chunks;
+    for (size_t q = 0; q < PL.nf_boxes.size(); q++) {
+        int64_t np = npts(PL.nf_boxes[q]);
+        int best = low;
+        auto waves = [&](int s) { return (double)((np * s + 63) / 64) / s; };   // lane-time of the box
+        for (int s = 2 * low; s <= std::min(64, 4 * low); s *= 2)
+            if (waves(s) < 0.95 * waves(best)) best = s;
+        for (int64_t l0 = 0; l0 < np * best; l0 += PN_THREADS) {
+            chunks.push_back((int)q);
+            chunks.push_back((int)l0);
+            chunks.push_back(best);
+        }
+    }
+    return chunks;
+}
+
 // The point-source apply (elfmm3dparttarg, src/elfmm3dpart.f:104-500):
 // the octree of the points with the particle FMM's leaf size, the far
 // field of the triangle apply with one node per point (k_pgather), the
@@ -2850,16 +2941,7 @@ int parttarg_dev(int iprec, double rlam, double rmu, int n, const double *d_src,
     build_plan(T, n, oc ? &oc->ops : nullptr, src_eval, false, NRHS, PL, false);
     plan_lk.unlock();
     for (int i = 0; i < 16; i++) g_stats[i] = PL.stats[i];
-    // near-field workgroups: (near box, first point), PN_THREADS points each
-    std::vector<int> chunks;
-    for (size_t q = 0; q < PL.nf_boxes.size(); q++) {
-        int b = PL.nf_boxes[q];
-        int npb = (src_eval ? T.src_count[b] : 0) + T.tgt_count[b];
-        for (int p0 = 0; p0 < npb; p0 += PN_THREADS) {
-            chunks.push_back((int)q);
-            chunks.push_back(p0);
-        }
-    }
+    const std::vector<int> chunks = point_chunks(T, PL, src_eval);
     Packer pk;
     PlanOffsets po;
     pack_plan(pk, T, PL, po);
@@ -2894,8 +2976,12 @@ int parttarg_dev(int iprec, double rlam, double rmu, int n, const double *d_src,
     hipStream_t ns = W.near_stream;
     HIPOK(hipEventRecord(W.ev_fork, stream));
     HIPOK(hipStreamWaitEvent(ns, W.ev_fork, 0));
-    if (!chunks.empty())
-        hipLaunchKernelGGL(k_pnear, dim3(chunks.size() / 2), dim3(PN_THREADS), 0, ns, n, src_eval, I(po.nfb),
+    bool strain = ifst || ifstt;
+    auto pnear = ifsl && ifdl ? (strain ? k_pnear<true, true, true> : k_pnear<true, true, false>)
+                 : ifdl       ? (strain ? k_pnear<false, true, true> : k_pnear<false, true, false>)
+                              : (strain ? k_pnear<true, false, true> : k_pnear<true, false, false>);
+    if (!chunks.empty() && (ifsl || ifdl))            // no layer: the near field stays zero
+        hipLaunchKernelGGL(pnear, dim3(chunks.size() / 3), dim3(PN_THREADS), 0, ns, n, src_eval, I(po.nfb),
                            I(po.nfs), I(po.nfi), I(po.ss), I(po.sc), I(po.ts), I(po.tc), I(o_ch),
                            W.pts.get<double>(), W.nodes.get<double>(), c1, W.nf.get<double>());
     HIPOK(hipGetLastError());
