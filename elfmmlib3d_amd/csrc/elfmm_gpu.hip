@@ -34,6 +34,7 @@
 #include "elfmm_internal.h"
 #include "elfmm_math.h"
 #include "elfmm_mindlin.h"
+#include "elfmm_near.h"
 #include "elfmm_octree.h"
 
 namespace elfmm {
@@ -1047,67 +1048,87 @@ __global__ __launch_bounds__(64 * EW_WAVES, 3) void k_m2t(int p, int nwt, const 
 
 
 // ------------------------------------------------------------------------
-// Near field: self + list 1 pair quadratures, one workgroup per leaf
+// Near field: self + list 1 pair quadratures, one wave per workgroup
 // ------------------------------------------------------------------------
 
 constexpr int NF_THREADS = 256;
 
-__global__ __launch_bounds__(NF_THREADS) void k_near(
+// Wave b takes lanes [l0, l0 + 64) of leaf q's (point, lane) pairs, (q, l0, split)
+// = tasks[3b..]: each point's near triangles (the lists of its boxes one after
+// another) are dealt to `split` lanes, a power of two chosen per leaf
+// (near_tasks), so every lane has a triangle in every step but the last. Up
+// to 64 boxes of the near list at a time: their first triangles and running
+// counts are scanned across the wave into LDS, and a lane finds the box of
+// its next triangle by walking those counts. Bound by FP64 vector issue (pair
+// code: elfmm_near.h). 81,920 triangles + 100,000 targets, iprec 2 (25.0e6
+// pairs, both layers, strain): 4.25 ms with two passes over the edges
+// and a 256-thread workgroup per leaf whose lanes idled in boxes of fewer
+// triangles than lanes per point, 1.23 ms in this form; 217 points against 180
+// triangles: 0.23 and 0.014 ms.
+template <bool SL, bool DL, bool ST>
+__global__ __launch_bounds__(64) void k_near(
     int n, int n_src_eval, const int *__restrict__ boxes, const int *__restrict__ lstart,
     const int *__restrict__ litems, const int *__restrict__ src_start,
     const int *__restrict__ src_count, const int *__restrict__ tgt_start,
-    const int *__restrict__ tgt_count, const double *__restrict__ pts,
-    const double *__restrict__ rec, double rlam, double rmu, double c1, int ifsl, int ifdl,
-    double *__restrict__ nf)
+    const int *__restrict__ tgt_count, const int *__restrict__ tasks, const double *__restrict__ pts,
+    const double *__restrict__ rec, double rlam, double rmu, double c1, double *__restrict__ nf)
 {
-    __shared__ double red[NF_THREADS][9];
-    int tbox = boxes[blockIdx.x];
+    __shared__ int pre[65], first[64];               // triangles before each box of the pass; its first triangle
+    int lane = threadIdx.x;
+    int q = tasks[3 * blockIdx.x], l0 = tasks[3 * blockIdx.x + 1], split = tasks[3 * blockIdx.x + 2];
+    int tbox = boxes[q];
     int ns_eval = n_src_eval ? src_count[tbox] : 0;
     int npts = ns_eval + tgt_count[tbox];
-    int b0 = lstart[blockIdx.x], b1 = lstart[blockIdx.x + 1];
-    for (int ip0 = 0; ip0 < npts; ip0 += NF_THREADS) {
-        int cnt = min(NF_THREADS, npts - ip0);
-        int tpp = max(1, NF_THREADS / cnt);
-        int ip = threadIdx.x / tpp, sub = threadIdx.x % tpp;
-        double acc[9];
+    int k = (l0 + lane) / split, sub = lane & (split - 1);
+    bool has = k < npts;
+    int selfidx = has && k < ns_eval ? src_start[tbox] + k : -1;
+    int gp = !has ? -1 : (k < ns_eval ? selfidx : n + tgt_start[tbox] + (k - ns_eval));
+    double P[3] = {0.0, 0.0, 0.0};
+    if (has)
+        for (int d = 0; d < 3; d++) P[d] = pts[3 * (size_t)gp + d];
+    double acc[9];
 #pragma unroll
-        for (int q = 0; q < 9; q++) acc[q] = 0.0;
-        int gp = -1, selfidx = -1;
-        if (ip < cnt) {
-            int k = ip0 + ip;
-            if (k < ns_eval) {
-                gp = src_start[tbox] + k;
-                selfidx = gp;
-            } else {
-                gp = n + tgt_start[tbox] + (k - ns_eval);
-            }
-            double P[3] = {pts[3 * (size_t)gp], pts[3 * (size_t)gp + 1], pts[3 * (size_t)gp + 2]};
-            // the point's triangles, concatenated over its near boxes, are
-            // dealt round-robin to its tpp lanes; every lane steps through
-            // its own share so the lanes of a wave stay converged
-            int j0 = sub;                   // position of this lane's next triangle in the current box
-            for (int bb = b0; bb < b1; bb++) {
-                int sbox = litems[bb];
-                int s0 = src_start[sbox], sn = src_count[sbox];
-                for (; j0 < sn; j0 += tpp) {
-                    int i = s0 + j0;
-                    nf_pair(rec + (size_t)i * NF_REC, P, i == selfidx, rlam, rmu, c1, ifsl, ifdl, acc);
-                }
-                j0 -= sn;
-            }
+    for (int c = 0; c < 9; c++) acc[c] = 0.0;
+    for (int b0 = lstart[q], b1 = lstart[q + 1]; b0 < b1; b0 += 64) {
+        int cnt = 0, s0 = 0;
+        if (b0 + lane < b1) {
+            int sbox = litems[b0 + lane];
+            s0 = src_start[sbox];
+            cnt = src_count[sbox];
         }
-#pragma unroll
-        for (int q = 0; q < 9; q++) red[threadIdx.x][q] = acc[q];
-        __syncthreads();
-        if (ip < cnt && sub == 0) {
-            for (int t = 1; t < tpp; t++)
-#pragma unroll
-                for (int q = 0; q < 9; q++) acc[q] += red[threadIdx.x + t][q];
-#pragma unroll
-            for (int q = 0; q < 9; q++) nf[(size_t)gp * 9 + q] = acc[q];
+        int end = cnt;
+        for (int off = 1; off < 64; off <<= 1) {
+            int v = __shfl_up(end, off);
+            if (lane >= off) end += v;
         }
+        __syncthreads();                              // the previous pass has been walked
+        if (lane == 0) pre[0] = 0;
+        pre[lane + 1] = end;
+        first[lane] = s0;
         __syncthreads();
+        int total = pre[64], bi = 0;
+        for (int t = has ? sub : total; t < total; t += split) {
+            while (t >= pre[bi + 1]) bi++;
+            int i = first[bi] + t - pre[bi];
+            near_pair<SL, DL, ST>(rec + (size_t)i * NF_REC, P, i == selfidx, rlam, rmu, c1, acc);
+        }
     }
+    constexpr int NO = ST ? 9 : 3;
+    for (int off = split >> 1; off > 0; off >>= 1)
+#pragma unroll
+        for (int c = 0; c < NO; c++) acc[c] += __shfl_xor(acc[c], off);
+    if (!has || sub) return;
+    const double sc = 0.5 / rmu;
+#pragma unroll
+    for (int c = 0; c < 9; c++) nf[(size_t)gp * 9 + c] = sc * acc[c];
+}
+
+// The variant for the layers and outputs of a call.
+inline auto near_kernel(bool sl, bool dl, bool strain)
+{
+    return sl && dl ? (strain ? k_near<true, true, true> : k_near<true, true, false>)
+           : dl     ? (strain ? k_near<false, true, true> : k_near<false, true, false>)
+                    : (strain ? k_near<true, false, true> : k_near<true, false, false>);
 }
 
 // Stored near-field interactions (iter mode). For near box q with npts
@@ -2072,7 +2093,7 @@ int max_lds()
 // Offsets of the arrays of a tree and its plan in one packed device buffer.
 struct PlanOffsets {
     size_t iz, izt, cen, side, ss, sc, ts, tc, p2m, p2lb, p2ls, p2li, l2t, l2tp, m2tsb, m2tp, l2tw, m2tw, m2tbt;
-    size_t nfb, nfs, nfi, m2lt;
+    size_t nfb, nfs, nfi, nfw, m2lt;
     std::vector<LaunchOff> m2m, l2l;
     LaunchOff m2l;
 };
@@ -2101,6 +2122,7 @@ void pack_plan(Packer &pk, const Tree &T, const Plan &PL, PlanOffsets &o)
     o.nfb = pk.add(PL.nf_boxes);
     o.nfs = pk.add(PL.nf_start);
     o.nfi = pk.add(PL.nf_items);
+    o.nfw = pk.add(PL.nf_tasks);
     auto add_launch = [&](const GemmLaunch &g) {
         LaunchOff l;
         l.tiles = pk.add(g.tiles);
@@ -2547,7 +2569,7 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
     // ---- upload plan
     Packer pk;
     PlanOffsets po;
-    size_t o_iz, o_izt, o_ss, o_sc, o_ts, o_tc, o_nfb, o_nfs, o_nfi;
+    size_t o_iz, o_izt, o_ss, o_sc, o_ts, o_tc, o_nfb, o_nfs, o_nfi, o_nfw;
     if (split) {
         // what the gather, the near field and the assembly read; the far
         // field gets its own buffer once its lists exist
@@ -2560,10 +2582,11 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
         o_nfb = pk.add(PL.nf_boxes);
         o_nfs = pk.add(PL.nf_start);
         o_nfi = pk.add(PL.nf_items);
+        o_nfw = pk.add(PL.nf_tasks);
     } else {
         pack_plan(pk, T, PL, po);
         o_iz = po.iz, o_izt = po.izt, o_ss = po.ss, o_sc = po.sc, o_ts = po.ts, o_tc = po.tc;
-        o_nfb = po.nfb, o_nfs = po.nfs, o_nfi = po.nfi;
+        o_nfb = po.nfb, o_nfs = po.nfs, o_nfi = po.nfi, o_nfw = po.nfw;
     }
     size_t o_sbase = pk.add(nf_sbase), o_ntri = pk.add(nf_ntri), o_pst = pk.add(nf_pstart);
     size_t o_nfc = pk.add(nf_chunk);
@@ -2713,11 +2736,10 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
                            W.nf.get<double>());
     } else if (!nf_boxes.empty() && store && icomp == 3) {
         HIPOK(nrhs > 1 ? run_replay_multi(ns) : run_replay(ns));
-    } else if (!nf_boxes.empty()) {
-        hipLaunchKernelGGL(k_near, dim3(nf_boxes.size()), dim3(NF_THREADS), 0, ns, n, src_eval,
-                           I(o_nfb), I(o_nfs), I(o_nfi), I(o_ss), I(o_sc), I(o_ts), I(o_tc),
-                           W.pts.get<double>(), W.rec.get<double>(), rlam, rmu, c1, ifsl, ifdl,
-                           W.nf.get<double>());
+    } else if (!PL.nf_tasks.empty() && (ifsl || ifdl)) {   // no layer: the near field stays zero
+        hipLaunchKernelGGL(near_kernel(ifsl, ifdl, ifst || ifstt), dim3(PL.nf_tasks.size() / 3), dim3(64), 0, ns, n,
+                           src_eval, I(o_nfb), I(o_nfs), I(o_nfi), I(o_ss), I(o_sc), I(o_ts), I(o_tc), I(o_nfw),
+                           W.pts.get<double>(), W.rec.get<double>(), rlam, rmu, c1, W.nf.get<double>());
     }
     HIPOK(hipGetLastError());
     ev_end(9, ns);
@@ -3619,12 +3641,12 @@ void batch_enqueue_view(Batch &B, const BatchView &V, Lane &f, Lane &q)
              B.ifdl, B.ifdl ? (const double *)(B.sdl + 3 * V.off) : none,
              nt ? (const double *)(B.tgt + 3 * V.offt) : none, tri_s, nrm_s, ssl_s, sdl_s, V.pts, V.rec);
     f.fill0(V.nf, (size_t)np * 9);
-    bool near = !V.PL->nf_boxes.empty();
+    bool near = !V.PL->nf_tasks.empty() && (B.ifsl || B.ifdl);
     if (near) {
         q.after(f);
-        q.launch(k_near, dim3(V.PL->nf_boxes.size()), dim3(NF_THREADS), 0, n, B.src_eval, I(po.nfb), I(po.nfs),
-                 I(po.nfi), I(po.ss), I(po.sc), I(po.ts), I(po.tc), (const double *)V.pts, (const double *)V.rec,
-                 B.rlam, B.rmu, c1, B.ifsl, B.ifdl, V.nf);
+        q.launch(near_kernel(B.ifsl, B.ifdl, B.ifst || B.ifstt), dim3(V.PL->nf_tasks.size() / 3), dim3(64), 0, n,
+                 B.src_eval, I(po.nfb), I(po.nfs), I(po.nfi), I(po.ss), I(po.sc), I(po.ts), I(po.tc), I(po.nfw),
+                 (const double *)V.pts, (const double *)V.rec, B.rlam, B.rmu, c1, V.nf);
     }
     if (V.usefar) {
         FarLaunch fl{B.ds, B.oc, V.PL, V.po, P, B.iprec, n, V.nb, tri_s, nrm_s, ssl_s, sdl_s, B.ifsl, B.ifdl,

@@ -139,6 +139,7 @@ struct Plan {
     std::vector<int> p2l_boxes, p2l_start, p2l_items;   // box <- sources of its list-4 boxes
     std::vector<int> m2t_boxes, m2t_start, m2t_items;   // box <- multipoles of its list-3 boxes
     std::vector<int> l2t_boxes, nf_boxes, nf_start, nf_items;
+    std::vector<int> nf_tasks;                       // near-field waves: (near box, first lane, lanes per point)
     std::vector<int> l2t_tpt;                        // points of each l2t slot, slot after slot
     std::vector<int> m2t_slot_box, m2t_tpt;          // points of each m2t slot, slot after slot
     // evaluation wave tasks: (slot, first task, task count <= EW_PTS) triples

@@ -63,7 +63,8 @@ namespace elfmm {
 //   [12..14] a, b, c: local vertices (0,0), (a,0), (b,c)
 //   [15..17] single-layer density in the local frame
 //   [18..20] double-layer density in the local frame
-//   [21..23] padding
+//   [21..22] inverse lengths of the second and third edge
+//   [23]     padding
 constexpr int NF_REC = 24;
 
 // Frame of the reference's rotshift3d (src/trilib.f:453-533).
@@ -99,7 +100,11 @@ ELFMM_HD void nf_make_record(const double *tri, const double *ssl, const double 
         rec[15 + j] = ssl ? e[0] * ssl[0] + e[1] * ssl[1] + e[2] * ssl[2] : 0.0;
         rec[18 + j] = sdl ? e[0] * sdl[0] + e[1] * sdl[1] + e[2] * sdl[2] : 0.0;
     }
-    rec[21] = rec[22] = rec[23] = 0.0;
+    // inverse lengths of the edges (a,0)-(b,c) and (b,c)-(0,0)
+    double ex = rec[13] - rec[12];
+    rec[21] = 1.0 / sqrt(ex * ex + rec[14] * rec[14]);
+    rec[22] = 1.0 / sqrt(rec[13] * rec[13] + rec[14] * rec[14]);
+    rec[23] = 0.0;
 }
 
 struct EdgePrims {

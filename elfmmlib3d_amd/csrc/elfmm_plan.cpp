@@ -140,6 +140,34 @@ void wave_tasks(const std::vector<I> &off, std::vector<int> &wt)
         }
 }
 
+// Waves of the near field: lanes per point of each near box, the power of two
+// that costs the box the least time, waves x (steps per wave + 1): the last
+// step and the last wave of a box run partly idle, and setting a wave up and
+// adding its lanes costs about a step (20 points, 135 triangles: 2 waves x 35
+// at 4 lanes, 3 x 18 at 8, 5 x 10 at 16, 10 x 6 at 32). A call too small to
+// give the device NF_WAVES waves that way starts from more lanes per point:
+// 217 points against 180 triangles took 205 us as one workgroup per leaf.
+template <class NP>
+void near_tasks(Plan &P, const std::vector<int> &ntri, NP &&npts, double npt)
+{
+    constexpr int NF_WAVES = 2048;                   // 256 CUs x 4 SIMDs x 2
+    int low = 1;
+    while (low < 64 && npt * low < NF_WAVES * 64.0) low *= 2;
+    P.nf_tasks.clear();
+    for (size_t q = 0; q < P.nf_boxes.size(); q++) {
+        int64_t np = npts(P.nf_boxes[q]), best = 0, cost = 0;
+        for (int64_t s = low; s <= 64; s *= 2) {
+            int64_t c = (np * s + 63) / 64 * ((ntri[q] + s - 1) / s + 1);
+            if (!best || c < cost) best = s, cost = c;
+        }
+        for (int64_t l0 = 0; l0 < np * best; l0 += 64) {
+            P.nf_tasks.push_back((int)q);
+            P.nf_tasks.push_back((int)l0);
+            P.nf_tasks.push_back((int)best);
+        }
+    }
+}
+
 }  // namespace
 
 void build_plan_near(const Tree &T, bool src_eval, bool direct_only, bool iter, Plan &P)
@@ -203,13 +231,15 @@ void build_plan_near(const Tree &T, bool src_eval, bool direct_only, bool iter, 
         P.nf_items.swap(it);
     }
     if (direct_only) P.nf_boxes.clear();
-    double npair_near = 0;
+    double npair_near = 0, npt_near = 0;
+    std::vector<int> ntri(P.nf_boxes.size(), 0);
     for (size_t q = 0; q < P.nf_boxes.size(); q++) {
-        double ns = 0;
-        for (int k = P.nf_start[q]; k < P.nf_start[q + 1]; k++) ns += T.src_count[P.nf_items[k]];
-        npair_near += npts(P.nf_boxes[q]) * ns;
+        for (int k = P.nf_start[q]; k < P.nf_start[q + 1]; k++) ntri[q] += T.src_count[P.nf_items[k]];
+        npair_near += (double)npts(P.nf_boxes[q]) * ntri[q];
+        npt_near += npts(P.nf_boxes[q]);
     }
     P.stats[6] = npair_near;
+    near_tasks(P, ntri, npts, npt_near);
 }
 
 void plan_reset(Plan &P)
