@@ -108,10 +108,13 @@ struct HipFailure {
     hipError_t err;
 };
 
-__device__ __forceinline__ int hidx(int l, int m) { return l * (l + 1) / 2 + m; }
-
 // accumulator of one v_mfma_f64_16x16x4f64 (four doubles per lane)
 typedef double gemm_d4 __attribute__((ext_vector_type(4)));
+
+#include "elfmm_moments.h"
+
+__device__ __forceinline__ int hidx(int l, int m) { return l * (l + 1) / 2 + m; }
+
 
 // order m of packed coefficient index c = l*(l+1)/2 + m (c < 2^20), from
 // a float square root and one correction each way: no table load
@@ -121,15 +124,6 @@ __device__ __forceinline__ int coef_m(int c)
     if ((l + 1) * (l + 2) / 2 <= c) l++;
     if (l * (l + 1) / 2 > c) l--;
     return c - l * (l + 1) / 2;
-}
-
-// degree and order of packed coefficient index c = l*(l+1)/2 + m
-__device__ __forceinline__ void coef_nk(int c, int &n, int &k)
-{
-    n = (int)((sqrt(8.0 * c + 1.0) - 1.0) * 0.5);
-    while ((n + 1) * (n + 2) / 2 <= c) n++;
-    while (n * (n + 1) / 2 > c) n--;
-    k = c - n * (n + 1) / 2;
 }
 
 
@@ -284,15 +278,6 @@ __global__ void k_nodes(int n, int nq, int q0, const double *__restrict__ tri_s,
 // ------------------------------------------------------------------------
 // P2M and P2L: quadrature nodes -> expansion, one workgroup per box
 // ------------------------------------------------------------------------
-
-// 1/sqrt((l+m)! (l-m)!): the factor between the integer-coefficient
-// harmonics V below and the normalised R_l^m / I_l^m.
-__device__ __forceinline__ double hnorm(int l, int m)
-{
-    m = m < 0 ? -m : m;
-    return 1.0 / sqrt(g_fact[l + m] * g_fact[l - m]);
-}
-
 
 // Column m of the unnormalised harmonics of one point, stored in stream
 // order: V_l^m at doubles 2*pos and 2*pos + 1, pos = m*(ph+1) - m*(m-1)/2
@@ -490,7 +475,7 @@ __device__ __forceinline__ void p2x_body(
             int ld = IRR ? l + 1 : l - 1;
             double fh = hnorm(l, m) * f0s, fp, fm, fz;
             if (!IRR) {
-                bool vp = ld >= 0 && m + 1 <= ld, vm = ld >= 0 && m - 1 <= ld, vz = ld >= 0 && m <= ld;
+                bool vp = ld >= 0 && m + 1 <= ld, vm = ld >= 0 && m - 1 <= ld && m + ld > 0, vz = ld >= 0 && m <= ld;
                 fp = vp ? sqrt((double)((l - m) * (l - m - 1))) * hnorm(ld, m + 1) : 0.0;
                 fm = vm ? sqrt((double)((l + m) * (l + m - 1))) * hnorm(ld, m - 1) : 0.0;
                 fz = vz ? sqrt((double)((l - m) * (l + m))) * hnorm(ld, m) : 0.0;
@@ -547,6 +532,30 @@ __global__ __launch_bounds__(64 * WB, TW <= 7 ? 4 : 2) void k_p2l(
 }
 
 
+
+// P2M and P2L of triangles through their moments (elfmm_moments.h)
+template <class Z>
+__global__ __launch_bounds__(Z::NT, 2) void k_p2m_tri(
+    int p, const int *__restrict__ boxes, const double *__restrict__ centers, const double *__restrict__ sides,
+    const int *__restrict__ src_start, const int *__restrict__ src_count, const double *__restrict__ tri_s,
+    const double *__restrict__ tcoef, int nc, double *__restrict__ expn)
+{
+    extern __shared__ double lds[];                  // no static LDS beside it: it starts at 0
+    p2t_body<false, Z>(p, boxes, nullptr, nullptr, centers, sides, src_start, src_count, tri_s, tcoef, nc, expn,
+                       lds);
+}
+
+template <class Z>
+__global__ __launch_bounds__(Z::NT, 2) void k_p2l_tri(
+    int p, const int *__restrict__ boxes, const int *__restrict__ lstart, const int *__restrict__ litems,
+    const double *__restrict__ centers, const double *__restrict__ sides, const int *__restrict__ src_start,
+    const int *__restrict__ src_count, const double *__restrict__ tri_s, const double *__restrict__ tcoef, int nc,
+    double *__restrict__ expn)
+{
+    extern __shared__ double lds[];                  // no static LDS beside it: it starts at 0
+    p2t_body<true, Z>(p, boxes, lstart, litems, centers, sides, src_start, src_count, tri_s, tcoef, nc, expn,
+                      lds);
+}
 
 // ------------------------------------------------------------------------
 // Translations (M2L, M2M, L2L): gather columns, multiply, scatter-add
@@ -1863,6 +1872,7 @@ constexpr int NPHASE = 12;
 struct DeviceState {
     bool tables = false;
     bool p2x_wide = false;                           // 16-wave P2M/P2L for orders above 26
+    bool p2t = false;                                // P2M/P2L through triangle moments (156 KB of LDS per CU)
     std::map<int, std::unique_ptr<OpsCache>> ops;   // by iprec
 };
 
@@ -1899,7 +1909,18 @@ DeviceState &device_state()
                 hipSuccess &&
             hipFuncSetAttribute((const void *)k_p2l<16, 7, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, wide) ==
                 hipSuccess;
-        (void)hipGetLastError();                     // a refused size leaves the narrow shape in use
+        auto lds_ok = [](auto z) {
+            using Z = decltype(z);
+            int ph = 0;
+            while (Z::fits(ph + 1)) ph++;
+            int b = Z::lds(ph) * 8;
+            return hipFuncSetAttribute((const void *)k_p2m_tri<Z>, hipFuncAttributeMaxDynamicSharedMemorySize, b) ==
+                       hipSuccess &&
+                   hipFuncSetAttribute((const void *)k_p2l_tri<Z>, hipFuncAttributeMaxDynamicSharedMemorySize, b) ==
+                       hipSuccess;
+        };
+        ds->p2t = lds_ok(P2TShape0{}) && lds_ok(P2TShape1{}) && lds_ok(P2TShape2{}) && lds_ok(P2TShape3{});
+        (void)hipGetLastError();                     // a refused size leaves the narrow shape, or the node products, in use
         ds->tables = true;
     }
     return *ds;
@@ -2163,7 +2184,7 @@ void far_scratch(int iprec, int n, int np, int nb, int p, size_t &nodes, size_t 
 {
     int nq, q0;
     quad_rule(iprec, nq, q0);
-    nodes = (size_t)n * nq * NODE_STRIDE;
+    nodes = (size_t)n * nq * NODE_STRIDE;            // or 48 coefficients per triangle (k_tcoef), nq >= 6
     exps = (size_t)2 * nb * NRHS * ncoef(p);
     lap = (size_t)np * 40;
 }
@@ -2189,9 +2210,26 @@ void enqueue_far(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
     mark(2, true);
     ln.fill0(a.exps, (size_t)2 * a.nb * NRHS * nc);
     ln.fill0(a.lap, np * 40);
-    if (!a.points)
+    // triangles with 6 or 12 nodes go through three moments each, where the
+    // device gives the LDS that takes; rules of 1 and 3 nodes and point sources
+    // through one product per node
+    const bool tri = !a.points && a.ds->p2t && p2t_shape(p, nq) >= 0 && p2t_shape(p + 1, nq) >= 0;
+    if (tri)
+        ln.launch(k_tcoef, dim3((n + 255) / 256), dim3(256), 0, n, a.tri_s, a.nrm_s, a.ssl, a.sdl, a.ifsl, a.ifdl,
+                  a.mu, a.c1, a.c2, a.dls, a.nodes);
+    else if (!a.points)
         ln.launch(k_nodes, dim3((nq * n + 255) / 256), dim3(256), 0, n, nq, q0, a.tri_s, a.nrm_s, a.ssl, a.sdl,
                   a.ifsl, a.ifdl, a.mu, a.c1, a.c2, a.dls, a.nodes);
+    auto p2t = [&](auto z, bool irr, size_t nbx, const int *bx, const int *ls, const int *li, double *out) {
+        using Z = decltype(z);
+        size_t sh = (size_t)Z::lds(irr ? p + 1 : p) * 8;
+        if (irr)
+            ln.launch(k_p2l_tri<Z>, dim3(nbx), dim3(Z::NT), sh, p, bx, ls, li, D(o.cen), D(o.side), I(o.ss), I(o.sc),
+                      a.tri_s, (const double *)a.nodes, nc, out);
+        else
+            ln.launch(k_p2m_tri<Z>, dim3(nbx), dim3(Z::NT), sh, p, bx, D(o.cen), D(o.side), I(o.ss), I(o.sc), a.tri_s,
+                      (const double *)a.nodes, nc, out);
+    };
     // P2M / P2L: moments on the matrix cores (shapes at P2X_WIDE_STRIDE)
     auto p2x = [&](bool irr, size_t nbx, const int *bx, const int *ls, const int *li, double *out) {
         int ph = irr ? p + 1 : p;
@@ -2208,7 +2246,16 @@ void enqueue_far(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
         ln.launch(kern, dim3(nbx), dim3(64 * wb), sh, p, nq, stride, bx, ls, li, D(o.cen), D(o.side), I(o.ss),
                   I(o.sc), (const double *)a.nodes, nc, out);
     };
-    if (!PL.p2m_boxes.empty()) p2x(false, PL.p2m_boxes.size(), I(o.p2m), nullptr, nullptr, mp);
+    auto p2 = [&](bool irr, size_t nbx, const int *bx, const int *ls, const int *li, double *out) {
+        switch (tri ? p2t_shape(irr ? p + 1 : p, nq) : -1) {
+        case 0: return p2t(P2TShape0{}, irr, nbx, bx, ls, li, out);
+        case 1: return p2t(P2TShape1{}, irr, nbx, bx, ls, li, out);
+        case 2: return p2t(P2TShape2{}, irr, nbx, bx, ls, li, out);
+        case 3: return p2t(P2TShape3{}, irr, nbx, bx, ls, li, out);
+        default: return p2x(irr, nbx, bx, ls, li, out);
+        }
+    };
+    if (!PL.p2m_boxes.empty()) p2(false, PL.p2m_boxes.size(), I(o.p2m), nullptr, nullptr, mp);
     mark(2, false);
     // M2M / L2L: rotated translations, the kernel of M2L (unit scale)
     auto run_trans = [&](const GemmLaunch &g, const LaunchOff &lo_, const double *A, const double *X, double *Y) {
@@ -2229,7 +2276,7 @@ void enqueue_far(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
     }
     mark(4, false);
     mark(5, true);
-    if (!PL.p2l_boxes.empty()) p2x(true, PL.p2l_boxes.size(), I(o.p2lb), I(o.p2ls), I(o.p2li), lo);
+    if (!PL.p2l_boxes.empty()) p2(true, PL.p2l_boxes.size(), I(o.p2lb), I(o.p2ls), I(o.p2li), lo);
     mark(5, false);
     mark(6, true);
     for (size_t k = 0; k < PL.l2l_l.size(); k++) run_trans(PL.l2l_l[k], o.l2l[k], (const double *)oc.l2l.p, lo, lo);
