@@ -2020,14 +2020,16 @@ struct MindScratch {
 // stream) run concurrently: host planning of one overlaps device work of
 // the others.
 struct Workspace {
-    DevBuf plan, plan2, inp, exps, pts, lap, nf, nodes, rec;   // plan2: far-field lists of a split plan
+    DevBuf plan, inp, exps, pts, lap, nf, nodes, rec;
+    DevBuf part[3];                                  // far-field lists of a plan sent in parts
     DevBuf tgtm, htmp, hq;                           // half space: mirrored targets, icomp-1 pairs, queue
     MindScratch mind[SET_LANES];                     // Mindlin far field, one per set lane
     DevBuf dmulti, nfm;                           // several density sets: densities, near fields
     std::vector<double> hsrc, htgt;
     std::unique_ptr<OctreeWork> oct;                 // device octree buffers
     Plan planh;
-    PinnedBuf stage, stage2;   // plan staging; the call that filled them has completed before reuse
+    Tree treeh;
+    PinnedBuf stage, part_stage[3];   // plan staging; the call that filled them has completed before reuse
     hipStream_t near_stream = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_done = nullptr;
     hipEvent_t ev[2 * NPHASE] = {};
@@ -2111,7 +2113,8 @@ int max_lds()
     return v;
 }
 
-// Offsets of the arrays of a tree and its plan in one packed device buffer.
+// Offsets of the arrays of a tree and its plan, each in the packed device
+// buffer of its part (FarLaunch), which may be one and the same.
 struct PlanOffsets {
     size_t iz, izt, cen, side, ss, sc, ts, tc, p2m, p2lb, p2ls, p2li, l2t, l2tp, m2tsb, m2tp, l2tw, m2tw, m2tbt;
     size_t nfb, nfs, nfi, nfw, m2lt;
@@ -2119,20 +2122,55 @@ struct PlanOffsets {
     LaunchOff m2l;
 };
 
-void pack_plan(Packer &pk, const Tree &T, const Plan &PL, PlanOffsets &o)
+// Points and near field: what the gather, the near field and the assembly
+// read, and the boxes' sources.
+void pack_near(Packer &pk, const Tree &T, const Plan &PL, PlanOffsets &o)
 {
     o.iz = pk.add(T.iz);
     o.izt = pk.add(T.iztarg);
-    o.cen = pk.add(T.centers);
-    o.side = pk.add(PL.sides);
     o.ss = pk.add(T.src_start);
     o.sc = pk.add(T.src_count);
     o.ts = pk.add(T.tgt_start);
     o.tc = pk.add(T.tgt_count);
+    o.nfb = pk.add(PL.nf_boxes);
+    o.nfs = pk.add(PL.nf_start);
+    o.nfi = pk.add(PL.nf_items);
+    o.nfw = pk.add(PL.nf_tasks);
+}
+
+LaunchOff pack_launch(Packer &pk, const GemmLaunch &g)
+{
+    LaunchOff l;
+    l.tiles = pk.add(g.tiles);
+    l.src = pk.add(g.src);
+    l.dst = pk.add(g.dst);
+    l.sc = pk.add(g.scale);
+    return l;
+}
+
+// The three parts of the far-field lists (build_plan_up, _m2l, _eval)
+void pack_up(Packer &pk, const Tree &T, const Plan &PL, PlanOffsets &o)
+{
+    o.cen = pk.add(T.centers);
+    o.side = pk.add(PL.sides);
     o.p2m = pk.add(PL.p2m_boxes);
     o.p2lb = pk.add(PL.p2l_boxes);
     o.p2ls = pk.add(PL.p2l_start);
     o.p2li = pk.add(PL.p2l_items);
+    o.m2m.clear();
+    for (auto &g : PL.m2m_l) o.m2m.push_back(pack_launch(pk, g));
+}
+
+void pack_m2l(Packer &pk, const Plan &PL, PlanOffsets &o)
+{
+    o.l2l.clear();
+    for (auto &g : PL.l2l_l) o.l2l.push_back(pack_launch(pk, g));
+    o.m2l = pack_launch(pk, PL.m2l);
+    o.m2lt = pk.add(PL.m2l_tiles);
+}
+
+void pack_eval(Packer &pk, const Plan &PL, PlanOffsets &o)
+{
     o.l2t = pk.add(PL.l2t_boxes);
     o.l2tp = pk.add(PL.l2t_tpt);
     o.m2tsb = pk.add(PL.m2t_slot_box);
@@ -2140,24 +2178,14 @@ void pack_plan(Packer &pk, const Tree &T, const Plan &PL, PlanOffsets &o)
     o.l2tw = pk.add(PL.l2t_wt);
     o.m2tw = pk.add(PL.m2t_wt);
     o.m2tbt = pk.add(PL.m2t_bt);
-    o.nfb = pk.add(PL.nf_boxes);
-    o.nfs = pk.add(PL.nf_start);
-    o.nfi = pk.add(PL.nf_items);
-    o.nfw = pk.add(PL.nf_tasks);
-    auto add_launch = [&](const GemmLaunch &g) {
-        LaunchOff l;
-        l.tiles = pk.add(g.tiles);
-        l.src = pk.add(g.src);
-        l.dst = pk.add(g.dst);
-        l.sc = pk.add(g.scale);
-        return l;
-    };
-    o.m2m.clear();
-    o.l2l.clear();
-    for (auto &g : PL.m2m_l) o.m2m.push_back(add_launch(g));
-    for (auto &g : PL.l2l_l) o.l2l.push_back(add_launch(g));
-    o.m2l = add_launch(PL.m2l);
-    o.m2lt = pk.add(PL.m2l_tiles);
+}
+
+void pack_plan(Packer &pk, const Tree &T, const Plan &PL, PlanOffsets &o)
+{
+    pack_near(pk, T, PL, o);
+    pack_up(pk, T, PL, o);
+    pack_m2l(pk, PL, o);
+    pack_eval(pk, PL, o);
 }
 
 // One far field of the free-space (or anti-image) FMM: the four Laplace
@@ -2168,7 +2196,9 @@ struct FarLaunch {
     const OpsCache *oc;
     const Plan *PL;
     const PlanOffsets *o;
-    const char *P;                                   // the packed plan on the device
+    // the packed plan on the device: points and near field, then the parts of
+    // the far field
+    const char *P, *PU, *PM, *PE;
     int iprec, n, nb;
     const double *tri_s, *nrm_s, *ssl, *sdl;         // tree order
     int ifsl, ifdl;
@@ -2193,15 +2223,27 @@ void far_scratch(int iprec, int n, int np, int nb, int p, size_t &nodes, size_t 
 // memsets, copies or host waits), so that it can be captured into a graph.
 // mark(k, begin), when given, brackets phase k (2 nodes and P2M, 3 M2M, 4
 // M2L, 5 P2L, 6 L2L, 7 L2T, 8 M2T) for the caller's timing events.
+// M2M / L2L of one level: rotated translations, the kernel of M2L (unit scale)
+void enqueue_trans(const GemmLaunch &g, const LaunchOff &l, const char *P, const DevBuf &A, const double *X, double *Y,
+                   int nc, Lane &ln)
+{
+    if (g.tiles.empty()) return;
+    int ntiles = (int)g.tiles.size();
+    ln.launch(k_m2m_l2l, dim3(ntiles), dim3(ML_THREADS), 0, (const M2LTile *)(P + l.tiles), ntiles,
+              (const double *)A.p, (const int *)(P + l.src), (const int *)(P + l.dst), (const double *)(P + l.sc), X,
+              Y, nc);
+}
+
+// P2M, M2M and P2L (build_plan_up)
 template <class Mark>
-void enqueue_far(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
+void enqueue_up(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
 {
     const Plan &PL = *a.PL;
     const PlanOffsets &o = *a.o;
     const OpsCache &oc = *a.oc;
-    const char *P = a.P;
-    auto I = [&](size_t off) { return (const int *)(P + off); };
-    auto D = [&](size_t off) { return (const double *)(P + off); };
+    const int *ss = (const int *)(a.P + o.ss), *sc = (const int *)(a.P + o.sc);
+    auto I = [&](size_t off) { return (const int *)(a.PU + off); };
+    auto D = [&](size_t off) { return (const double *)(a.PU + off); };
     const int p = oc.p, nc = ncoef(p), n = a.n;
     int nq, q0;
     quad_rule(a.iprec, nq, q0);
@@ -2224,10 +2266,10 @@ void enqueue_far(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
         using Z = decltype(z);
         size_t sh = (size_t)Z::lds(irr ? p + 1 : p) * 8;
         if (irr)
-            ln.launch(k_p2l_tri<Z>, dim3(nbx), dim3(Z::NT), sh, p, bx, ls, li, D(o.cen), D(o.side), I(o.ss), I(o.sc),
+            ln.launch(k_p2l_tri<Z>, dim3(nbx), dim3(Z::NT), sh, p, bx, ls, li, D(o.cen), D(o.side), ss, sc,
                       a.tri_s, (const double *)a.nodes, nc, out);
         else
-            ln.launch(k_p2m_tri<Z>, dim3(nbx), dim3(Z::NT), sh, p, bx, D(o.cen), D(o.side), I(o.ss), I(o.sc), a.tri_s,
+            ln.launch(k_p2m_tri<Z>, dim3(nbx), dim3(Z::NT), sh, p, bx, D(o.cen), D(o.side), ss, sc, a.tri_s,
                       (const double *)a.nodes, nc, out);
     };
     // P2M / P2L: moments on the matrix cores (shapes at P2X_WIDE_STRIDE)
@@ -2243,8 +2285,8 @@ void enqueue_far(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
             HIPOK(hipErrorInvalidValue);
         auto kern = irr ? (shape == 0 ? k_p2l<8, 7, 8> : shape == 1 ? k_p2l<16, 7, 8> : k_p2l<8, 14, 4>)
                         : (shape == 0 ? k_p2m<8, 7, 8> : shape == 1 ? k_p2m<16, 7, 8> : k_p2m<8, 14, 4>);
-        ln.launch(kern, dim3(nbx), dim3(64 * wb), sh, p, nq, stride, bx, ls, li, D(o.cen), D(o.side), I(o.ss),
-                  I(o.sc), (const double *)a.nodes, nc, out);
+        ln.launch(kern, dim3(nbx), dim3(64 * wb), sh, p, nq, stride, bx, ls, li, D(o.cen), D(o.side), ss,
+                  sc, (const double *)a.nodes, nc, out);
     };
     auto p2 = [&](bool irr, size_t nbx, const int *bx, const int *ls, const int *li, double *out) {
         switch (tri ? p2t_shape(irr ? p + 1 : p, nq) : -1) {
@@ -2257,16 +2299,24 @@ void enqueue_far(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
     };
     if (!PL.p2m_boxes.empty()) p2(false, PL.p2m_boxes.size(), I(o.p2m), nullptr, nullptr, mp);
     mark(2, false);
-    // M2M / L2L: rotated translations, the kernel of M2L (unit scale)
-    auto run_trans = [&](const GemmLaunch &g, const LaunchOff &lo_, const double *A, const double *X, double *Y) {
-        if (g.tiles.empty()) return;
-        int ntiles = (int)g.tiles.size();
-        ln.launch(k_m2m_l2l, dim3(ntiles), dim3(ML_THREADS), 0, (const M2LTile *)(P + lo_.tiles), ntiles, A,
-                  (const int *)(P + lo_.src), (const int *)(P + lo_.dst), (const double *)(P + lo_.sc), X, Y, nc);
-    };
     mark(3, true);
-    for (size_t k = 0; k < PL.m2m_l.size(); k++) run_trans(PL.m2m_l[k], o.m2m[k], (const double *)oc.m2m.p, mp, mp);
+    for (size_t k = 0; k < PL.m2m_l.size(); k++) enqueue_trans(PL.m2m_l[k], o.m2m[k], a.PU, oc.m2m, mp, mp, nc, ln);
     mark(3, false);
+    mark(5, true);
+    if (!PL.p2l_boxes.empty()) p2(true, PL.p2l_boxes.size(), I(o.p2lb), I(o.p2ls), I(o.p2li), lo);
+    mark(5, false);
+}
+
+// M2L and L2L (build_plan_m2l)
+template <class Mark>
+void enqueue_m2l(const FarLaunch &a, Lane &ln, Mark mark)
+{
+    const Plan &PL = *a.PL;
+    const PlanOffsets &o = *a.o;
+    const OpsCache &oc = *a.oc;
+    const char *P = a.PM;
+    const int nc = ncoef(oc.p);
+    double *mp = a.exps, *lo = mp + (size_t)a.nb * NRHS * nc;
     mark(4, true);
     if (!PL.m2l_tiles.empty()) {
         int ntiles = (int)PL.m2l_tiles.size();
@@ -2275,22 +2325,32 @@ void enqueue_far(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
                   (const double *)(P + o.m2l.sc), (const double *)mp, lo, nc);
     }
     mark(4, false);
-    mark(5, true);
-    if (!PL.p2l_boxes.empty()) p2(true, PL.p2l_boxes.size(), I(o.p2lb), I(o.p2ls), I(o.p2li), lo);
-    mark(5, false);
     mark(6, true);
-    for (size_t k = 0; k < PL.l2l_l.size(); k++) run_trans(PL.l2l_l[k], o.l2l[k], (const double *)oc.l2l.p, lo, lo);
+    for (size_t k = 0; k < PL.l2l_l.size(); k++) enqueue_trans(PL.l2l_l[k], o.l2l[k], P, oc.l2l, lo, lo, nc, ln);
     mark(6, false);
+}
+
+// L2T and M2T (build_plan_eval)
+template <class Mark>
+void enqueue_eval(const FarLaunch &a, Lane &ln, Mark mark)
+{
+    const Plan &PL = *a.PL;
+    const PlanOffsets &o = *a.o;
+    const OpsCache &oc = *a.oc;
+    const double *cen = (const double *)(a.PU + o.cen), *side = (const double *)(a.PU + o.side);
+    auto I = [&](size_t off) { return (const int *)(a.PE + off); };
+    const int p = oc.p, nc = ncoef(p);
+    double *mp = a.exps, *lo = mp + (size_t)a.nb * NRHS * nc;
     auto meval = [&](bool irr, size_t o_sb, size_t o_wt, int nwt, size_t o_bt, int nbt, size_t o_tp, const double *ex) {
         int ph = irr ? p + 2 : p;
         int nsteps = ((ph + 1) * (ph + 2) / 2 + 1) / 2;
         if (irr) {   // M2T: several wave tasks per slot sharing the operand, formed in LDS
             size_t sh = (size_t)NRHS * nc * 8;
             ln.launch(k_m2t, dim3(nbt), dim3(64 * EW_WAVES), sh, p, nwt, I(o_wt), I(o_bt), I(o_tp), I(o_sb),
-                      D(o.cen), D(o.side), a.pts, ex, nc, (const FieldTerm *)oc.ft_mp.p, nsteps, a.lap);
+                      cen, side, a.pts, ex, nc, (const FieldTerm *)oc.ft_mp.p, nsteps, a.lap);
         } else {     // L2T: mostly one wave task per leaf; each wave forms its operand
             ln.launch(k_l2t, dim3((nwt + EB_WAVES - 1) / EB_WAVES), dim3(64 * EB_WAVES), 0, p, nwt, I(o_wt),
-                      I(o_tp), I(o_sb), D(o.cen), D(o.side), a.pts, ex, nc, (const FieldTerm *)oc.ft_loc.p, nsteps,
+                      I(o_tp), I(o_sb), cen, side, a.pts, ex, nc, (const FieldTerm *)oc.ft_loc.p, nsteps,
                       a.lap);
         }
     };
@@ -2303,7 +2363,54 @@ void enqueue_far(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
     mark(8, false);
 }
 
+template <class Mark>
+void enqueue_far(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
+{
+    enqueue_up(a, np, ln, mark);
+    enqueue_m2l(a, ln, mark);
+    enqueue_eval(a, ln, mark);
+}
+
+// The far-field lists of a plan in three parts, each packed, sent and started
+// before the next is built, so that the host builds M2L's lists beside P2M, M2M
+// and P2L and the evaluation's beside M2L (81,920 triangles + 100,000 targets:
+// the lists take 3 ms of host time, the kernels before M2L 3.3 ms; apply 19.8 ->
+// 16.2 ms). Only for an apply that is alone: its far field would hold up the
+// others' while the host builds (far fields run in order).
+template <class Mark>
+void run_far_parts(FarLaunch a, const Tree &T, Plan &PL, PlanOffsets &o, bool src_eval, size_t np, Workspace &W,
+                   Lane &ln, Mark mark)
+{
+    auto send = [&](int part, auto &&pack) {
+        Packer pk;
+        pack(pk);
+        W.part[part].ensure(pk.size);
+        W.part_stage[part].ensure(pk.size);
+        pk.pack(W.part_stage[part].p);
+        HIPOK(hipMemcpyAsync(W.part[part].p, W.part_stage[part].p, pk.size, hipMemcpyHostToDevice, ln.stream));
+        return (const char *)W.part[part].p;
+    };
+    const Operators *ops = &a.oc->ops;
+    build_plan_up(T, ops, PL, false);
+    a.PU = send(0, [&](Packer &pk) { pack_up(pk, T, PL, o); });
+    enqueue_up(a, np, ln, mark);
+    build_plan_m2l(T, ops, src_eval, NRHS, PL);
+    a.PM = send(1, [&](Packer &pk) { pack_m2l(pk, PL, o); });
+    enqueue_m2l(a, ln, mark);
+    build_plan_eval(T, a.n, ops, src_eval, PL, false);
+    a.PE = send(2, [&](Packer &pk) { pack_eval(pk, PL, o); });
+    enqueue_eval(a, ln, mark);
+}
+
 }  // namespace
+
+// Whether an octree of np points, nbox per leaf, is built on the host although
+// the device is free: the device build is a chain of about 20 launches and a
+// round trip per level (0.34 ms for 217 points, 0.69 for 3,880, 0.82 for 9,200),
+// the host's costs about 0.02 us a point and 1 us a box (0.005, 0.43 and 1.0
+// ms for the same points at 40 to a leaf; 0.24 against 0.43 ms for 12,000 at 400
+// to a leaf).
+bool small_tree(int np, int nbox) { return np <= 6000 || (np <= 20000 && np / 64 <= nbox); }
 
 // The apply: device pointers in, device pointers out.
 // Stored near-field interactions of the iter entry points, owned by the
@@ -2414,12 +2521,14 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
     const bool half = it && it->half;
     const double *d_tgt_in = d_tgt;                  // before the half space mirrors it
     // the octree is built on the device when this is the only apply in
-    // flight; beside other applies it is built on the host, where it
-    // overlaps their kernels instead of queueing behind them
-    // (ELFMM_HOST_TREE=1: always on the host, =0: always on the device)
+    // flight and the points are not few; beside other applies it is built on
+    // the host, where it overlaps their kernels instead of queueing behind
+    // them (ELFMM_HOST_TREE=1: always on the host, =0: always on the device)
     const char *ht_env = std::getenv("ELFMM_HOST_TREE");
     bool host_tree = direct_only || (ht_env && ht_env[0] == '1');
-    if (!host_tree && !(ht_env && ht_env[0] == '0')) host_tree = inflight.others > 0;
+    const int nbox =
+        direct_only ? n + nt : (it ? iprec_nbox_iter(iprec, n + nt) : iprec_nbox(iprec, n + nt));
+    if (!host_tree && !(ht_env && ht_env[0] == '0')) host_tree = inflight.others > 0 || small_tree(n + nt, nbox);
     bool have_host = false;
     auto host_coords = [&]() {
         if (have_host) return;
@@ -2458,8 +2567,7 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
             same_coords(st->xs, W.hsrc.data(), 3 * (size_t)n) && same_coords(st->xt, W.htgt.data(), 3 * (size_t)nt))
             kept = st;
     }
-    int nbox = direct_only ? n + nt : (iter ? iprec_nbox_iter(iprec, n + nt) : iprec_nbox(iprec, n + nt));
-    Tree Tnew;
+    Tree &Tnew = W.treeh;
     if (!kept) {
         bool deep = host_tree;
         if (!host_tree) {
@@ -2616,25 +2724,13 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
     // ---- upload plan
     Packer pk;
     PlanOffsets po;
-    size_t o_iz, o_izt, o_ss, o_sc, o_ts, o_tc, o_nfb, o_nfs, o_nfi, o_nfw;
     if (split) {
-        // what the gather, the near field and the assembly read; the far
-        // field gets its own buffer once its lists exist
-        o_iz = pk.add(T.iz);
-        o_izt = pk.add(T.iztarg);
-        o_ss = pk.add(T.src_start);
-        o_sc = pk.add(T.src_count);
-        o_ts = pk.add(T.tgt_start);
-        o_tc = pk.add(T.tgt_count);
-        o_nfb = pk.add(PL.nf_boxes);
-        o_nfs = pk.add(PL.nf_start);
-        o_nfi = pk.add(PL.nf_items);
-        o_nfw = pk.add(PL.nf_tasks);
+        pack_near(pk, T, PL, po);                    // the far field gets its own buffers once its lists exist
     } else {
         pack_plan(pk, T, PL, po);
-        o_iz = po.iz, o_izt = po.izt, o_ss = po.ss, o_sc = po.sc, o_ts = po.ts, o_tc = po.tc;
-        o_nfb = po.nfb, o_nfs = po.nfs, o_nfi = po.nfi, o_nfw = po.nfw;
     }
+    const size_t o_iz = po.iz, o_izt = po.izt, o_ss = po.ss, o_sc = po.sc, o_ts = po.ts, o_tc = po.tc;
+    const size_t o_nfb = po.nfb, o_nfs = po.nfs, o_nfi = po.nfi, o_nfw = po.nfw;
     size_t o_sbase = pk.add(nf_sbase), o_ntri = pk.add(nf_ntri), o_pst = pk.add(nf_pstart);
     size_t o_nfc = pk.add(nf_chunk);
     size_t o_htb = pk.add(h_tb), o_htbase = pk.add(h_tbase);
@@ -2792,23 +2888,34 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
     ev_end(9, ns);
     HIPOK(hipEventRecord(W.ev_join, ns));
 
-    // split plan: the far-field lists, built while the near field runs
+    // split plan: the far-field lists, built while the near field runs; in
+    // parts while the far field runs too when no other apply is in flight
+    const bool usefar = oc && T.nlev >= 2 && !near_only && !(half && !(g_half_parts.load() & 2));
+    const bool parts = split && usefar && inflight.others == 0;
     const char *PF = P;
-    if (split) {
-        double tf0 = now_ms();
-        build_plan_far(T, n, &oc->ops, src_eval, NRHS, PL, false);
+    double tf0 = now_ms();
+    auto planned = [&]() {
         plan_lk.unlock();
         for (int i = 0; i < 16; i++) g_stats[i] = PL.stats[i];
-        Packer pkf;
-        pack_plan(pkf, T, PL, po);
-        W.plan2.ensure(pkf.size);
-        W.stage2.ensure(pkf.size);
-        pkf.pack(W.stage2.p);
-        HIPOK(hipMemcpyAsync(W.plan2.p, W.stage2.p, pkf.size, hipMemcpyHostToDevice, stream));
-        PF = W.plan2.get<char>();
         double tf1 = now_ms();
         g_times[13] += tf1 - tf0;
         g_times[0] += tf1 - tf0;
+    };
+    if (split && !usefar) {
+        build_plan_up(T, &oc->ops, PL, false);       // its counts (no far field below level 2)
+        planned();
+    } else if (split && !parts) {
+        build_plan_far(T, n, &oc->ops, src_eval, NRHS, PL, false);
+        Packer pkf;
+        pack_up(pkf, T, PL, po);
+        pack_m2l(pkf, PL, po);
+        pack_eval(pkf, PL, po);
+        W.part[0].ensure(pkf.size);
+        W.part_stage[0].ensure(pkf.size);
+        pkf.pack(W.part_stage[0].p);
+        HIPOK(hipMemcpyAsync(W.part[0].p, W.part_stage[0].p, pkf.size, hipMemcpyHostToDevice, stream));
+        PF = W.part[0].get<char>();
+        planned();
     }
 
     // far fields of different applies run in order (see g_order_mu)
@@ -2818,7 +2925,6 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
     if (dev < ORDER_DEVICES && g_order_tail[dev]) HIPOK(hipStreamWaitEvent(stream, g_order_tail[dev], 0));
 
     // ---- far field (and assembly) of each density set
-    bool usefar = oc && T.nlev >= 2 && !near_only && !(half && !(g_half_parts.load() & 2));
     if (nrhs > 1) {
         // several sets: their far fields SET_LANES at a time on streams of
         // their own (one set's far field leaves much of the device idle),
@@ -2843,7 +2949,7 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
             const double *ssl_r = dm0 + (size_t)r * n * 3, *sdl_r = dm1 + (size_t)r * n * 3;
             double *lap_j = usefar ? W.set_lap[j].get<double>() : nullptr;
             if (usefar) {
-                FarLaunch fl{&ds, oc, &PL, &po, PF, iprec, n, nb, tri_s, nrm_s, ssl_r, sdl_r, ifsl, ifdl,
+                FarLaunch fl{&ds, oc, &PL, &po, P, PF, PF, PF, iprec, n, nb, tri_s, nrm_s, ssl_r, sdl_r, ifsl, ifdl,
                              muF, c1F, c2F, half ? -1.0 : 1.0, W.pts.get<double>(), W.set_nodes[j].get<double>(),
                              W.set_exps[j].get<double>(), lap_j};
                 Lane ln;
@@ -2880,17 +2986,23 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
             W.exps.ensure(n_exps * 8);
             W.lap.ensure(n_lap * 8);
             W.nodes.ensure(n_nodes * 8);
-            FarLaunch fl{&ds, oc, &PL, &po, PF, iprec, n, nb, tri_s, nrm_s, ssl_r, sdl_r, ifsl, ifdl,
+            FarLaunch fl{&ds, oc, &PL, &po, P, PF, PF, PF, iprec, n, nb, tri_s, nrm_s, ssl_r, sdl_r, ifsl, ifdl,
                          muF, c1F, c2F, half ? -1.0 : 1.0, W.pts.get<double>(), W.nodes.get<double>(),
                          W.exps.get<double>(), W.lap.get<double>()};
             Lane ln;
             ln.stream = stream;
-            enqueue_far(fl, (size_t)np, ln, [&](int k, bool begin) {
+            auto mark = [&](int k, bool begin) {
                 if (begin)
                     ev_begin(k, stream);
                 else
                     ev_end(k, stream);
-            });
+            };
+            if (parts) {
+                run_far_parts(fl, T, PL, po, src_eval, (size_t)np, W, ln, mark);
+                planned();
+            } else {
+                enqueue_far(fl, (size_t)np, ln, mark);
+            }
         }
         if (r + 1 == nrhs) {
             HIPOK(hipEventRecord(W.ev_done, stream));
@@ -2976,16 +3088,16 @@ int parttarg_dev(int iprec, double rlam, double rmu, int n, const double *d_src,
     int src_eval = (ifpt || ifst) ? 1 : 0;
     if (!(ifptt || ifstt)) nt = 0;
     double c1 = (rlam + rmu) / (rlam + 2 * rmu), c2 = rmu / (rlam + 2 * rmu);
-    // octree on the device unless another apply is in flight (as the
-    // triangle apply); the one-box tree of the direct sum on the host
+    // octree on the device unless another apply is in flight or the points
+    // are few (as the triangle apply); the one-box tree of the direct sum on the host
     const char *ht_env = std::getenv("ELFMM_HOST_TREE");
     bool host_tree = direct || (ht_env && ht_env[0] == '1');
-    if (!host_tree && !(ht_env && ht_env[0] == '0')) host_tree = inflight.others > 0;
+    const int nbox = direct ? n + nt : iprec_nbox_part(iprec, n + nt);
+    if (!host_tree && !(ht_env && ht_env[0] == '0')) host_tree = inflight.others > 0 || small_tree(n + nt, nbox);
 
     std::unique_lock<std::mutex> plan_lk(g_plan_mu);
     double t0 = now_ms();
-    int nbox = direct ? n + nt : iprec_nbox_part(iprec, n + nt);
-    Tree T;
+    Tree &T = W.treeh;
     bool deep = host_tree;
     if (!host_tree) {
         if (!W.oct) W.oct.reset(new OctreeWork());
@@ -3007,13 +3119,12 @@ int parttarg_dev(int iprec, double rlam, double rmu, int n, const double *d_src,
     }
     int p = oc ? oc->p : 0;
     Plan &PL = W.planh;
-    build_plan(T, n, oc ? &oc->ops : nullptr, src_eval, false, NRHS, PL, false);
-    plan_lk.unlock();
-    for (int i = 0; i < 16; i++) g_stats[i] = PL.stats[i];
+    plan_reset(PL);
+    build_plan_near(T, src_eval, false, false, PL);
     const std::vector<int> chunks = point_chunks(T, PL, src_eval);
     Packer pk;
     PlanOffsets po;
-    pack_plan(pk, T, PL, po);
+    pack_near(pk, T, PL, po);
     size_t o_ch = pk.add(chunks);
     W.plan.ensure(pk.size);
     W.stage.ensure(pk.size);
@@ -3055,18 +3166,49 @@ int parttarg_dev(int iprec, double rlam, double rmu, int n, const double *d_src,
                            W.pts.get<double>(), W.nodes.get<double>(), c1, W.nf.get<double>());
     HIPOK(hipGetLastError());
     HIPOK(hipEventRecord(W.ev_join, ns));
+    // far-field lists, as the triangle apply
+    const bool parts = usefar && inflight.others == 0;
+    const char *PF = P;
+    double tf0 = now_ms();
+    auto planned = [&]() {
+        plan_lk.unlock();
+        for (int i = 0; i < 16; i++) g_stats[i] = PL.stats[i];
+        g_times[0] += now_ms() - tf0;
+    };
+    if (!usefar) {
+        build_plan_up(T, oc ? &oc->ops : nullptr, PL, false);
+        planned();
+    } else if (!parts) {
+        build_plan_far(T, n, &oc->ops, src_eval, NRHS, PL, false);
+        Packer pkf;
+        pack_up(pkf, T, PL, po);
+        pack_m2l(pkf, PL, po);
+        pack_eval(pkf, PL, po);
+        W.part[0].ensure(pkf.size);
+        W.part_stage[0].ensure(pkf.size);
+        pkf.pack(W.part_stage[0].p);
+        HIPOK(hipMemcpyAsync(W.part[0].p, W.part_stage[0].p, pkf.size, hipMemcpyHostToDevice, stream));
+        PF = W.part[0].get<char>();
+        planned();
+    }
     // far fields of different applies run in order (see g_order_mu)
     int dev = 0;
     HIPOK(hipGetDevice(&dev));
     std::unique_lock<std::mutex> order(g_order_mu);
     if (dev < ORDER_DEVICES && g_order_tail[dev]) HIPOK(hipStreamWaitEvent(stream, g_order_tail[dev], 0));
     if (usefar) {
-        FarLaunch fl{&ds, oc, &PL, &po, P, iprec, n, nb, nullptr, nullptr, nullptr, nullptr, ifsl, ifdl,
+        FarLaunch fl{&ds, oc, &PL, &po, P, PF, PF, PF, iprec, n, nb, nullptr, nullptr, nullptr, nullptr, ifsl, ifdl,
                      rmu, c1, c2, 1.0, W.pts.get<double>(), W.nodes.get<double>(), W.exps.get<double>(),
                      W.lap.get<double>(), true};
         Lane ln;
         ln.stream = stream;
-        enqueue_far(fl, (size_t)np, ln, [](int, bool) {});
+        auto mark = [](int, bool) {};
+        if (parts) {
+            run_far_parts(fl, T, PL, po, src_eval, (size_t)np, W, ln, mark);
+            planned();
+        } else {
+            enqueue_far(fl, (size_t)np, ln, mark);
+        }
     }
     HIPOK(hipEventRecord(W.ev_done, stream));
     if (dev < ORDER_DEVICES) g_order_tail[dev] = W.ev_done;
@@ -3696,7 +3838,7 @@ void batch_enqueue_view(Batch &B, const BatchView &V, Lane &f, Lane &q)
                  (const double *)V.pts, (const double *)V.rec, B.rlam, B.rmu, c1, V.nf);
     }
     if (V.usefar) {
-        FarLaunch fl{B.ds, B.oc, V.PL, V.po, P, B.iprec, n, V.nb, tri_s, nrm_s, ssl_s, sdl_s, B.ifsl, B.ifdl,
+        FarLaunch fl{B.ds, B.oc, V.PL, V.po, P, P, P, P, B.iprec, n, V.nb, tri_s, nrm_s, ssl_s, sdl_s, B.ifsl, B.ifdl,
                      B.rmu, c1, c2, 1.0, V.pts, V.nodes, V.exps, V.lap};
         enqueue_far(fl, (size_t)np, f, [](int, bool) {});
     }

@@ -137,7 +137,7 @@ struct Plan {
     GemmLaunch m2l;                                  // all list-2 pairs, grouped by offset (src/dst/scale)
     std::vector<M2LTile> m2l_tiles;                  // rotated-M2L tiles over those pairs
     std::vector<int> p2l_boxes, p2l_start, p2l_items;   // box <- sources of its list-4 boxes
-    std::vector<int> m2t_boxes, m2t_start, m2t_items;   // box <- multipoles of its list-3 boxes
+    std::vector<int> m2t_items;                      // boxes taking the multipole of each m2t slot, slot after slot
     std::vector<int> l2t_boxes, nf_boxes, nf_start, nf_items;
     std::vector<int> nf_tasks;                       // near-field waves: (near box, first lane, lanes per point)
     std::vector<int> l2t_tpt;                        // points of each l2t slot, slot after slot
@@ -161,16 +161,21 @@ constexpr int EW_PTS = 32;                           // points per evaluation wa
 // field (src/elfmm3dtria_iter_1.f:1061-1110).
 void build_plan(const Tree &T, int n, const Operators *ops, bool src_eval, bool direct_only, int nrhs,
                 Plan &P, bool iter = false);
-// The two halves of build_plan, for a caller that starts the near field
-// before the far-field lists exist: build_plan_near fills the near-field
-// lists (nf_*, stats[6]) of P, build_plan_far everything else; neither
-// clears what the other fills (P starts from plan_reset).
+// The parts of build_plan, for a caller that starts the device on each as soon
+// as its lists exist: build_plan_near fills the near-field lists (nf_*,
+// stats[6]) of P, build_plan_far everything else, in three parts:
+// build_plan_up the box sides, P2M, M2M and P2L, build_plan_m2l M2L and L2L,
+// build_plan_eval L2T and M2T. None clears what another fills (P starts from
+// plan_reset).
 void build_plan_near(const Tree &T, bool src_eval, bool direct_only, bool iter, Plan &P);
-// Empties P for a new plan (zero stats); the M2L pair arrays keep their
-// memory and length, which the next build_plan_far resizes and overwrites
-// (no fresh allocation or clearing of its largest arrays per apply).
+// Empties P for a new plan (zero stats), keeping its arrays' memory; the M2L
+// pair arrays keep their length too, which the next build_plan_m2l resizes and
+// overwrites (no clearing of the largest arrays per apply).
 void plan_reset(Plan &P);
 void build_plan_far(const Tree &T, int n, const Operators *ops, bool src_eval, int nrhs, Plan &P, bool iter);
+void build_plan_up(const Tree &T, const Operators *ops, Plan &P, bool iter);
+void build_plan_m2l(const Tree &T, const Operators *ops, bool src_eval, int nrhs, Plan &P);
+void build_plan_eval(const Tree &T, int n, const Operators *ops, bool src_eval, Plan &P, bool iter);
 
 // Task lists of the Mindlin harmonic far field (lfmm3d_list2_mindlin,
 // src/lfmm3droutsmindlin.f:28-529) on its own octree, beside the Laplace

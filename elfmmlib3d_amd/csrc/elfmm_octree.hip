@@ -462,6 +462,22 @@ __global__ void k_oct_cnt1(int nb, const int *__restrict__ acnt, const int *__re
     if (i == nb) c[i] = 0;
 }
 
+// The tree's arrays into one buffer for one transfer (26 transfers into
+// pageable memory took about 0.3 ms).
+constexpr int OCT_ARR = 24;
+struct OctPack {
+    const int *src[OCT_ARR];
+    size_t off[OCT_ARR + 1];                          // in ints; off[k + 1] - off[k] ints of array k
+    int n;
+};
+__global__ void k_oct_pack(OctPack p, int *__restrict__ out)
+{
+    int a = blockIdx.y;
+    size_t n = p.off[a + 1] - p.off[a];
+    for (size_t i = (size_t)blockIdx.x * OCT_T + threadIdx.x; i < n; i += (size_t)gridDim.x * OCT_T)
+        out[p.off[a] + i] = p.src[a][i];
+}
+
 int bits_for(long v)
 {
     int b = 1;
@@ -521,6 +537,26 @@ struct OctreeWork::Impl {
             return (T *)p;
         }
     };
+    // pinned host memory: the counts read back while building, then the tree
+    struct Pin {
+        int *p = nullptr;
+        size_t bytes = 0;
+        ~Pin()
+        {
+            if (p) (void)hipHostFree(p);
+        }
+        hipError_t ensure(size_t b)
+        {
+            if (b <= bytes) return hipSuccess;
+            if (p) (void)hipHostFree(p);
+            p = nullptr;
+            bytes = 0;
+            hipError_t e = hipHostMalloc((void **)&p, b + b / 4, hipHostMallocDefault);
+            if (e == hipSuccess) bytes = b + b / 4;
+            return e;
+        }
+    } pin;
+    Buf packed;
     Buf part, root, key, key2, idx, idx2, tag, sexcl, head, incl, active, cur, dcount, tmp;
     Buf box[11];                                    // level, ijk, parent, kids, nkids, ss, sc, ts, tc, split, firstkid
     Buf sleaf, tleaf, iota, skey, iz, izt;
@@ -618,7 +654,8 @@ hipError_t build_tree_dev(const double *d_src, int n, const double *d_tgt, int n
     std::vector<int> laddr = {0, 1};
     int nb = 1, nlev = 0;
     int nsplit = (n > nbox || nt > nbox) ? 1 : 0;
-    int hc[2];
+    OCTOK(W.pin.ensure(256));
+    int *hc = W.pin.p;                                // pinned: a readback is one transfer and one wait
     for (int lev = 1; nsplit > 0; lev++) {
         if (lev > OCT_D) {
             too_deep = true;
@@ -685,10 +722,10 @@ hipError_t build_tree_dev(const double *d_src, int n, const double *d_tgt, int n
     OCTOK(hipMemsetAsync(W.n2.get<int>() + nb, 0, 4, s));
     OCTOK(cub_excl(W.n5.get<int>(), W.st[5].get<int>(), nb + 1));
     OCTOK(cub_excl(W.n2.get<int>(), W.st[2].get<int>(), nb + 1));
-    int t5 = 0, t2 = 0;
-    OCTOK(hipMemcpyAsync(&t5, W.st[5].get<int>() + nb, 4, hipMemcpyDeviceToHost, s));
-    OCTOK(hipMemcpyAsync(&t2, W.st[2].get<int>() + nb, 4, hipMemcpyDeviceToHost, s));
+    OCTOK(hipMemcpyAsync(hc, W.st[5].get<int>() + nb, 4, hipMemcpyDeviceToHost, s));
+    OCTOK(hipMemcpyAsync(hc + 1, W.st[2].get<int>() + nb, 4, hipMemcpyDeviceToHost, s));
     OCTOK(hipStreamSynchronize(s));
+    const int t5 = hc[0], t2 = hc[1];
     OCTOK(W.it[5].ensure((size_t)t5 * 4 + 4));
     OCTOK(W.it[2].ensure((size_t)t2 * 4 + 4));
     OCTOK(W.owner.ensure((size_t)t5 * 4 + 4));
@@ -712,7 +749,7 @@ hipError_t build_tree_dev(const double *d_src, int n, const double *d_tgt, int n
     OCTOK(cub_excl(W.c1.get<int>(), W.o1q.get<int>(), t5 + 1));
     OCTOK(cub_excl(W.c3.get<int>(), W.o3q.get<int>(), t5 + 1));
     OCTOK(cub_excl(W.ca.get<int>(), W.oaq.get<int>(), t5 + 1));
-    int tot[3];
+    int *tot = hc;
     OCTOK(hipMemcpyAsync(&tot[0], W.o1q.get<int>() + t5, 4, hipMemcpyDeviceToHost, s));
     OCTOK(hipMemcpyAsync(&tot[1], W.o3q.get<int>() + t5, 4, hipMemcpyDeviceToHost, s));
     OCTOK(hipMemcpyAsync(&tot[2], W.oaq.get<int>() + t5, 4, hipMemcpyDeviceToHost, s));
@@ -766,39 +803,50 @@ hipError_t build_tree_dev(const double *d_src, int n, const double *d_tgt, int n
                        W.t1.get<int>(), W.st[1].get<int>(), W.it[1].get<int>());
     OCTOK(hipGetLastError());
 
-    // to the host
-    T = Tree();
+    // to the host, in one piece (T's arrays keep their memory)
     T.nboxes = nb;
     T.nlev = nlev;
     T.laddr = laddr;
-    double root[4];
-    OCTOK(hipMemcpyAsync(root, W.root.p, 32, hipMemcpyDeviceToHost, s));
-    T.level.resize(nb);
-    T.ijk.resize(3 * (size_t)nb);
-    T.parent.resize(nb);
-    T.kids.resize(8 * (size_t)nb);
-    T.nkids.resize(nb);
-    T.src_start.resize(nb);
-    T.src_count.resize(nb);
-    T.tgt_start.resize(nb);
-    T.tgt_count.resize(nb);
-    std::vector<int> *dst[9] = {&T.level, &T.ijk, &T.parent, &T.kids, &T.nkids, &T.src_start, &T.src_count,
+    T.box_side.clear();
+    OctPack op;
+    std::vector<int> *dst[OCT_ARR];
+    op.n = 0;
+    op.off[0] = 8;                                    // after the root cube
+    auto put = [&](const void *src, std::vector<int> &v, size_t count) {
+        v.resize(count);
+        dst[op.n] = &v;
+        op.src[op.n] = (const int *)src;
+        op.off[op.n + 1] = op.off[op.n] + count;
+        op.n++;
+    };
+    std::vector<int> *box[9] = {&T.level, &T.ijk, &T.parent, &T.kids, &T.nkids, &T.src_start, &T.src_count,
                                 &T.tgt_start, &T.tgt_count};
-    for (int a = 0; a < 9; a++)
-        OCTOK(hipMemcpyAsync(dst[a]->data(), W.box[a].p, dst[a]->size() * 4, hipMemcpyDeviceToHost, s));
-    T.iz.resize(n);
-    T.iztarg.resize(nt);
-    OCTOK(hipMemcpyAsync(T.iz.data(), W.iz.p, (size_t)n * 4, hipMemcpyDeviceToHost, s));
-    if (nt) OCTOK(hipMemcpyAsync(T.iztarg.data(), W.izt.p, (size_t)nt * 4, hipMemcpyDeviceToHost, s));
+    for (int a = 0; a < 9; a++) put(W.box[a].p, *box[a], (size_t)nb * ints_per_box[a]);
+    put(W.iz.p, T.iz, n);
+    put(W.izt.p, T.iztarg, nt);
     const int tot_items[6] = {0, n1own + nap, t2, n3, n3, t5};
     for (int t = 1; t <= 5; t++) {
-        T.lstart[t].resize(nb + 1);
-        T.litems[t].resize(tot_items[t]);
-        OCTOK(hipMemcpyAsync(T.lstart[t].data(), W.st[t].p, (size_t)(nb + 1) * 4, hipMemcpyDeviceToHost, s));
-        if (tot_items[t])
-            OCTOK(hipMemcpyAsync(T.litems[t].data(), W.it[t].p, (size_t)tot_items[t] * 4, hipMemcpyDeviceToHost, s));
+        put(W.st[t].p, T.lstart[t], nb + 1);
+        put(W.it[t].p, T.litems[t], tot_items[t]);
     }
+    const size_t total = op.off[op.n];
+    OCTOK(W.packed.ensure(total * 4));
+    OCTOK(W.pin.ensure(total * 4));
+    hipLaunchKernelGGL(k_oct_pack, dim3(64, op.n), dim3(OCT_T), 0, s, op, W.packed.get<int>());
+    OCTOK(hipGetLastError());
+    OCTOK(hipMemcpyAsync(W.packed.p, W.root.p, 32, hipMemcpyDeviceToDevice, s));
+    OCTOK(hipMemcpyAsync(W.pin.p, W.packed.p, total * 4, hipMemcpyDeviceToHost, s));
     OCTOK(hipStreamSynchronize(s));
+    const double *root = (const double *)W.pin.p;
+    constexpr size_t PIECE = 1 << 16;                 // ints per host copy
+    std::vector<std::pair<int, size_t>> piece;
+    for (int a = 0; a < op.n; a++)
+        for (size_t i = 0; i < dst[a]->size(); i += PIECE) piece.push_back({a, i});
+    parallel_chunks((int)piece.size(), [&](int k, int) {
+        std::vector<int> &v = *dst[piece[k].first];
+        size_t i = piece[k].second, m = std::min(PIECE, v.size() - i);
+        std::copy_n(W.pin.p + op.off[piece[k].first] + i, m, v.data() + i);
+    });
     for (int d = 0; d < 3; d++) T.center[d] = root[d];
     T.size = root[3];
     // box centres of d3tcentc (src/d3tstrcr.f:1596-1676), as build_tree

@@ -151,21 +151,38 @@ template <class NP>
 void near_tasks(Plan &P, const std::vector<int> &ntri, NP &&npts, double npt)
 {
     constexpr int NF_WAVES = 2048;                   // 256 CUs x 4 SIMDs x 2
-    int low = 1;
-    while (low < 64 && npt * low < NF_WAVES * 64.0) low *= 2;
-    P.nf_tasks.clear();
-    for (size_t q = 0; q < P.nf_boxes.size(); q++) {
-        int64_t np = npts(P.nf_boxes[q]), best = 0, cost = 0;
-        for (int64_t s = low; s <= 64; s *= 2) {
-            int64_t c = (np * s + 63) / 64 * ((ntri[q] + s - 1) / s + 1);
-            if (!best || c < cost) best = s, cost = c;
+    int low = 0;                                     // log2 of the lanes per point
+    while (low < 6 && npt * (1 << low) < NF_WAVES * 64.0) low++;
+    int nq = (int)P.nf_boxes.size();
+    std::vector<int> start(nq + 1, 0);
+    std::vector<unsigned char> lanes(nq);
+    for (int q = 0; q < nq; q++) {
+        int64_t np = npts(P.nf_boxes[q]), cost = 0;
+        for (int k = low; k <= 6; k++) {
+            int64_t c = (((np << k) + 63) >> 6) * (((ntri[q] + (1 << k) - 1) >> k) + 1);
+            if (!cost || c < cost) lanes[q] = (unsigned char)k, cost = c;
         }
-        for (int64_t l0 = 0; l0 < np * best; l0 += 64) {
-            P.nf_tasks.push_back((int)q);
-            P.nf_tasks.push_back((int)l0);
-            P.nf_tasks.push_back((int)best);
-        }
+        start[q + 1] = start[q] + (int)(((np << lanes[q]) + 63) >> 6);
     }
+    P.nf_tasks.resize(3 * (size_t)start[nq]);
+    for (int q = 0; q < nq; q++)
+        for (int k = 0; k < start[q + 1] - start[q]; k++) {
+            int *t = &P.nf_tasks[3 * (size_t)(start[q] + k)];
+            t[0] = q;
+            t[1] = 64 * k;
+            t[2] = 1 << lanes[q];
+        }
+}
+
+// Order of n entries by decreasing weight, equal weights in their order.
+std::vector<int> heaviest_first(const std::vector<double> &w)
+{
+    std::vector<std::pair<double, int>> k(w.size());
+    for (size_t i = 0; i < w.size(); i++) k[i] = {-w[i], (int)i};
+    std::sort(k.begin(), k.end());
+    std::vector<int> o(w.size());
+    for (size_t i = 0; i < w.size(); i++) o[i] = k[i].second;
+    return o;
 }
 
 }  // namespace
@@ -175,83 +192,80 @@ void build_plan_near(const Tree &T, bool src_eval, bool direct_only, bool iter, 
     int nb = T.nboxes;
     auto npts = [&](int b) { return (src_eval ? T.src_count[b] : 0) + T.tgt_count[b]; };
     P.nf_boxes.clear();
-    P.nf_start.clear();
+    P.nf_start.assign(1, 0);
     P.nf_items.clear();
+    P.nf_tasks.clear();
+    P.stats[6] = 0;
+    if (direct_only) return;
     // leaves: near field over self + list 1. With iter, lists 3 and 4 join
     // the near field; the reference evaluates a box's list 4 at every point
     // below it, so a leaf also takes the list 4 of each of its ancestors and
     // every point is handled once, by its leaf.
-    P.nf_start.push_back(0);
-    for (int b = 0; b < nb; b++) {
-        if (T.nkids[b] || !npts(b)) continue;
-        size_t before = P.nf_items.size();
-        for (int q = T.lstart[1][b]; q < T.lstart[1][b + 1]; q++) {
-            int j = T.litems[1][q];
-            if (T.src_count[j]) P.nf_items.push_back(j);
+    auto each = [&](int b, auto &&f) {
+        for (int q = T.lstart[1][b]; q < T.lstart[1][b + 1]; q++)
+            if (int j = T.litems[1][q]; T.src_count[j]) f(j);
+        if (T.src_count[b]) f(b);
+        if (!iter) return;
+        for (int q = T.lstart[3][b]; q < T.lstart[3][b + 1]; q++)
+            if (int j = T.litems[3][q]; T.src_count[j]) f(j);
+        for (int a = b; a >= 0; a = T.parent[a])
+            for (int q = T.lstart[4][a]; q < T.lstart[4][a + 1]; q++)
+                if (int j = T.litems[4][q]; T.src_count[j]) f(j);
+    };
+    // entries and triangles of every box's list, by chunks of boxes
+    std::vector<int> items(nb, 0), tris(nb, 0);
+    int nchunk = (nb + CHUNK - 1) / CHUNK;
+    parallel_chunks(nchunk, [&](int ch, int) {
+        for (int b = ch * CHUNK; b < std::min(nb, (ch + 1) * CHUNK); b++)
+            if (!T.nkids[b] && npts(b))
+                each(b, [&](int j) {
+                    items[b]++;
+                    tris[b] += T.src_count[j];
+                });
+    });
+    std::vector<int> box;
+    std::vector<double> w;
+    for (int b = 0; b < nb; b++)
+        if (items[b]) {
+            box.push_back(b);
+            w.push_back((double)tris[b] * npts(b));
         }
-        if (T.src_count[b]) P.nf_items.push_back(b);
-        if (iter) {
-            for (int q = T.lstart[3][b]; q < T.lstart[3][b + 1]; q++) {
-                int j = T.litems[3][q];
-                if (T.src_count[j]) P.nf_items.push_back(j);
-            }
-            for (int a = b; a >= 0; a = T.parent[a])
-                for (int q = T.lstart[4][a]; q < T.lstart[4][a + 1]; q++) {
-                    int j = T.litems[4][q];
-                    if (T.src_count[j]) P.nf_items.push_back(j);
-                }
-        }
-        if (P.nf_items.size() == before) continue;
-        P.nf_boxes.push_back(b);
-        P.nf_start.push_back((int)P.nf_items.size());
-    }
-    {
-        // one workgroup per box, heaviest (points x triangles) first, so
-        // the long boxes do not start last
-        size_t nq = P.nf_boxes.size();
-        std::vector<double> w(nq);
-        std::vector<int> ord(nq);
-        for (size_t q = 0; q < nq; q++) {
-            double ns = 0;
-            for (int k = P.nf_start[q]; k < P.nf_start[q + 1]; k++) ns += T.src_count[P.nf_items[k]];
-            w[q] = ns * npts(P.nf_boxes[q]);
-            ord[q] = (int)q;
-        }
-        std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return w[a] > w[b]; });
-        std::vector<int> bx(nq), st(1, 0), it;
-        it.reserve(P.nf_items.size());
-        for (size_t q = 0; q < nq; q++) {
-            int o = ord[q];
-            bx[q] = P.nf_boxes[o];
-            it.insert(it.end(), P.nf_items.begin() + P.nf_start[o], P.nf_items.begin() + P.nf_start[o + 1]);
-            st.push_back((int)it.size());
-        }
-        P.nf_boxes.swap(bx);
-        P.nf_start.swap(st);
-        P.nf_items.swap(it);
-    }
-    if (direct_only) P.nf_boxes.clear();
+    // heaviest (points x triangles) first, so the long boxes do not start last
+    std::vector<int> ord = heaviest_first(w);
+    int nq = (int)box.size();
+    P.nf_boxes.resize(nq);
+    P.nf_start.resize(nq + 1);
+    std::vector<int> ntri(nq);
     double npair_near = 0, npt_near = 0;
-    std::vector<int> ntri(P.nf_boxes.size(), 0);
-    for (size_t q = 0; q < P.nf_boxes.size(); q++) {
-        for (int k = P.nf_start[q]; k < P.nf_start[q + 1]; k++) ntri[q] += T.src_count[P.nf_items[k]];
-        npair_near += (double)npts(P.nf_boxes[q]) * ntri[q];
-        npt_near += npts(P.nf_boxes[q]);
+    for (int q = 0; q < nq; q++) {
+        int b = P.nf_boxes[q] = box[ord[q]];
+        P.nf_start[q + 1] = P.nf_start[q] + items[b];
+        ntri[q] = tris[b];
+        npair_near += w[ord[q]];
+        npt_near += npts(b);
     }
+    P.nf_items.resize(P.nf_start[nq]);
+    parallel_chunks((nq + CHUNK - 1) / CHUNK, [&](int ch, int) {
+        for (int q = ch * CHUNK; q < std::min(nq, (ch + 1) * CHUNK); q++) {
+            int k = P.nf_start[q];
+            each(P.nf_boxes[q], [&](int j) { P.nf_items[k++] = j; });
+        }
+    });
     P.stats[6] = npair_near;
     near_tasks(P, ntri, npts, npt_near);
 }
 
 void plan_reset(Plan &P)
 {
-    GemmLaunch keep;
-    keep.src.swap(P.m2l.src);
-    keep.dst.swap(P.m2l.dst);
-    keep.scale.swap(P.m2l.scale);
-    P = Plan();
-    P.m2l.src.swap(keep.src);
-    P.m2l.dst.swap(keep.dst);
-    P.m2l.scale.swap(keep.scale);
+    for (std::vector<int> *v : {&P.p2m_boxes, &P.p2l_boxes, &P.p2l_start, &P.p2l_items, &P.m2t_items, &P.l2t_boxes,
+                                &P.nf_boxes, &P.nf_start, &P.nf_items, &P.nf_tasks, &P.l2t_tpt, &P.m2t_slot_box,
+                                &P.m2t_tpt, &P.l2t_wt, &P.m2t_wt, &P.m2t_bt})
+        v->clear();
+    P.sides.clear();
+    P.m2m_l.clear();
+    P.l2l_l.clear();
+    P.m2l.tiles.clear();
+    P.m2l_tiles.clear();
     for (double &v : P.stats) v = 0;
 }
 
@@ -265,36 +279,85 @@ void build_plan(const Tree &T, int n, const Operators *ops, bool src_eval, bool 
 
 void build_plan_far(const Tree &T, int n, const Operators *ops, bool src_eval, int nrhs, Plan &P, bool iter)
 {
+    build_plan_up(T, ops, P, iter);
+    build_plan_m2l(T, ops, src_eval, nrhs, P);
+    build_plan_eval(T, n, ops, src_eval, P, iter);
+}
+
+void build_plan_up(const Tree &T, const Operators *ops, Plan &P, bool iter)
+{
+    int nb = T.nboxes;
+    P.sides.resize(nb);
+    for (int b = 0; b < nb; b++) P.sides[b] = T.box_side.empty() ? T.size / (double)(1 << T.level[b]) : T.box_side[b];
+    P.stats[0] = nb;
+    P.stats[1] = T.nlev;
+    P.stats[2] = ops ? ops->p : 0;
+    P.p2l_start.assign(1, 0);
+    if (!ops) return;
+    // M2M children at lev+1 -> parents at lev, for lev = nlev-1 .. 2, the P2M
+    // leaves and the P2L lists side by side
+    int nup = std::max(0, T.nlev - 2);
+    std::vector<GemmLaunch> up(nup);
+    parallel_chunks(nup + 2, [&](int task, int) {
+        if (task >= 2) {
+            up[task - 2] = tree_pass(T, T.nlev - 1 - (task - 2), ncoef(ops->p), ops->oct_phi, true);
+        } else if (task == 1) {
+            std::vector<int> bx;
+            std::vector<double> w;
+            for (int b = 0; b < nb; b++)
+                if (!T.nkids[b] && T.level[b] >= 2 && T.src_count[b] > 0) {
+                    bx.push_back(b);
+                    w.push_back(T.src_count[b]);
+                }
+            // one workgroup per box, most sources first
+            for (int q : heaviest_first(w)) P.p2m_boxes.push_back(bx[q]);
+        } else if (!iter) {
+            // P2L: local of box j from the sources of i with j in list3(i)
+            // (src/lfmm3dtrilhess.f:760-829); owner j, sources list4(j).
+            // Heaviest first: one workgroup per box, so the longest ones
+            // start first and the launch ends evenly.
+            std::vector<int> bx;
+            std::vector<double> w;
+            for (int j = 0; j < nb; j++) {
+                double n4 = 0;
+                for (int q = T.lstart[4][j]; q < T.lstart[4][j + 1]; q++) n4 += T.src_count[T.litems[4][q]];
+                if (n4 > 0) {
+                    bx.push_back(j);
+                    w.push_back(n4);
+                }
+            }
+            for (int q : heaviest_first(w)) {
+                int j = bx[q];
+                P.p2l_boxes.push_back(j);
+                for (int k = T.lstart[4][j]; k < T.lstart[4][j + 1]; k++)
+                    if (T.src_count[T.litems[4][k]]) P.p2l_items.push_back(T.litems[4][k]);
+                P.p2l_start.push_back((int)P.p2l_items.size());
+            }
+        }
+    });
+    double m2m_pairs = 0;
+    for (GemmLaunch &g : up) {
+        if (g.tiles.empty()) continue;
+        m2m_pairs += g.src.size();
+        P.m2m_l.push_back(std::move(g));
+    }
+    P.stats[8] = m2m_pairs;
+    P.stats[10] = (double)P.p2m_boxes.size();
+    P.stats[11] = (double)P.p2l_items.size();
+}
+
+void build_plan_m2l(const Tree &T, const Operators *ops, bool src_eval, int nrhs, Plan &P)
+{
     int nb = T.nboxes;
     int p = ops ? ops->p : 0;
-    int nc = ncoef(p);
     int nchunk = (nb + CHUNK - 1) / CHUNK;
     if (!ops) {
         P.m2l.src.clear();
         P.m2l.dst.clear();
         P.m2l.scale.clear();
+        return;
     }
-    P.sides.resize(nb);
-    for (int b = 0; b < nb; b++) P.sides[b] = T.box_side.empty() ? T.size / (double)(1 << T.level[b]) : T.box_side[b];
-    auto npts = [&](int b) { return (src_eval ? T.src_count[b] : 0) + T.tgt_count[b]; };
-
-    if (ops) {
-        for (int b = 0; b < nb; b++)
-            if (!T.nkids[b] && T.level[b] >= 2 && T.src_count[b] > 0) P.p2m_boxes.push_back(b);
-        // one workgroup per box, most sources first
-        std::stable_sort(P.p2m_boxes.begin(), P.p2m_boxes.end(),
-                         [&](int a, int c) { return T.src_count[a] > T.src_count[c]; });
-        // M2M children at lev+1 -> parents at lev, for lev = nlev-1 .. 2;
-        // L2L parents at lev -> children, for lev = 2 .. nlev-1
-        for (int lev = T.nlev - 1; lev >= 2; lev--) {
-            GemmLaunch g = tree_pass(T, lev, nc, ops->oct_phi, true);
-            if (!g.tiles.empty()) P.m2m_l.push_back(std::move(g));
-        }
-        for (int lev = 2; lev <= T.nlev - 1; lev++) {
-            GemmLaunch g = tree_pass(T, lev, nc, ops->oct_phi, false);
-            if (!g.tiles.empty()) P.l2l_l.push_back(std::move(g));
-        }
-
+    {
         // M2L over list 2, grouped by offset: per-chunk counts by offset,
         // then every chunk fills its slice of each offset's run, so the
         // pairs of one offset stay in increasing target-box order.
@@ -387,64 +450,32 @@ void build_plan_far(const Tree &T, int n, const Operators *ops, bool src_eval, i
                     *t++ = M2LTile{ops->m2l_off[o], h, r0, ostart[o] + p0, std::min(ML_P, m - p0), ops->m2l_phi[o],
                                    ops->m2l_refl[o]};
         });
-        xcd_order(P.m2l_tiles);
+        // L2L parents at lev -> children, for lev = 2 .. nlev-1, beside the
+        // launch order of the M2L tiles
+        int ndown = std::max(0, T.nlev - 2);
+        std::vector<GemmLaunch> down(ndown);
+        parallel_chunks(ndown + 1, [&](int task, int) {
+            if (task) down[task - 1] = tree_pass(T, 1 + task, ncoef(p), ops->oct_phi, false);
+            else xcd_order(P.m2l_tiles);
+        });
+        double l2l_pairs = 0;
+        for (GemmLaunch &g : down) {
+            if (g.tiles.empty()) continue;
+            l2l_pairs += g.src.size();
+            P.l2l_l.push_back(std::move(g));
+        }
         P.stats[3] = npair;
         P.stats[4] = dense;
         P.stats[5] = alg;
-
-        // P2L: local of box j from the sources of i with j in list3(i)
-        // (src/lfmm3dtrilhess.f:760-829); owner j, sources list4(j).
-        // M2T: multipole of i at the points of j with j in list4(i)
-        // (src/lfmm3dtrilhess.f:864-981); owner j, sources list3(j).
-        P.p2l_start.push_back(0);
-        P.m2t_start.push_back(0);
-        for (int j = 0; j < nb && !iter; j++) {
-            int c = 0;
-            for (int q = T.lstart[4][j]; q < T.lstart[4][j + 1]; q++) {
-                int i = T.litems[4][q];
-                if (!T.src_count[i]) continue;
-                P.p2l_items.push_back(i);
-                c++;
-            }
-            if (c) {
-                P.p2l_boxes.push_back(j);
-                P.p2l_start.push_back((int)P.p2l_items.size());
-            }
-            if (!npts(j)) continue;
-            c = 0;
-            for (int q = T.lstart[3][j]; q < T.lstart[3][j + 1]; q++) {
-                int i = T.litems[3][q];
-                if (!T.src_count[i]) continue;
-                P.m2t_items.push_back(i);
-                c++;
-            }
-            if (c) {
-                P.m2t_boxes.push_back(j);
-                P.m2t_start.push_back((int)P.m2t_items.size());
-            }
-        }
-        // P2L boxes in decreasing order of source count: one workgroup per
-        // box, so the longest ones start first and the launch ends evenly
-        int n4 = (int)P.p2l_boxes.size();
-        std::vector<int64_t> work(n4, 0);
-        for (int q = 0; q < n4; q++)
-            for (int k = P.p2l_start[q]; k < P.p2l_start[q + 1]; k++) work[q] += T.src_count[P.p2l_items[k]];
-        std::vector<int> ord(n4);
-        for (int q = 0; q < n4; q++) ord[q] = q;
-        std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return work[a] > work[b]; });
-        std::vector<int> bx(n4), st(1, 0), it;
-        it.reserve(P.p2l_items.size());
-        for (int q = 0; q < n4; q++) {
-            int o = ord[q];
-            bx[q] = P.p2l_boxes[o];
-            it.insert(it.end(), P.p2l_items.begin() + P.p2l_start[o], P.p2l_items.begin() + P.p2l_start[o + 1]);
-            st.push_back((int)it.size());
-        }
-        P.p2l_boxes.swap(bx);
-        P.p2l_start.swap(st);
-        P.p2l_items.swap(it);
+        P.stats[7] = (double)std::count_if(P.m2l_tiles.begin(), P.m2l_tiles.end(), [](const M2LTile &t) { return t.npair > 0; });
+        P.stats[9] = l2l_pairs;
     }
+}
 
+void build_plan_eval(const Tree &T, int n, const Operators *ops, bool src_eval, Plan &P, bool iter)
+{
+    int nb = T.nboxes;
+    auto npts = [&](int b) { return (src_eval ? T.src_count[b] : 0) + T.tgt_count[b]; };
     // L2T: the leaves with points at level >= 2
     for (int b = 0; b < nb; b++)
         if (!T.nkids[b] && npts(b) && ops && T.level[b] >= 2) P.l2t_boxes.push_back(b);
@@ -468,32 +499,28 @@ void build_plan_far(const Tree &T, int n, const Operators *ops, bool src_eval, i
         });
         wave_tasks(off, P.l2t_wt);
     }
-    if (!P.m2t_items.empty()) {
-        // slots in order of first use; the owners of each slot in order
-        std::vector<int> slot_of(nb, -1), nown;
-        for (size_t q = 0; q < P.m2t_boxes.size(); q++)
-            for (int k = P.m2t_start[q]; k < P.m2t_start[q + 1]; k++) {
-                int i = P.m2t_items[k];
-                if (slot_of[i] < 0) {
-                    slot_of[i] = (int)P.m2t_slot_box.size();
-                    P.m2t_slot_box.push_back(i);
-                    nown.push_back(0);
-                }
-                nown[slot_of[i]]++;
-            }
-        int ns = (int)P.m2t_slot_box.size();
-        std::vector<int> ostart(ns + 1, 0);
-        for (int sl = 0; sl < ns; sl++) ostart[sl + 1] = ostart[sl] + nown[sl];
-        std::vector<int> owners(ostart[ns]), fill(ostart.begin(), ostart.end() - 1);
-        for (size_t q = 0; q < P.m2t_boxes.size(); q++)
-            for (int k = P.m2t_start[q]; k < P.m2t_start[q + 1]; k++)
-                owners[fill[slot_of[P.m2t_items[k]]]++] = P.m2t_boxes[q];
-        std::vector<int64_t> toff(ns + 1, 0);
-        for (int sl = 0; sl < ns; sl++) {
+    // M2T: multipole of i at the points of j with j in list4(i)
+    // (src/lfmm3dtrilhess.f:864-981): a slot per sourced box i, its owners the
+    // boxes with points of list 4, the dual of list 3
+    if (ops && !iter) {
+        std::vector<int> ostart(1, 0);
+        std::vector<int64_t> toff(1, 0);
+        for (int i = 0; i < nb; i++) {
+            if (!T.src_count[i]) continue;
             int64_t t = 0;
-            for (int k = ostart[sl]; k < ostart[sl + 1]; k++) t += npts(owners[k]);
-            toff[sl + 1] = toff[sl] + t;
+            for (int q = T.lstart[4][i]; q < T.lstart[4][i + 1]; q++) {
+                int j = T.litems[4][q];
+                if (!npts(j)) continue;
+                P.m2t_items.push_back(j);
+                t += npts(j);
+            }
+            if (!t) continue;
+            P.m2t_slot_box.push_back(i);
+            ostart.push_back((int)P.m2t_items.size());
+            toff.push_back(toff.back() + t);
         }
+        int ns = (int)P.m2t_slot_box.size();
+        const std::vector<int> &owners = P.m2t_items;
         P.m2t_tpt.resize(toff[ns]);
         parallel_chunks((ns + CHUNK - 1) / CHUNK, [&](int ch, int) {
             for (int sl = ch * CHUNK; sl < std::min(ns, (ch + 1) * CHUNK); sl++) {
@@ -509,21 +536,8 @@ void build_plan_far(const Tree &T, int n, const Operators *ops, bool src_eval, i
         int nw = (int)P.m2t_wt.size() / 3;
         for (int w = 0; w < nw; w++)
             if (w == 0 || P.m2t_wt[3 * w] != P.m2t_wt[3 * (w - 1)] || w - P.m2t_bt.back() == 4) P.m2t_bt.push_back(w);
-        P.m2t_bt.push_back(nw);
+        if (nw) P.m2t_bt.push_back(nw);
     }
-
-    // remaining work counts (elfmm_gfx950_last_stats)
-    P.stats[0] = nb;
-    P.stats[1] = T.nlev;
-    P.stats[2] = p;
-    P.stats[7] = (double)std::count_if(P.m2l_tiles.begin(), P.m2l_tiles.end(), [](const M2LTile &t) { return t.npair > 0; });
-    double m2m_pairs = 0, l2l_pairs = 0;
-    for (auto &g : P.m2m_l) m2m_pairs += g.src.size();
-    for (auto &g : P.l2l_l) l2l_pairs += g.src.size();
-    P.stats[8] = m2m_pairs;
-    P.stats[9] = l2l_pairs;
-    P.stats[10] = (double)P.p2m_boxes.size();
-    P.stats[11] = (double)P.p2l_items.size();
     P.stats[12] = (double)P.m2t_items.size();
     P.stats[13] = (double)P.l2t_boxes.size();
 }
