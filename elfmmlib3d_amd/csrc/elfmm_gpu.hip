@@ -534,15 +534,16 @@ __global__ __launch_bounds__(64 * WB, TW <= 7 ? 4 : 2) void k_p2l(
 
 
 // P2M and P2L of triangles through their moments (elfmm_moments.h)
-template <class Z>
+template <class Z, bool MIND>
 __global__ __launch_bounds__(Z::NT, 2) void k_p2m_tri(
-    int p, const int *__restrict__ boxes, const double *__restrict__ centers, const double *__restrict__ sides,
-    const int *__restrict__ src_start, const int *__restrict__ src_count, const double *__restrict__ tri_s,
-    const double *__restrict__ tcoef, int nc, double *__restrict__ expn)
+    int p, const int *__restrict__ boxes, const int *__restrict__ parts, MindMoments mind,
+    const double *__restrict__ centers, const double *__restrict__ sides, const int *__restrict__ src_start,
+    const int *__restrict__ src_count, const double *__restrict__ tri_s, const double *__restrict__ tcoef, int nc,
+    double *__restrict__ expn)
 {
     extern __shared__ double lds[];                  // no static LDS beside it: it starts at 0
-    p2t_body<false, Z>(p, boxes, nullptr, nullptr, centers, sides, src_start, src_count, tri_s, tcoef, nc, expn,
-                       lds);
+    p2t_body<false, Z, MIND>(p, boxes, parts, mind, nullptr, nullptr, centers, sides, src_start, src_count, tri_s,
+                             tcoef, nc, expn, lds);
 }
 
 template <class Z>
@@ -553,8 +554,8 @@ __global__ __launch_bounds__(Z::NT, 2) void k_p2l_tri(
     double *__restrict__ expn)
 {
     extern __shared__ double lds[];                  // no static LDS beside it: it starts at 0
-    p2t_body<true, Z>(p, boxes, lstart, litems, centers, sides, src_start, src_count, tri_s, tcoef, nc, expn,
-                      lds);
+    p2t_body<true, Z, false>(p, boxes, nullptr, MindMoments{}, lstart, litems, centers, sides, src_start, src_count,
+                             tri_s, tcoef, nc, expn, lds);
 }
 
 // ------------------------------------------------------------------------
@@ -1859,9 +1860,9 @@ struct OpsCache {
     // offsets (|dz| <= 1) and the plane-wave / proxy tables
     bool mind_ready = false;
     Operators mind_ops;
-    DevBuf mind_m2l, mind_tab;
+    DevBuf mind_m2l, mind_tab, mind_px, mind_pxo;    // ..., proxy matrices and their offsets
     MindPw mind_pw{};
-    int mind_nq = 0, mind_nquad = 0;
+    int mind_nq = 0;
     size_t mind_off[8] = {};                         // ycst, gl, ytab, eph, wl, pw tab, pw ints
 };
 
@@ -1914,8 +1915,10 @@ DeviceState &device_state()
             int ph = 0;
             while (Z::fits(ph + 1)) ph++;
             int b = Z::lds(ph) * 8;
-            return hipFuncSetAttribute((const void *)k_p2m_tri<Z>, hipFuncAttributeMaxDynamicSharedMemorySize, b) ==
-                       hipSuccess &&
+            return hipFuncSetAttribute((const void *)k_p2m_tri<Z, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       b) == hipSuccess &&
+                   hipFuncSetAttribute((const void *)k_p2m_tri<Z, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       b) == hipSuccess &&
                    hipFuncSetAttribute((const void *)k_p2l_tri<Z>, hipFuncAttributeMaxDynamicSharedMemorySize, b) ==
                        hipSuccess;
         };
@@ -2011,7 +2014,7 @@ constexpr int SET_LANES = 8;
 
 // Device buffers of one Mindlin far field.
 struct MindScratch {
-    DevBuf exps, pts, lap, inp, rec, pw, skel, gm;
+    DevBuf exps, pts, lap, inp, rec, pw, skel, gm, tcoef;
     std::shared_ptr<elfmm::MindPlan> plan;           // of the last far field (for a later assembly)
 };
 
@@ -2116,7 +2119,7 @@ int max_lds()
 // Offsets of the arrays of a tree and its plan, each in the packed device
 // buffer of its part (FarLaunch), which may be one and the same.
 struct PlanOffsets {
-    size_t iz, izt, cen, side, ss, sc, ts, tc, p2m, p2lb, p2ls, p2li, l2t, l2tp, m2tsb, m2tp, l2tw, m2tw, m2tbt;
+    size_t iz, izt, cen, side, ss, sc, ts, tc, p2m, p2mp, p2lb, p2ls, p2li, l2t, l2tp, m2tsb, m2tp, l2tw, m2tw, m2tbt;
     size_t nfb, nfs, nfi, nfw, m2lt;
     std::vector<LaunchOff> m2m, l2l;
     LaunchOff m2l;
@@ -2154,6 +2157,7 @@ void pack_up(Packer &pk, const Tree &T, const Plan &PL, PlanOffsets &o)
     o.cen = pk.add(T.centers);
     o.side = pk.add(PL.sides);
     o.p2m = pk.add(PL.p2m_boxes);
+    o.p2mp = pk.add(PL.p2m_parts);
     o.p2lb = pk.add(PL.p2l_boxes);
     o.p2ls = pk.add(PL.p2l_start);
     o.p2li = pk.add(PL.p2l_items);
@@ -2269,8 +2273,8 @@ void enqueue_up(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
             ln.launch(k_p2l_tri<Z>, dim3(nbx), dim3(Z::NT), sh, p, bx, ls, li, D(o.cen), D(o.side), ss, sc,
                       a.tri_s, (const double *)a.nodes, nc, out);
         else
-            ln.launch(k_p2m_tri<Z>, dim3(nbx), dim3(Z::NT), sh, p, bx, D(o.cen), D(o.side), ss, sc, a.tri_s,
-                      (const double *)a.nodes, nc, out);
+            ln.launch(k_p2m_tri<Z, false>, dim3(PL.p2m_parts.size() / 3), dim3(Z::NT), sh, p, bx, I(o.p2mp),
+                      MindMoments{}, D(o.cen), D(o.side), ss, sc, a.tri_s, (const double *)a.nodes, nc, out);
     };
     // P2M / P2L: moments on the matrix cores (shapes at P2X_WIDE_STRIDE)
     auto p2x = [&](bool irr, size_t nbx, const int *bx, const int *ls, const int *li, double *out) {
@@ -3307,8 +3311,18 @@ void mindlin_tables(OpsCache &oc, int iprec)
     pw.nfour = (const int *)(base + ioff[3]);
     pw.nphys = (const int *)(base + ioff[4]);
     oc.mind_nq = nq;
-    oc.mind_nquad = nquad;
-    mind_set_lds_limits(mind_proxy_lds(p, nquad, nq), mind_far_lds(ntp, foff[nl]));
+    mind_set_lds_limits(mind_far_lds(ntp, foff[nl]));
+    // proxy matrices of the near offsets
+    int index[343];
+    std::vector<int> offs = mind_proxy_offsets(index);
+    int noff = (int)offs.size() / 3;
+    oc.mind_pxo.ensure(offs.size() * 4);
+    HIPOK(hipMemcpy(oc.mind_pxo.p, offs.data(), offs.size() * 4, hipMemcpyHostToDevice));
+    oc.mind_px.ensure(mind_proxy_op_doubles(p, nq, noff) * 8);
+    HIPOK(launch_mind_proxy_op(p, nq, nquad, noff, oc.mind_pxo.get<int>(), (const double *)(base + doff[1]),
+                               (const double *)(base + doff[2]), (const double *)(base + doff[3]),
+                               oc.mind_px.get<double>(), nullptr));
+    HIPOK(hipStreamSynchronize(nullptr));
     oc.mind_ready = true;
 }
 
@@ -3324,7 +3338,7 @@ struct MindPlan {
     std::vector<std::vector<int>> bsc;        // per M2M launch: boxes whose B is rescaled after it
     DevBuf dev;                               // packed plan
     size_t o_iz, o_izt, o_cen, o_side, o_lev, o_ss, o_sc, o_p2m, o_l2t, o_l2tp, o_l2tw, o_src, o_slot, o_fb, o_fs,
-        o_fi, o_nb, o_ns, o_ni;
+        o_fi, o_px, o_parts;
     std::vector<size_t> o_bsc;
     std::vector<LaunchOff> off_m2m, off_l2l;
     LaunchOff off_m2l;
@@ -3395,9 +3409,8 @@ int build_mind_plan(OpsCache &oc, int iprec, int n, const double *d_src, int nt,
     M.o_fb = pk.add(MP.far_boxes);
     M.o_fs = pk.add(MP.far_start);
     M.o_fi = pk.add(MP.far_items);
-    M.o_nb = pk.add(MP.near_boxes);
-    M.o_ns = pk.add(MP.near_start);
-    M.o_ni = pk.add(MP.near_items);
+    M.o_px = pk.add(MP.px_tasks);
+    M.o_parts = pk.add(PL.p2m_parts);
     for (auto &v : M.bsc) M.o_bsc.push_back(pk.add(v));
     auto add_launch = [&](const GemmLaunch &g) {
         LaunchOff o;
@@ -3498,17 +3511,42 @@ int mindlin_far_dev(int iprec, double rlam, double rmu, int n, const double *d_t
     md.slot = I(M.o_slot);
     md.ycst = (const double *)(tb + oc->mind_off[0]);
     md.nq = oc->mind_nq;
-    md.nquad = oc->mind_nquad;
     md.pwo = S.pw.get<double>();
     md.skel = S.skel.get<double>();
-    md.gl = (const double *)(tb + oc->mind_off[1]);
-    md.ytab = (const double *)(tb + oc->mind_off[2]);
-    md.eph = (const double *)(tb + oc->mind_off[3]);
+    md.pxoffs = oc->mind_pxo.get<int>();
+    md.pxop = oc->mind_px.get<double>();
     md.wl = (const double *)(tb + oc->mind_off[4]);
     S.gm.ensure(mind_p2m_scratch_bytes(p, (int)PL.p2m_boxes.size()));
     md.gmom = S.gm.get<double>();
     // upward pass
-    HIPOK(launch_mind_p2m(md, I(M.o_p2m), (int)PL.p2m_boxes.size(), stream));
+    const int nbx = (int)PL.p2m_boxes.size(), nown = nc / 2;
+    const int nqn = iprec >= 1 ? 12 : iprec == 0 ? 6 : 3, shape = dsp->p2t ? p2t_shape(p, nqn) : -1;
+    if (nbx && shape >= 0) {
+        // triangle moments (elfmm_moments.h), one layer at a time: 6 or 12 columns
+        HIPOK(launch_fill0(S.gm.get<double>(), (size_t)2 * nbx * MindMoments::MCOLS * nown, stream));
+        S.tcoef.ensure((size_t)48 * n * 8);
+        for (int dl = 0; dl < 2; dl++) {
+            if (!(dl ? ifdl : ifsl)) continue;
+            hipLaunchKernelGGL(k_mind_tcoef, dim3((n + 255) / 256), dim3(256), 0, stream, n, dl, tri_s, nrm_s,
+                               dl ? sdl_s : ssl_s, S.tcoef.get<double>());
+            HIPOK(hipGetLastError());
+            MindMoments mm;
+            for (int c = 0; c < 16; c++) mm.col[c] = dl ? (c < 12 ? 6 + c : -1) : (c < 6 ? c : -1);
+            mm.G = S.gm.get<double2>();
+            auto run = [&](auto z) {
+                using Z = decltype(z);
+                hipLaunchKernelGGL((k_p2m_tri<Z, true>), dim3(PL.p2m_parts.size() / 3), dim3(Z::NT),
+                                   (size_t)Z::lds(p) * 8, stream, p, I(M.o_p2m), I(M.o_parts), mm, D(M.o_cen),
+                                   D(M.o_side), I(M.o_ss), I(M.o_sc), tri_s, S.tcoef.get<double>(), nc,
+                                   (double *)nullptr);
+                HIPOK(hipGetLastError());
+            };
+            shape == 0 ? run(P2TShape0{}) : shape == 1 ? run(P2TShape1{}) : shape == 2 ? run(P2TShape2{}) : run(P2TShape3{});
+        }
+        HIPOK(launch_mind_combine(md, I(M.o_p2m), nbx, stream));
+    } else {
+        HIPOK(launch_mind_p2m(md, I(M.o_p2m), nbx, stream));
+    }
     auto run_trans = [&](const GemmLaunch &g, const LaunchOff &o, const double *A, const double *X, double *Y,
                          bool m2l) {
         if (g.tiles.empty()) return;
@@ -3532,7 +3570,7 @@ int mindlin_far_dev(int iprec, double rlam, double rmu, int n, const double *d_t
     // list 2: near pairs (exact M2L of the remainder of B, and of C1, C2;
     // the proxies' field), far pairs (plane waves)
     run_trans(MP.m2l, M.off_m2l, oc->mind_m2l.get<double>(), mp, lo, true);
-    HIPOK(launch_mind_proxy(md, I(M.o_nb), I(M.o_ns), I(M.o_ni), (int)MP.near_boxes.size(), stream));
+    HIPOK(launch_mind_proxy(md, I(M.o_px), (int)MP.px_tasks.size() / 3, I(M.off_m2l.src), I(M.off_m2l.dst), stream));
     HIPOK(launch_mind_far(md, I(M.o_fb), I(M.o_fs), I(M.o_fi), (int)MP.far_boxes.size(), stream));
     // downward pass and evaluation
     for (size_t k = 0; k < PL.l2l_l.size(); k++)

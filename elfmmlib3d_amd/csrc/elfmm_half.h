@@ -67,22 +67,31 @@ struct MindDev {
     MindPw pw;
     const int *slot;              // per box: plane-wave / proxy slot (-1: none)
     const double *ycst;           // ylgndr(p, 1/sqrt(3))
-    int nq, nquad;                // proxy charges per ring; sphere quadrature size
+    int nq;                       // proxy charges per ring
     double *pwo, *skel;           // outgoing plane waves, proxy charges
-    const double *gl, *ytab, *eph, *wl;
+    const double *wl;
+    const int *pxoffs;            // offsets of the proxy matrices (3 per matrix), and the matrices
+    const double *pxop;
     double *gmom;                 // P2M moments, mind_p2m_scratch_bytes
 };
 // scratch of launch_mind_p2m for nbx boxes
 size_t mind_p2m_scratch_bytes(int p, int nbx);
+// P2M of nbx boxes: the moments (3-node rule) and the expansions from them; the
+// second step alone
 hipError_t launch_mind_p2m(const MindDev &d, const int *boxes, int nbx, hipStream_t st);
+hipError_t launch_mind_combine(const MindDev &d, const int *boxes, int nbx, hipStream_t st);
 hipError_t launch_mind_bscale(const MindDev &d, const int *boxes, int nbx, hipStream_t st);
 hipError_t launch_mind_bmod(const MindDev &d, const int *boxes, int nbx, hipStream_t st);
-hipError_t launch_mind_proxy(const MindDev &d, const int *tb, const int *ts, const int *ti, int nbx, hipStream_t st);
+// matrices of the proxy rings' field for noff box offsets (3 ints each)
+size_t mind_proxy_op_doubles(int p, int nq, int noff);
+hipError_t launch_mind_proxy_op(int p, int nq, int nquad, int noff, const int *offs, const double *gl,
+                                const double *ytab, const double *eph, double *op, hipStream_t st);
+hipError_t launch_mind_proxy(const MindDev &d, const int *task, int ntask, const int *psrc, const int *pdst,
+                             hipStream_t st);
 hipError_t launch_mind_far(const MindDev &d, const int *tb, const int *ts, const int *ti, int nbx, hipStream_t st);
 hipError_t launch_mind_assemble(int n, int nt, const int *izt, const double *pts, const double *lap, double mu,
                                 int ifpt, double *ptt, int ifst, double *stt, hipStream_t st);
-size_t mind_proxy_lds(int p, int nquad, int nq);
 size_t mind_far_lds(int nexptotp, int nexptot);
-void mind_set_lds_limits(size_t proxy, size_t far);
+void mind_set_lds_limits(size_t far);
 
 }  // namespace elfmm

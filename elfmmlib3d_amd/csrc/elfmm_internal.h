@@ -133,6 +133,7 @@ struct LaunchOff {
 struct Plan {
     std::vector<double> sides;                       // per box
     std::vector<int> p2m_boxes;                      // leaves forming a multipole
+    std::vector<int> p2m_parts;                      // P2M workgroups of triangles: (box of the list, first, triangles)
     std::vector<GemmLaunch> m2m_l, l2l_l;            // one launch per level
     GemmLaunch m2l;                                  // all list-2 pairs, grouped by offset (src/dst/scale)
     std::vector<M2LTile> m2l_tiles;                  // rotated-M2L tiles over those pairs
@@ -184,10 +185,10 @@ struct MindlinPlan {
     std::vector<int> src_boxes;                // boxes of level >= 2 with sources
     std::vector<int> b_scale_boxes[64];        // per level: boxes with sources and kids (B rescaled after M2M)
     // per target box of level >= 2 with targets: far list-2 sources (|dz| >=
-    // 1.5 sides: plane waves), near ones (proxy-charge local); CSR
+    // 1.5 sides: plane waves); CSR
     std::vector<int> far_boxes, far_start, far_items;
-    std::vector<int> near_boxes, near_start, near_items;
     GemmLaunch m2l;                            // near pairs, grouped by offset (full order)
+    std::vector<int> px_tasks;                 // proxy fields of the near pairs: (matrix, first pair, pairs <= MIND_PX)
     std::vector<M2LTile> m2l_tiles;
     std::vector<int> pw_slot;                  // per box: plane-wave slot (-1: none)
     int npw = 0;
@@ -195,5 +196,10 @@ struct MindlinPlan {
 // ops: translation operators of full order p for the near offsets
 // (|dz| <= 1) of list 2.
 void build_mindlin_plan(const Tree &T, const Operators &ops, MindlinPlan &MP);
+constexpr int MIND_PX = 8;
+// The box offsets (source minus target, in sides) of near list-2 pairs,
+// |k| <= 1 and not adjacent: 3 ints per proxy matrix; index[343] the matrix of
+// offset (i+3)*49 + (j+3)*7 + (k+3), -1 if none.
+std::vector<int> mind_proxy_offsets(int *index);
 
 }  // namespace elfmm

@@ -16,11 +16,11 @@
 namespace elfmm {
 
 constexpr int MW = 256;                      // threads per workgroup
-constexpr int MPX = 1024;                    // threads per workgroup of the proxy projection
 constexpr int MP_MAX = 39;                   // largest supported order (iprec 3)
 constexpr int MH = (MP_MAX + 1) * (MP_MAX + 2) / 2;
 constexpr int MPW_FOUR = 544;                // Fourier modes of the largest plane-wave table (525)
-constexpr size_t MIND_P2M_LDS = 100 * 1024;   // LDS of the P2M moment pass
+constexpr size_t MIND_P2M_LDS = 100 * 1024;   // LDS and threads of the P2M moment pass
+constexpr int MIND_P2M_NT = 512;
 
 // rows 0-2: order 2, rows 3-8: order 4, rows 9-20: order 6
 __constant__ double c_mrule[21][3] = {ELFMM_RULE2, ELFMM_RULE4, ELFMM_RULE6};
@@ -105,15 +105,15 @@ __device__ __forceinline__ double lmn(int l, int m)
 
 constexpr int MCOLS = 18;
 
-// Pass 1: one workgroup per box, thread = coefficient (l, m). The columns
+// Pass 1 (for the 3-node rule; rules of 6 and 12 nodes go through
+// elfmm_moments.h): one workgroup per box, thread = coefficient (l, m). The columns
 // are per-triangle values times per-node factors: a triangle's moments are
 // its 9 values (sigma_sl, q) times U = sum_nodes w R(x) and U' = sum_nodes
 // w y3 R(x), w = rule weight * 2 * area. Nodes go through LDS nch at a time
 // (their harmonics by column recurrences with the constants tabulated in
 // LDS); each thread folds a finished triangle into its 18 moments.
-// NT >= (p+1)(p+2)/2.
-template <int NT>
-__global__ __launch_bounds__(NT) void k_mind_moments(MindArgs a, const int *__restrict__ boxes, int nch,
+// MIND_P2M_NT >= (p+1)(p+2)/2.
+__global__ __launch_bounds__(MIND_P2M_NT) void k_mind_moments(MindArgs a, const int *__restrict__ boxes, int nch,
                                                      double2 *__restrict__ G)
 {
     extern __shared__ double smem[];
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(NT) void k_mind_moments(MindArgs a, const int *__re
     double *Xs = Tv + 9 * nch;                              // [nch][3] node - centre
     int *Is = (int *)(Xs + 3 * nch);                        // [nch] triangle of the node (in the box)
     int tid = threadIdx.x;
-    for (int k = tid; k < nown; k += NT) {
+    for (int k = tid; k < nown; k += MIND_P2M_NT) {
         int l = 0;
         while ((l + 1) * (l + 2) / 2 <= k) l++;
         int m = k - l * (l + 1) / 2;
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(NT) void k_mind_moments(MindArgs a, const int *__re
         }
         Rc[k] = make_double2(ca, cb);
     }
-    for (int k = tid; k <= p; k += NT) Dg[k] = k ? sqrt((2.0 * k - 1) / (2.0 * k)) : 1.0;
+    for (int k = tid; k <= p; k += MIND_P2M_NT) Dg[k] = k ? sqrt((2.0 * k - 1) / (2.0 * k)) : 1.0;
     int b = boxes[blockIdx.x];
     const double *c = a.centers + 3 * (size_t)b;
     int q0 = a.nqtri == 2 ? 0 : a.nqtri == 4 ? 3 : 9, q1 = a.nqtri == 2 ? 3 : a.nqtri == 4 ? 9 : 21;
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(NT) void k_mind_moments(MindArgs a, const int *__re
         }
         __syncthreads();
         // harmonics of the chunk's nodes, one column (node, m) per task
-        for (int task = tid; task < nk * (p + 1); task += NT) {
+        for (int task = tid; task < nk * (p + 1); task += MIND_P2M_NT) {
             int k = task / (p + 1), m = task % (p + 1);
             double x = Xs[3 * k], y = Xs[3 * k + 1], z = Xs[3 * k + 2];
             double2 *H = Hs + (size_t)k * nown;
@@ -566,86 +566,113 @@ __global__ __launch_bounds__(MW) void k_mind_bmod(MindArgs a, MindPw pw, const i
     }
 }
 
-// Per target box: the U-field of the proxy rings of each near list-2 source
-// box, tabulated on the sphere about the target centre and projected on
-// the local expansion of B (l3dformtaintkerbf90sc, src/mindlinformta.f:980).
+// The U-field of the proxy rings of a near list-2 source box, tabulated on the
+// sphere about the target centre and projected on the local expansion of B
+// (l3dformtaintkerbf90sc, src/mindlinformta.f:980), is linear in the charges and,
+// for boxes of side s, U(s x) = s (U(x) - x_3 log s): one matrix per offset of
+// the two boxes in sides serves every pair, level and density (charges x
+// coefficients), beside a term of degrees 0 and 1 for log s. Evaluating the
+// kernel per pair instead (nquad^2 points x 2 nq charges, a square root and a
+// logarithm each, 281,000 at order 26) took 5.1 ms of the 20,020-triangle
+// fault mesh's product; the matrices take 0.11 ms there, and 1.3 ms
+// once per precision to build.
+
+// Matrix of one charge (blockIdx.x) and offset (blockIdx.y, source box minus
+// target box, in sides): op[offset][charge][2 coefficient + part].
 // gl: Gauss-Legendre nodes (nquad) then weights (nquad); ytab: ylgndr at the
 // nodes, [nquad][(p+1)^2]; eph: e^{-i m 2 pi (k+1)/nquad}, [m][nquad].
-__global__ __launch_bounds__(MPX) void k_mind_proxy(MindArgs a, const int *__restrict__ tboxes,
-                                                   const int *__restrict__ tstart, const int *__restrict__ titems,
-                                                   const int *__restrict__ slot, const double *__restrict__ skel,
-                                                   int nq, int nquad, const double *__restrict__ gl,
-                                                   const double *__restrict__ ytab, const double2 *__restrict__ eph)
+__global__ __launch_bounds__(MW) void k_mind_proxy_op(int p, int nq, int nquad, const int *__restrict__ offs,
+                                                     const double *__restrict__ gl, const double *__restrict__ ytab,
+                                                     const double2 *__restrict__ eph, double *__restrict__ op)
 {
     extern __shared__ double smem[];
     double *phi = smem;                                   // nquad * nquad
     double2 *marr = (double2 *)(smem + nquad * nquad);    // nquad * (p + 1)
-    double *sk = (double *)(marr + nquad * (a.p + 1));    // 2 nq * 4
-    int t = tboxes[blockIdx.x];
-    int p = a.p, nown = (p + 1) * (p + 2) / 2;
-    double side = a.tsize / (double)(1 << a.level[t]);
-    const double *c = a.centers + 3 * (size_t)t;
-    double al = (a.lam + a.mu) / (a.lam + 2 * a.mu);
-    double radius = side * sqrt(3.0) / 2;
-    double rs = side / radius;                            // 1 / (rscale * radius)
-    double2 acc[2] = {make_double2(0, 0), make_double2(0, 0)};
-    for (int it = tstart[blockIdx.x]; it < tstart[blockIdx.x + 1]; it++) {
-        int s = titems[it];
-        double sside = a.tsize / (double)(1 << a.level[s]);
-        double sc = (1.0 - al) / al / sside;              // times the source box's scale
-        const double *ks = skel + (size_t)slot[s] * 2 * nq * 4;
-        __syncthreads();
-        for (int k = threadIdx.x; k < 2 * nq * 4; k += MPX) sk[k] = ks[k];
-        __syncthreads();
-        for (int g = threadIdx.x; g < nquad * nquad; g += MPX) {
-            int jj = g / nquad, kk = g % nquad;
-            double cth = gl[jj], sth = sqrt(1.0 - cth * cth);
-            double ph = 2 * M_PI * (kk + 1) / nquad;
-            double tx = c[0] + radius * sth * cos(ph), ty = c[1] + radius * sth * sin(ph), tz = c[2] + radius * cth;
-            double v = 0.0;
-            for (int i = 0; i < 2 * nq; i++) {
-                double r1 = tx - sk[4 * i], r2 = ty - sk[4 * i + 1], r3 = tz - sk[4 * i + 2];
-                double rr = sqrt(r1 * r1 + r2 * r2 + r3 * r3);
-                v += sk[4 * i + 3] * (-r3 * log(rr - r3) - rr);
-            }
-            phi[g] = v * sc;
-        }
-        __syncthreads();
-        for (int g = threadIdx.x; g < nquad * (p + 1); g += MPX) {
-            int jj = g / (p + 1), m = g % (p + 1);
-            double sr = 0, si = 0;
-            for (int kk = 0; kk < nquad; kk++) {
-                double2 e = eph[m * nquad + kk];
-                sr += phi[jj * nquad + kk] * e.x;
-                si += phi[jj * nquad + kk] * e.y;
-            }
-            marr[jj * (p + 1) + m] = make_double2(sr / (2 * nquad) * gl[nquad + jj], si / (2 * nquad) * gl[nquad + jj]);
-        }
-        __syncthreads();
-        for (int k = 0; k < 2; k++) {
-            int idx = threadIdx.x + k * MPX;
-            if (idx >= nown) break;
-            int l = 0;
-            while ((l + 1) * (l + 2) / 2 <= idx) l++;
-            int m = idx - l * (l + 1) / 2;
-            double f0 = sqrt(2 * l + 1.0) * pow(rs, (double)l);
-            double sr = 0, si = 0;
-            for (int jj = 0; jj < nquad; jj++) {
-                double y = ytab[(size_t)jj * (p + 1) * (p + 1) + l * (p + 1) + m];
-                double2 mv = marr[jj * (p + 1) + m];
-                sr += mv.x * y;
-                si += mv.y * y;
-            }
-            acc[k].x += sr * f0;
-            acc[k].y += si * f0;
-        }
+    const int nown = (p + 1) * (p + 2) / 2;
+    const double radius = sqrt(3.0) / 2, ct = 1.0 / sqrt(3.0), st = sqrt(2.0 / 3.0), rs = 1.0 / radius;
+    const int i = blockIdx.x, ring = i / nq;
+    const double ang = (i - ring * nq) * (2 * M_PI / nq);
+    const double xs = offs[3 * blockIdx.y] + radius * st * cos(ang), ys = offs[3 * blockIdx.y + 1] + radius * st * sin(ang),
+                 zs = offs[3 * blockIdx.y + 2] + (ring ? -radius * ct : radius * ct);
+    for (int g = threadIdx.x; g < nquad * nquad; g += MW) {
+        int jj = g / nquad, kk = g % nquad;
+        double cth = gl[jj], sth = sqrt(1.0 - cth * cth), ph = 2 * M_PI * (kk + 1) / nquad;
+        double r1 = radius * sth * cos(ph) - xs, r2 = radius * sth * sin(ph) - ys, r3 = radius * cth - zs;
+        double rr = sqrt(r1 * r1 + r2 * r2 + r3 * r3);
+        phi[g] = -r3 * log(rr - r3) - rr;
     }
-    for (int k = 0; k < 2; k++) {
-        int idx = threadIdx.x + k * MPX;
-        if (idx >= nown) break;
-        double *o = a.lo + (size_t)t * 4 * a.nc + 2 * idx;
-        o[0] += acc[k].x;
-        o[1] += acc[k].y;
+    __syncthreads();
+    for (int g = threadIdx.x; g < nquad * (p + 1); g += MW) {
+        int jj = g / (p + 1), m = g % (p + 1);
+        double sr = 0, si = 0;
+        for (int kk = 0; kk < nquad; kk++) {
+            double2 e = eph[m * nquad + kk];
+            sr += phi[jj * nquad + kk] * e.x;
+            si += phi[jj * nquad + kk] * e.y;
+        }
+        marr[g] = make_double2(sr / (2 * nquad) * gl[nquad + jj], si / (2 * nquad) * gl[nquad + jj]);
+    }
+    __syncthreads();
+    double *o = op + ((size_t)blockIdx.y * gridDim.x + i) * 2 * nown;
+    for (int idx = threadIdx.x; idx < nown; idx += MW) {
+        int l = 0;
+        while ((l + 1) * (l + 2) / 2 <= idx) l++;
+        int m = idx - l * (l + 1) / 2;
+        double f0 = sqrt(2 * l + 1.0) * pow(rs, (double)l);
+        double sr = 0, si = 0;
+        for (int jj = 0; jj < nquad; jj++) {
+            double y = ytab[(size_t)jj * (p + 1) * (p + 1) + l * (p + 1) + m];
+            double2 mv = marr[jj * (p + 1) + m];
+            sr += mv.x * y;
+            si += mv.y * y;
+        }
+        o[2 * idx] = sr * f0;
+        o[2 * idx + 1] = si * f0;
+    }
+}
+
+// Up to MIND_PX pairs of one offset per workgroup, MW rows of the local
+// expansions each (blockIdx.y): task = (matrix, first pair, pairs). The
+// matrix column of a charge is read once for all the pairs; their charges are
+// in LDS. Several pairs share a target box: FP64 atomic adds.
+__global__ __launch_bounds__(MW) void k_mind_proxy(MindArgs a, const int *__restrict__ task, const int *__restrict__ psrc,
+                                                   const int *__restrict__ pdst, const int *__restrict__ slot,
+                                                   const double *__restrict__ skel, int nq,
+                                                   const int *__restrict__ offs, const double *__restrict__ op)
+{
+    extern __shared__ __align__(16) double q[];            // [charge][MIND_PX]
+    const int o = task[3 * blockIdx.x], p0 = task[3 * blockIdx.x + 1], np = task[3 * blockIdx.x + 2];
+    const int rows = (a.p + 1) * (a.p + 2), row = blockIdx.y * MW + threadIdx.x;
+    for (int e = threadIdx.x; e < 2 * nq * MIND_PX; e += MW) {
+        int i = e / MIND_PX, k = e - i * MIND_PX;
+        q[e] = k < np ? skel[((size_t)slot[psrc[p0 + k]] * 2 * nq + i) * 4 + 3] : 0.0;
+    }
+    __syncthreads();
+    if (row >= rows) return;
+    const double *M = op + (size_t)o * 2 * nq * rows + row;
+    double acc[MIND_PX];
+#pragma unroll
+    for (int k = 0; k < MIND_PX; k++) acc[k] = 0.0;
+#pragma unroll 4
+    for (int i = 0; i < 2 * nq; i++) {
+        double v = M[(size_t)i * rows];
+#pragma unroll
+        for (int k = 0; k < MIND_PX; k++) acc[k] += v * q[i * MIND_PX + k];
+    }
+    const double al = (a.lam + a.mu) / (a.lam + 2 * a.mu), f = (1.0 - al) / al;
+    for (int k = 0; k < np; k++) {
+        int t = pdst[p0 + k];
+        double v = acc[k];
+        if (row == 0 || row == 2) {                        // (0, 0) and (1, 0): the log s term
+            double s = 0.0, z = 0.0;
+            for (int i = 0; i < 2 * nq; i++) {
+                s += q[i * MIND_PX + k];
+                z += q[i * MIND_PX + k] * (offs[3 * o + 2] + (i < nq ? 0.5 : -0.5));
+            }
+            double ls = log(a.tsize / (double)(1 << a.level[t]));
+            v += row == 0 ? ls * z : -ls * s;
+        }
+        unsafeAtomicAdd(a.lo + (size_t)t * 4 * a.nc + row, f * v);
     }
 }
 
@@ -818,13 +845,16 @@ hipError_t launch_mind_p2m(const MindDev &d, const int *boxes, int nbx, hipStrea
     int nown = (a.p + 1) * (a.p + 2) / 2;
     int nch = (int)mind_p2m_nch(a.p);
     size_t sh = mind_p2m_lds(a.p, nch);
-    if (nown <= 512)
-        hipLaunchKernelGGL(k_mind_moments<512>, dim3(nbx), dim3(512), sh, st, a, boxes, nch, (double2 *)d.gmom);
-    else
-        hipLaunchKernelGGL(k_mind_moments<1024>, dim3(nbx), dim3(1024), sh, st, a, boxes, nch, (double2 *)d.gmom);
+    if (nown > MIND_P2M_NT) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_mind_moments, dim3(nbx), dim3(MIND_P2M_NT), sh, st, a, boxes, nch, (double2 *)d.gmom);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    size_t nth = (size_t)nbx * nown;
+    return e != hipSuccess ? e : launch_mind_combine(d, boxes, nbx, st);
+}
+
+hipError_t launch_mind_combine(const MindDev &d, const int *boxes, int nbx, hipStream_t st)
+{
+    const MindArgs &a = d.args;
+    size_t nth = (size_t)nbx * (a.p + 1) * (a.p + 2) / 2;
     hipLaunchKernelGGL(k_mind_p2m_combine, dim3((unsigned)((nth + 255) / 256)), dim3(256), 0, st, a, boxes, nbx,
                        (const double2 *)d.gmom);
     return hipGetLastError();
@@ -846,13 +876,27 @@ hipError_t launch_mind_bmod(const MindDev &d, const int *boxes, int nbx, hipStre
     return hipGetLastError();
 }
 
-hipError_t launch_mind_proxy(const MindDev &d, const int *tb, const int *ts, const int *ti, int nbx, hipStream_t st)
+size_t mind_proxy_op_doubles(int p, int nq, int noff) { return (size_t)noff * 2 * nq * (p + 1) * (p + 2); }
+
+hipError_t launch_mind_proxy_op(int p, int nq, int nquad, int noff, const int *offs, const double *gl,
+                                const double *ytab, const double *eph, double *op, hipStream_t st)
 {
-    if (nbx <= 0) return hipSuccess;
+    size_t sh = (size_t)nquad * nquad * 8 + (size_t)nquad * (p + 1) * 16;
+    hipError_t e = hipFuncSetAttribute((const void *)k_mind_proxy_op, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_mind_proxy_op, dim3(2 * nq, noff), dim3(MW), sh, st, p, nq, nquad, offs, gl, ytab,
+                       (const double2 *)eph, op);
+    return hipGetLastError();
+}
+
+hipError_t launch_mind_proxy(const MindDev &d, const int *task, int ntask, const int *psrc, const int *pdst,
+                             hipStream_t st)
+{
+    if (ntask <= 0) return hipSuccess;
     const MindArgs &a = d.args;
-    size_t sh = (size_t)d.nquad * d.nquad * 8 + (size_t)d.nquad * (a.p + 1) * 16 + (size_t)2 * d.nq * 4 * 8;
-    hipLaunchKernelGGL(k_mind_proxy, dim3(nbx), dim3(MPX), sh, st, a, tb, ts, ti, d.slot, d.skel, d.nq, d.nquad, d.gl,
-                       d.ytab, (const double2 *)d.eph);
+    int rows = (a.p + 1) * (a.p + 2);
+    hipLaunchKernelGGL(k_mind_proxy, dim3(ntask, (rows + MW - 1) / MW), dim3(MW), (size_t)2 * d.nq * MIND_PX * 8, st, a,
+                       task, psrc, pdst, d.slot, d.skel, d.nq, d.pxoffs, d.pxop);
     return hipGetLastError();
 }
 
@@ -875,20 +919,12 @@ hipError_t launch_mind_assemble(int n, int nt, const int *izt, const double *pts
     return hipGetLastError();
 }
 
-size_t mind_proxy_lds(int p, int nquad, int nq)
-{
-    return (size_t)nquad * nquad * 8 + (size_t)nquad * (p + 1) * 16 + (size_t)2 * nq * 4 * 8;
-}
-
 size_t mind_far_lds(int nexptotp, int nexptot) { return (size_t)3 * (nexptotp + nexptot) * 16; }
 
-void mind_set_lds_limits(size_t proxy, size_t far)
+void mind_set_lds_limits(size_t far)
 {
-    (void)hipFuncSetAttribute((const void *)k_mind_proxy, hipFuncAttributeMaxDynamicSharedMemorySize, (int)proxy);
     (void)hipFuncSetAttribute((const void *)k_mind_far, hipFuncAttributeMaxDynamicSharedMemorySize, (int)far);
-    (void)hipFuncSetAttribute((const void *)k_mind_moments<512>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)MIND_P2M_LDS);
-    (void)hipFuncSetAttribute((const void *)k_mind_moments<1024>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    (void)hipFuncSetAttribute((const void *)k_mind_moments, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)MIND_P2M_LDS);
     (void)hipGetLastError();
 }

@@ -112,6 +112,39 @@ __global__ void k_tcoef(int n, const double *__restrict__ tri_s, const double *_
     }
 }
 
+// The same for the Mindlin moments of one layer, whose sums are the same with
+// other columns (the 20,020-triangle fault mesh: 0.33 ms for both layers, 1.38
+// from the 12 nodes' harmonics per triangle; the densities of
+// elfmm_mindlin.hip, k_mind_moments): values v (single layer: sigma_sl; double:
+// the six sym-pairs of sigma_dl and the normal) in columns 0.., y3 v behind
+// them, y3 = the node's height, linear over the triangle.
+__global__ void k_mind_tcoef(int n, int dl, const double *__restrict__ tri_s, const double *__restrict__ nrm_s,
+                             const double *__restrict__ den_s, double *__restrict__ tcoef)
+{
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const double *t = tri_s + 9 * (size_t)i, *b = den_s + 3 * (size_t)i, *nv = nrm_s + 3 * (size_t)i;
+    double ax = t[3] - t[0], ay = t[4] - t[1], az = t[5] - t[2];
+    double bx = t[6] - t[0], by = t[7] - t[1], bz = t[8] - t[2];
+    double cx = ay * bz - az * by, cy = az * bx - ax * bz, cz = ax * by - ay * bx;
+    double w = sqrt(cx * cx + cy * cy + cz * cz);    // 2 x area
+    double v[6] = {b[0], b[1], b[2], 0.0, 0.0, 0.0};
+    if (dl) {
+        v[0] = b[0] * nv[0];
+        v[1] = b[1] * nv[1];
+        v[2] = b[2] * nv[2];
+        v[3] = b[0] * nv[1] + b[1] * nv[0];
+        v[4] = b[0] * nv[2] + b[2] * nv[0];
+        v[5] = b[1] * nv[2] + b[2] * nv[1];
+    }
+    const double y3[3] = {t[2], t[5] - t[2], t[8] - t[2]};
+    double *o = tcoef + (size_t)i * 48;
+    const int nv_ = dl ? 6 : 3;
+    for (int j = 0; j < 3; j++)
+        for (int q = 0; q < 16; q++)
+            o[16 * j + q] = q < nv_ ? (j ? 0.0 : w * v[q]) : (q < 2 * nv_ ? w * y3[j] * v[q - nv_] : 0.0);
+}
+
 // Shape of a launch: waves per workgroup, steps per slice, most slices, most
 // column pairs, nodes per half triangle; the row tiles of a slice go to the
 // waves in RT rounds (in the last of NS slices one step is left at most where
@@ -146,9 +179,22 @@ inline int p2t_shape(int ph, int nq)
     return P2TShape1::fits(ph) ? 1 : (P2TShape2::fits(ph) ? 2 : (P2TShape3::fits(ph) ? 3 : -1));
 }
 
+// Where the moments themselves are wanted (MIND, the Mindlin P2M): column c16
+// to col[c16] of G, [box of the list][MCOLS][coefficient], harmonics
+// Racah-normalised and unscaled, added with atomics; -1: column not wanted.
+struct MindMoments {
+    int col[16];
+    double2 *G;
+    static constexpr int MCOLS = 18;
+};
+
+// Workgroup b of P2M takes part b, (box of the list, its first triangle,
+// triangles), the whole of box b of the list if there are no parts; a part of
+// a box adds its coefficients with atomics.
 // lds: Z::lds() doubles, 16-byte aligned (16-byte accesses)
-template <bool IRR, class Z>
-__device__ __forceinline__ void p2t_body(int p, const int *__restrict__ boxes, const int *__restrict__ lstart,
+template <bool IRR, class Z, bool MIND>
+__device__ __forceinline__ void p2t_body(int p, const int *__restrict__ boxes, const int *__restrict__ parts,
+                                         MindMoments mind, const int *__restrict__ lstart,
                                          const int *__restrict__ litems, const double *__restrict__ centers,
                                          const double *__restrict__ sides, const int *__restrict__ src_start,
                                          const int *__restrict__ src_count, const double *__restrict__ tri_s,
@@ -170,7 +216,10 @@ __device__ __forceinline__ void p2t_body(int p, const int *__restrict__ boxes, c
     int half = 2 * wave / WB;                         // of the triangle's nodes
     int hl = tid - half * 32 * WB, c = hl / TC, mt = hl - c * TC;
     int len1 = ph + 1 - c;
-    int box = boxes[blockIdx.x];
+    const int bi = !IRR && parts ? parts[3 * blockIdx.x] : (int)blockIdx.x, box = boxes[bi];
+    const int part0 = !IRR && parts ? parts[3 * blockIdx.x + 1] : 0;
+    const int partn = !IRR && parts ? parts[3 * blockIdx.x + 2] : src_count[box];
+    const bool whole = IRR || partn == src_count[box];
     double side = sides[box], is = 1.0 / side;
     double cx = centers[3 * box], cy = centers[3 * box + 1], cz = centers[3 * box + 2];
     for (int e = tid; e < ubuf; e += NT) lds[e] = 0.0;   // rows that no lane writes stay finite
@@ -191,8 +240,8 @@ __device__ __forceinline__ void p2t_body(int p, const int *__restrict__ boxes, c
             int cnt = 0, s0 = 0;
             if (b0 + lane < b1) {
                 int sbox = IRR ? litems[b0 + lane] : box;
-                s0 = src_start[sbox];
-                cnt = src_count[sbox];
+                s0 = src_start[sbox] + part0;
+                cnt = IRR ? src_count[sbox] : partn;
             }
             int end = cnt;
             for (int off = 1; off < 64; off <<= 1) {
@@ -322,6 +371,27 @@ __device__ __forceinline__ void p2t_body(int p, const int *__restrict__ boxes, c
             }
         }
     }
+    if (MIND) {
+        const int nown = (p + 1) * (p + 2) / 2;
+#pragma unroll
+        for (int sl = 0; sl < NS; sl++)
+#pragma unroll
+            for (int rt = 0; rt < (sl == NS - 1 ? 1 : RT); rt++) {
+                int row = 16 * (wave + WB * rt) + n16, st = row / (2 * NP), rem = row - st * 2 * NP, cc = rem >> 1;
+                int s = sl * S + st, l1 = ph + 1 - cc;
+                bool second = s >= l1;
+                if (row >= ROWS || st >= S || s >= nst || cc >= npair || (second && 2 * cc == ph)) continue;
+                int m = second ? ph - cc : cc, l = second ? m + s - l1 : cc + s;
+                double f = pow(side, (double)l) * hnorm(l, m) * g_sdfact[l] * ((l + m) & 1 ? -1.0 : 1.0);
+                double *o = (double *)(mind.G + (size_t)bi * MindMoments::MCOLS * nown + l * (l + 1) / 2 + m) + (rem & 1);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    int col = mind.col[kq + 4 * i];
+                    if (col >= 0) unsafeAtomicAdd(o + (size_t)2 * col * nown, f * acc[sl][rt][i]);
+                }
+            }
+        return;
+    }
     // coefficients, one right-hand side at a time, as p2x_body; moment (col,
     // degree ll, order mm) at slice s / S, step s % S, column pair c
     int nco = (p + 1) * (p + 2) / 2;
@@ -392,9 +462,12 @@ __device__ __forceinline__ void p2t_body(int p, const int *__restrict__ boxes, c
             if (IRR) {
                 e[0] += re;
                 e[1] += im;
-            } else {
+            } else if (whole) {
                 e[0] = re;
                 e[1] = im;
+            } else {
+                unsafeAtomicAdd(e, re);
+                unsafeAtomicAdd(e + 1, im);
             }
         }
     }

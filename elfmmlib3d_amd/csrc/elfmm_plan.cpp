@@ -174,6 +174,27 @@ void near_tasks(Plan &P, const std::vector<int> &ntri, NP &&npts, double npt)
         }
 }
 
+// P2M workgroups: a box's triangles are a chain of chunks of 8 to 12, so where
+// the boxes are too few to fill the device (iter leaves hold up to 240
+// triangles) they are cut into equal parts, about P2M_WG of them, none under
+// P2M_MIN triangles (a part's coefficients cost about as much as three
+// triangles). A fault mesh of 20,020 triangles: the whole half-space product
+// 5.15 ms, 6.2 with a workgroup per box and the Mindlin moments per node.
+void p2m_parts(const Tree &T, Plan &P)
+{
+    constexpr int64_t P2M_WG = 1024, P2M_MIN = 18;
+    int64_t total = 0;
+    for (int b : P.p2m_boxes) total += T.src_count[b];
+    const int64_t per = std::max(P2M_MIN, (total + P2M_WG - 1) / P2M_WG);
+    for (size_t i = 0; i < P.p2m_boxes.size(); i++) {
+        int64_t c = T.src_count[P.p2m_boxes[i]], k = (int64_t)P.p2m_boxes.size() >= P2M_WG ? 1 : (c + per - 1) / per;
+        for (int64_t j = 0; j < k; j++) {
+            int a = (int)(c * j / k), e = (int)(c * (j + 1) / k);
+            for (int v : {(int)i, a, e - a}) P.p2m_parts.push_back(v);
+        }
+    }
+}
+
 // Order of n entries by decreasing weight, equal weights in their order.
 std::vector<int> heaviest_first(const std::vector<double> &w)
 {
@@ -257,7 +278,7 @@ void build_plan_near(const Tree &T, bool src_eval, bool direct_only, bool iter, 
 
 void plan_reset(Plan &P)
 {
-    for (std::vector<int> *v : {&P.p2m_boxes, &P.p2l_boxes, &P.p2l_start, &P.p2l_items, &P.m2t_items, &P.l2t_boxes,
+    for (std::vector<int> *v : {&P.p2m_boxes, &P.p2m_parts, &P.p2l_boxes, &P.p2l_start, &P.p2l_items, &P.m2t_items, &P.l2t_boxes,
                                 &P.nf_boxes, &P.nf_start, &P.nf_items, &P.nf_tasks, &P.l2t_tpt, &P.m2t_slot_box,
                                 &P.m2t_tpt, &P.l2t_wt, &P.m2t_wt, &P.m2t_bt})
         v->clear();
@@ -311,6 +332,7 @@ void build_plan_up(const Tree &T, const Operators *ops, Plan &P, bool iter)
                 }
             // one workgroup per box, most sources first
             for (int q : heaviest_first(w)) P.p2m_boxes.push_back(bx[q]);
+            p2m_parts(T, P);
         } else if (!iter) {
             // P2L: local of box j from the sources of i with j in list3(i)
             // (src/lfmm3dtrilhess.f:760-829); owner j, sources list4(j).
@@ -542,8 +564,22 @@ void build_plan_eval(const Tree &T, int n, const Operators *ops, bool src_eval, 
     P.stats[13] = (double)P.l2t_boxes.size();
 }
 
+std::vector<int> mind_proxy_offsets(int *index)
+{
+    std::vector<int> v;
+    for (int o = 0; o < 343; o++) {
+        int i = o / 49 - 3, j = o / 7 % 7 - 3, k = o % 7 - 3;
+        bool near = std::abs(k) <= 1 && (std::abs(i) > 1 || std::abs(j) > 1);
+        index[o] = near ? (int)v.size() / 3 : -1;
+        if (near) v.insert(v.end(), {i, j, k});
+    }
+    return v;
+}
+
 void build_mindlin_plan(const Tree &T, const Operators &ops, MindlinPlan &MP)
 {
+    int px[343];
+    mind_proxy_offsets(px);
     MP = MindlinPlan();
     int nb = T.nboxes;
     MP.pw_slot.assign(nb, -1);
@@ -557,10 +593,9 @@ void build_mindlin_plan(const Tree &T, const Operators &ops, MindlinPlan &MP)
     std::vector<std::pair<int, int>> near_pairs;   // (offset, pair index)
     std::vector<int> ns, nd;
     MP.far_start.push_back(0);
-    MP.near_start.push_back(0);
     for (int b = 0; b < nb; b++) {
         if (T.level[b] < 2 || !T.tgt_count[b]) continue;
-        int nfar = 0, nnear = 0;
+        int nfar = 0;
         for (int q = T.lstart[2][b]; q < T.lstart[2][b + 1]; q++) {
             int j = T.litems[2][q];
             if (!T.src_count[j]) continue;
@@ -568,8 +603,6 @@ void build_mindlin_plan(const Tree &T, const Operators &ops, MindlinPlan &MP)
             double side = T.size / (double)(1 << T.level[j]);
             double zdis = (T.centers[3 * b + 2] - T.centers[3 * j + 2]) / side;
             if (std::fabs(zdis) < 1.5) {
-                MP.near_items.push_back(j);
-                nnear++;
                 int o = offset_index(T, j, b);
                 near_pairs.push_back({o, (int)ns.size()});
                 ns.push_back(j);
@@ -582,10 +615,6 @@ void build_mindlin_plan(const Tree &T, const Operators &ops, MindlinPlan &MP)
         if (nfar) {
             MP.far_boxes.push_back(b);
             MP.far_start.push_back((int)MP.far_items.size());
-        }
-        if (nnear) {
-            MP.near_boxes.push_back(b);
-            MP.near_start.push_back((int)MP.near_items.size());
         }
     }
     // near pairs grouped by offset, tiles of the full-order operators
@@ -604,6 +633,8 @@ void build_mindlin_plan(const Tree &T, const Operators &ops, MindlinPlan &MP)
             sc[i - k] = (double)(1 << T.level[d[i - k]]) / T.size;
         }
         int h = ncoef(ops.m2l_pt[o]) / 2;
+        for (size_t i = k; i < e; i += MIND_PX)
+            for (int v : {px[o], (int)i, (int)std::min<size_t>(MIND_PX, e - i)}) MP.px_tasks.push_back(v);
         add_pairs(g, ops.m2l_off[o], h, ops.m2l_phi[o], s.data(), d.data(), sc.data(), (int)(e - k), ops.m2l_refl[o]);
         k = e;
     }

@@ -72,15 +72,16 @@ gemm_d4 mfma(double a, double b, gemm_d4 c)
 
 #define __builtin_amdgcn_readfirstlane(v) (v)
 #define __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, x, y, z) mfma(a, b, c)
+void unsafeAtomicAdd(double *p, double v) { *p += v; }    // no two lanes share a coefficient
 #include "../../elfmmlib3d_amd/csrc/elfmm_moments.h"
 
-template <bool IRR, class Z>
+template <bool IRR, class Z, bool MIND = false>
 void launch(int p, const std::vector<int> &boxes, const std::vector<int> &ls, const std::vector<int> &li,
             const double *cen, const double *sides, const int *ss, const int *sc, const double *tri, const double *tc,
-            int nc, double *ex)
+            int nc, double *ex, const std::vector<int> &parts = {}, MindMoments mind = {})
 {
-    size_t nl = (size_t)Z::lds(IRR ? p + 1 : p);
-    for (size_t b = 0; b < boxes.size(); b++) {
+    size_t nl = (size_t)Z::lds(IRR ? p + 1 : p), nwg = parts.empty() ? boxes.size() : parts.size() / 3;
+    for (size_t b = 0; b < nwg; b++) {
         blockIdx.x = (int)b;
         emu_lds = (double *)std::aligned_alloc(16, (nl * 8 + 15) / 16 * 16);
         std::fill(emu_lds, emu_lds + nl, NAN);
@@ -90,7 +91,8 @@ void launch(int p, const std::vector<int> &boxes, const std::vector<int> &ls, co
         for (int t = 0; t < Z::NT; t++)
             th.emplace_back([&, t] {
                 threadIdx.x = t;
-                p2t_body<IRR, Z>(p, boxes.data(), ls.data(), li.data(), cen, sides, ss, sc, tri, tc, nc, ex, emu_lds);
+                p2t_body<IRR, Z, MIND>(p, boxes.data(), parts.empty() ? nullptr : parts.data(), mind, ls.data(),
+                                       li.data(), cen, sides, ss, sc, tri, tc, nc, ex, emu_lds);
             });
         for (auto &t : th) t.join();
         pthread_barrier_destroy(&g_bar);
@@ -234,5 +236,113 @@ extern "C" double moments_host(int p, int nq, int irr, const int *counts, int nl
                 if (!(rel <= worst)) worst = rel;     // NaN stays
             }
     }
+    return worst;
+}
+
+// One box of `count` triangles in `nparts` parts beside a whole one: the worst
+// relative difference, over degrees, of the parts' multipole from the whole
+// box's, and of the Mindlin moments (both layers, in parts) from the node sums
+// in long double of the Racah-normalised harmonics (Condon-Shortley phase).
+extern "C" double moment_parts_host(int p, int nq, int count, int nparts, int seed)
+{
+    double f = 1, d = 1;
+    for (int k = 0; k < 2 * PMAX + 8; k++) g_fact[k] = f, f *= k + 1;
+    for (int m = 0; m < PMAX + 4; m++) g_sdfact[m] = d, d *= -(2.0 * m + 1);
+    const int nc = (p + 1) * (p + 2), nown = nc / 2, shape = p2t_shape(p, nq), n = count;
+    std::mt19937 g(seed);
+    std::uniform_real_distribution<double> U(-1, 1);
+    std::vector<double> tri(9 * n), nrm(3 * n), sl(3 * n), dl(3 * n), tc(48 * n), cen = {0.1, -0.05, -0.2}, sides = {1.3};
+    for (int i = 0; i < n; i++) {
+        double c[3] = {0.4 * U(g), 0.4 * U(g), 0.4 * U(g)};
+        for (int k = 0; k < 9; k++) tri[9 * i + k] = c[k % 3] + 0.1 * U(g);
+        for (int k = 0; k < 3; k++) nrm[3 * i + k] = U(g), sl[3 * i + k] = U(g), dl[3 * i + k] = U(g);
+    }
+    std::vector<int> boxes = {0}, none, ss = {0}, sc = {n}, parts;
+    for (int j = 0; j < nparts; j++) parts.insert(parts.end(), {0, n * j / nparts, n * (j + 1) / nparts - n * j / nparts});
+    auto each = [&](auto fn) {
+        blockDim.x = 1;
+        threadIdx.x = 0;
+        for (int i = 0; i < n; i++) blockIdx.x = i, fn();
+    };
+    auto shaped = [&](auto fn) {
+        shape == 0 ? fn(P2TShape0{}) : shape == 1 ? fn(P2TShape1{}) : shape == 2 ? fn(P2TShape2{}) : fn(P2TShape3{});
+    };
+    double worst = 0;
+    auto note = [&](LD num, LD den) {
+        double rel = (double)sqrtl(num / den);
+        if (!(rel <= worst)) worst = rel;             // NaN stays
+    };
+    std::vector<double> whole(NRHS * nc, 0.0), cut(NRHS * nc, 0.0), G((size_t)2 * MindMoments::MCOLS * nown, 0.0);
+    each([&] { k_tcoef(n, tri.data(), nrm.data(), sl.data(), dl.data(), 1, 1, 0.7, 0.6, 0.4, -1.0, tc.data()); });
+    shaped([&](auto z) {
+        using Z = decltype(z);
+        launch<false, Z>(p, boxes, none, none, cen.data(), sides.data(), ss.data(), sc.data(), tri.data(), tc.data(), nc, whole.data());
+        launch<false, Z>(p, boxes, none, none, cen.data(), sides.data(), ss.data(), sc.data(), tri.data(), tc.data(), nc, cut.data(), parts);
+    });
+    for (int r = 0; r < NRHS; r++)
+        for (int l = 0; l <= p; l++) {
+            LD num = 0, den = 0;
+            for (int k = l * (l + 1); k < (l + 1) * (l + 2); k++) {
+                LD w = whole[r * nc + k], e = cut[r * nc + k] - w;
+                num += e * e;
+                den += w * w;
+            }
+            if (den > 0) note(num, den);
+        }
+    for (int layer = 0; layer < 2; layer++) {
+        each([&] { k_mind_tcoef(n, layer, tri.data(), nrm.data(), layer ? dl.data() : sl.data(), tc.data()); });
+        MindMoments mm;
+        for (int c = 0; c < 16; c++) mm.col[c] = layer ? (c < 12 ? 6 + c : -1) : (c < 6 ? c : -1);
+        mm.G = (double2 *)G.data();
+        shaped([&](auto z) {
+            using Z = decltype(z);
+            launch<false, Z, true>(p, boxes, none, none, cen.data(), sides.data(), ss.data(), sc.data(), tri.data(), tc.data(), nc, nullptr, parts, mm);
+        });
+    }
+    std::vector<LD> want((size_t)2 * MindMoments::MCOLS * nown, 0);
+    for (int i = 0; i < n; i++)
+        for (int q = 0; q < nq; q++) {
+            const double *r = RULE[(nq == 12 ? 6 : 0) + q], *t = &tri[9 * i], *nv = &nrm[3 * i], *b = &dl[3 * i];
+            LD X[3], a[3], e[3], v[18];
+            for (int k = 0; k < 3; k++) {
+                a[k] = (LD)t[3 + k] - t[k], e[k] = (LD)t[6 + k] - t[k];
+                X[k] = t[k] + r[0] * a[k] + r[1] * e[k];
+            }
+            LD cx = a[1] * e[2] - a[2] * e[1], cy = a[2] * e[0] - a[0] * e[2], cz = a[0] * e[1] - a[1] * e[0];
+            LD w = r[2] * sqrtl(cx * cx + cy * cy + cz * cz);
+            for (int k = 0; k < 3; k++) v[k] = w * sl[3 * i + k], v[6 + k] = w * (LD)b[k] * nv[k];
+            v[9] = w * ((LD)b[0] * nv[1] + (LD)b[1] * nv[0]);
+            v[10] = w * ((LD)b[0] * nv[2] + (LD)b[2] * nv[0]);
+            v[11] = w * ((LD)b[1] * nv[2] + (LD)b[2] * nv[1]);
+            for (int k = 0; k < 3; k++) v[3 + k] = v[k] * X[2];
+            for (int k = 0; k < 6; k++) v[12 + k] = v[6 + k] * X[2];
+            LD x = X[0] - cen[0], y = X[1] - cen[1], z = X[2] - cen[2], r2 = x * x + y * y + z * z, dr = 1, di = 0;
+            for (int m = 0; m <= p; m++) {
+                if (m) {
+                    LD c = -sqrtl((2 * m - 1) / (LD)(2 * m)), nr = c * (x * dr - y * di);
+                    di = c * (x * di + y * dr), dr = nr;
+                }
+                LD ar = 0, ai = 0, br = dr, bi = di;
+                for (int l = m; l <= p; l++) {
+                    for (int c = 0; c < 18; c++) {
+                        LD *o = &want[2 * ((size_t)c * nown + l * (l + 1) / 2 + m)];
+                        o[0] += v[c] * br;
+                        o[1] += v[c] * bi;
+                    }
+                    LD dn = sqrtl((LD)(l + 1 + m) * (l + 1 - m)), k1 = (2 * l + 1) * z / dn, k2 = sqrtl((LD)(l + m) * (l - m)) * r2 / dn;
+                    LD nr = k1 * br - k2 * ar, ni = k1 * bi - k2 * ai;
+                    ar = br, ai = bi, br = nr, bi = ni;
+                }
+            }
+        }
+    for (int c = 0; c < 18; c++)
+        for (int l = 0; l <= p; l++) {
+            LD num = 0, den = 0;
+            for (size_t k = (size_t)c * 2 * nown + l * (l + 1); k < (size_t)c * 2 * nown + (l + 1) * (l + 2); k++) {
+                num += (G[k] - want[k]) * (G[k] - want[k]);
+                den += want[k] * want[k];
+            }
+            note(num, den);
+        }
     return worst;
 }

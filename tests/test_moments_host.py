@@ -22,6 +22,7 @@ def lib(tmp_path_factory):
                     os.path.join(ROOT, "tests", "csrc", "moments_host.cpp")], check=True)
     lib = C.CDLL(out)
     lib.moments_host.restype = C.c_double
+    lib.moment_parts_host.restype = C.c_double
     return lib
 
 
@@ -41,3 +42,11 @@ def test_other_orders_have_no_shape(lib):
     counts = (C.c_int * 4)(1, 1, 1, 1)
     for p, nq in ((5, 3), (2, 1), (44, 12), (26, 6)):
         assert lib.moments_host(p, nq, 0, counts, 1, 1) < 0
+
+
+@pytest.mark.parametrize("p,nq,count,nparts", [(9, 6, 1, 1), (9, 6, 23, 3), (14, 12, 37, 2), (26, 12, 36, 2),
+                                               (26, 12, 19, 1), (39, 12, 27, 5)])
+def test_parts_and_mindlin_moments(lib, p, nq, count, nparts):
+    """A box cut into parts whose coefficients are added, and the moments as they
+    are (the Mindlin P2M), in parts too: the same sums, the same tolerance."""
+    assert 0 <= lib.moment_parts_host(p, nq, count, nparts, 3 * p + count) <= 1e-12
