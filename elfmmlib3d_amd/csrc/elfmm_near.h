@@ -10,7 +10,13 @@
 //   - the primitives int t^m / (t^2 + rho^2)^(q/2) of an edge follow from the
 //     two distances without a branch on the foot point's side: with
 //     A = r + |t| at both ends and opp = foot point inside the edge,
-//       K01 = log(A1 A2 / rho^2)             (opp), log(max A / min A) (else)
+//       K01 = log(A1 A2 / rho^2)             (opp), log(max A / min A) (else),
+//             as log(1 + x), x a sum of terms of one sign: A1 A2 - rho^2 =
+//             r1 |t2| + r2 |t1| + |t1 t2| + (r1^2 r2^2 - rho^4) / (r1 r2 + rho^2),
+//             max A - min A = L + |t1 + t2| L / (r1 + r2), so K01 ~ L/R keeps its digits
+//             at distances R >> L (the sums over the edges lose R/L of them, not
+//             (R/L)^2: 6.0e-15 of a single layer's displacement at R = 8 L, 2.0e-14
+//             from the ratio's logarithm, measured against long double)
 //       K03 = 2 L (r1 + r2) A1 A2 / (r1 r2 E),
 //             E = rho^2 (A1 + A2)^2 (opp), (A1 A2 + rho^2)^2 (else)
 //       3 K25 = K03 (u1^2 + u1 u2 + u2^2),  u = t / r
@@ -53,6 +59,13 @@ ELFMM_HD double nf_rsqrt(double x)
 #endif
 }
 
+// log(1 + x), x >= 0: the rounding of 1 + x given back to first order.
+ELFMM_HD double nf_log1p(double x)
+{
+    double u = 1.0 + x;
+    return log(u) + (x - (u - 1.0)) * nf_rcp(u);
+}
+
 // Sums over the edges, in the triangle's frame (z normal), w = -z0.
 struct NearSums {
     double F, r1x, r1y;                              // K01: del, n_x, n_y
@@ -72,15 +85,17 @@ ELFMM_HD void near_edge(double sx, double sy, double L, double t1, double del, d
     bool opp = t1 < 0.0 && t2 > 0.0;
     double a1 = t1 < 0.0 ? -t1 : t1, a2 = t2 < 0.0 ? -t2 : t2;
     double A1 = r1 + a1, A2 = r2 + a2, A12 = A1 * A2, sum = r1 + r2, i12 = ir1 * ir2;
+    double k11 = L * (t1 + t2) * nf_rcp(sum);
     // K01
-    double hi = A1 > A2 ? A1 : A2, lo = A1 > A2 ? A2 : A1;
-    double irho2 = nf_rcp(opp ? rho2 : lo);
-    double k01 = log((opp ? A12 : hi) * irho2);
+    double r12 = r1 * r2, a12 = a1 * a2;
+    double x1 = (rho2 * (a1 * a1 + a2 * a2) + a12 * a12) * nf_rcp(r12 + rho2) + (r1 * a2 + r2 * a1 + a12);
+    double x2 = L + (k11 < 0.0 ? -k11 : k11);
+    double irho2 = nf_rcp(opp ? rho2 : (A1 > A2 ? A2 : A1));
+    double k01 = nf_log1p((opp ? x1 : x2) * irho2);
     double nxk = nx * k01, dk = del * k01;
     S.F += dk;
     S.r1x += nxk;
     S.r1y += ny * k01;
-    double k11 = L * (t1 + t2) * nf_rcp(sum);
     if (SL) {
         S.b2xx += p * k11 + sy2 * dk;
         S.b2xy += sy2 * k11 - p * dk;
@@ -116,7 +131,7 @@ ELFMM_HD void near_edge(double sx, double sy, double L, double t1, double del, d
     S.qxy += sy2 * k13 - p * g3;
     // order 4 of r: 3 K25 - K03, 3 K15, 3 K05
     double u1 = t1 * ir1, u2 = t2 * ir2, g1 = ir1 * ir1, g2 = ir2 * ir2;
-    double P = r1 * r2 + a1 * a2;
+    double P = r12 + a12;
     double M = t1 * t1 + t2 * t2 + rho2;
     double W = opp ? P * irho2 : M * nf_rcp(P);
     double y5 = g1 + g2 + W * i12;                                          // 3 K05 / K03

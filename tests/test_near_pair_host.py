@@ -89,3 +89,25 @@ def test_matches_direct_pair(nf, sl, dl):
             disp = pair(nf, "near_host_pair", tri, s, d, x, iself, lam, mu, sl, dl, 0)
             assert np.abs(disp - new)[:3].max() <= 1e-14 * np.abs(new[:3]).max()
             assert not disp[3:].any()
+
+
+@pytest.mark.parametrize("sl,dl", [(1, 0), (0, 1)])
+def test_distant_points_keep_their_digits(nf, tmp_path, sl, dl):
+    """Far from a triangle (a leaf of few triangles beside large ones) the sums over
+    its edges lose R/L of the digits and no more: 20 roundings a term, some tens of
+    terms, 1e-13 R/L, against the direct sum's code in long double."""
+    out = str(tmp_path / "near_long.so")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-o", out, os.path.join(CSRC, "near_pair_long.cpp")],
+                   check=True)
+    exact = C.CDLL(out)
+    rng = np.random.default_rng(3 + sl)
+    for r in (1.5, 8.0, 60.0, 1000.0):
+        for t in range(50):
+            tri = np.array([[0, 0, 0], [1, 0, 0], [0.4, 0.9, 0]]) + 0.2 * rng.normal(size=(3, 3))
+            v = rng.normal(size=3)
+            x = tri.mean(0) + r * v / np.linalg.norm(v)
+            s, d = rng.normal(size=(2, 3))
+            ref = pair(exact, "near_long", tri, s, d, x, 0, 1.1, 0.7, sl, dl)
+            new = pair(nf, "near_host_pair", tri, s, d, x, 0, 1.1, 0.7, sl, dl, 1)
+            for c in (slice(0, 3), slice(3, 9)):
+                assert np.linalg.norm((new - ref)[c]) <= 1e-13 * r * np.linalg.norm(ref[c]), (r, t)
