@@ -1251,147 +1251,141 @@ __global__ __launch_bounds__(NF_THREADS) void k_near_store(
     }
 }
 
-// icomp 3: near field from the stored fields and the current densities.
-// One wave per point (wave g of the launch takes point g of the near boxes'
-// points, box by box: the work is spread evenly whatever the leaf sizes).
-// The point's ntri slots are consecutive, so lane l
-// taking triangles l, l + 64, ... makes every load instruction read 64
-// consecutive doubles of the store and each step of the wave one stretch
-// of it (store_idx); the lanes' partial sums are then added across the
-// wave. The layers present (NL: d0, then d1) and the fields stored (FD
-// displacement, FS strain) are compile-time, so all words of a slot are
-// loaded before the first is used.
-template <int NL, bool FD, bool FS>
-__global__ __launch_bounds__(NF_THREADS) void k_near_replay(
+// icomp 3: near field from the stored fields and nr <= RB density sets; bound
+// by the read of the store. A task is PTS points of a near box (part
+// b % (ST_CHUNK / PTS) of chunk b / (ST_CHUNK / PTS)); the 4 waves take
+// its tiles of 64 triangles in turn: a lane finds its slot's triangle in the
+// box's list (first slots in LDS, RP_LIST boxes at a time), loads the
+// triangle's densities once and then streams that slot of every point, one
+// tile of the store (store_idx) per point and load. The layers present (NL:
+// d0, then d1) and the fields stored (FD displacement, FS strain) are
+// compile-time, so all words of a slot are loaded before the first is used.
+// Densities d0/d1: [set][triangle][3] in tree order (stride dstride doubles
+// per set); output nf: [set][point][9] (stride nstride).
+constexpr int RP_LIST = 512;
+constexpr int replay_pts(int nl, bool fd, bool fs, int rb)
+{
+    int w = nl * 3 * (3 * fd + 6 * fs);
+    return rb > 1 ? 1 : w <= 18 ? 4 : w <= 27 ? 2 : 1;
+}
+
+template <int NL, bool FD, bool FS, int RB>
+__global__ __launch_bounds__(NF_THREADS, 2) void k_near_replay(
     int n, int n_src_eval, const int *__restrict__ boxes, const int *__restrict__ lstart,
     const int *__restrict__ litems, const int *__restrict__ src_start,
     const int *__restrict__ src_count, const int *__restrict__ tgt_start,
     const int64_t *__restrict__ sbase, const int *__restrict__ ntri_q,
-    const int *__restrict__ pstart, int nq, const double *__restrict__ d0, const double *__restrict__ d1,
-    const double *__restrict__ store, double *__restrict__ nf)
+    const int *__restrict__ pstart, const int *__restrict__ chunk, int ntask, const double *__restrict__ d0,
+    const double *__restrict__ d1, size_t dstride, int nr, const double *__restrict__ store,
+    double *__restrict__ nf, size_t nstride)
 {
     constexpr int NF = 3 * FD + 6 * FS;                 // fields per unit density
     constexpr int W = NL * 3 * NF;                      // words per slot
     constexpr int Q0 = FD ? 0 : 3;                      // first output component
-    int lane = threadIdx.x & 63;
-    int g = __builtin_amdgcn_readfirstlane((int)blockIdx.x * (NF_THREADS / 64) + (int)(threadIdx.x >> 6));
-    if (g >= pstart[nq]) return;                        // no barriers below
-    int lo = 0, hi = nq - 1;                            // near box qb: pstart[qb] <= g < pstart[qb + 1]
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (pstart[mid] <= g) lo = mid;
-        else hi = mid - 1;
-    }
-    int qb = lo;
-    int tbox = boxes[qb];
-    int ns_eval = n_src_eval ? src_count[tbox] : 0;
-    int b0 = lstart[qb], b1 = lstart[qb + 1];
-    int ntri = ntri_q[qb];
-    const double *S = store + sbase[qb];
-    {
-        int k = g - pstart[qb];
-        double acc[NF];
+    constexpr int PTS = replay_pts(NL, FD, FS, RB);
+    constexpr int NWAVE = NF_THREADS / 64;
+    __shared__ int first[RP_LIST + 1], start[RP_LIST];  // first slot, first triangle of each box of the list
+    __shared__ double red[NWAVE][RB * PTS * NF];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    for (int task = blockIdx.x; task < ntask; task += gridDim.x) {
+        const int *ch = chunk + 2 * (task / (ST_CHUNK / PTS));
+        const int qb = ch[0], k0 = ch[1] + task % (ST_CHUNK / PTS) * PTS;
+        const int np = min(PTS, pstart[qb + 1] - pstart[qb] - k0);
+        if (np <= 0) continue;
+        const int ntri = ntri_q[qb], b0 = lstart[qb], b1 = lstart[qb + 1];
+        const double *S = store + sbase[qb] + (int64_t)k0 * ntri * W;
+        double acc[RB][PTS][NF];
 #pragma unroll
-        for (int q = 0; q < NF; q++) acc[q] = 0.0;
-        near_walk(b0, b1, litems, src_start, src_count, lane, 64, [&](int i, int t) {
-            int t0 = t & ~63;
-            int tw = ntri - t0 < 64 ? ntri - t0 : 64;
-            const double *Sx = S + store_idx(k, t, 0, ntri, W);   // word w at Sx[w * tw]
-            double c[NL][3], v[W];
+        for (int r = 0; r < RB; r++)
 #pragma unroll
-            for (int a = 0; a < NL; a++)
+            for (int k = 0; k < PTS; k++)
 #pragma unroll
-                for (int kk = 0; kk < 3; kk++) c[a][kk] = (a ? d1 : d0)[3 * (size_t)i + kk];
-#pragma unroll
-            for (int w = 0; w < W; w++) v[w] = Sx[w * tw];
-#pragma unroll
-            for (int a = 0; a < NL; a++)
-#pragma unroll
-                for (int kk = 0; kk < 3; kk++)
-#pragma unroll
-                    for (int q = 0; q < NF; q++) acc[q] += c[a][kk] * v[(a * 3 + kk) * NF + q];
-        });
-#pragma unroll
-        for (int q = 0; q < NF; q++)
-            for (int off = 32; off > 0; off >>= 1) acc[q] += __shfl_xor(acc[q], off);
-        if (lane == 0) {
-            int gp = k < ns_eval ? src_start[tbox] + k : n + tgt_start[tbox] + (k - ns_eval);
-            double *o = nf + (size_t)gp * 9;
-#pragma unroll
-            for (int q = 0; q < 9; q++) o[q] = (q >= Q0 && q < Q0 + NF) ? acc[q - Q0] : 0.0;
-        }
-    }
-}
-
-// icomp 3 for nr density sets at once (nr <= RB): as k_near_replay, each
-// loaded slot of the store is applied to every set, so the store is read
-// once per RB sets. Densities d0/d1: [set][triangle][3] in tree order
-// (stride dstride doubles per set); output nf: [set][point][9] (stride
-// nstride).
-template <int NL, bool FD, bool FS, int RB>
-__global__ __launch_bounds__(NF_THREADS) void k_near_replay_multi(
-    int n, int n_src_eval, const int *__restrict__ boxes, const int *__restrict__ lstart,
-    const int *__restrict__ litems, const int *__restrict__ src_start,
-    const int *__restrict__ src_count, const int *__restrict__ tgt_start,
-    const int64_t *__restrict__ sbase, const int *__restrict__ ntri_q,
-    const int *__restrict__ pstart, int nq, const double *__restrict__ d0, const double *__restrict__ d1,
-    size_t dstride, int nr, const double *__restrict__ store, double *__restrict__ nf, size_t nstride)
-{
-    constexpr int NF = 3 * FD + 6 * FS;
-    constexpr int W = NL * 3 * NF;
-    constexpr int Q0 = FD ? 0 : 3;
-    int lane = threadIdx.x & 63;
-    int g = __builtin_amdgcn_readfirstlane((int)blockIdx.x * (NF_THREADS / 64) + (int)(threadIdx.x >> 6));
-    if (g >= pstart[nq]) return;
-    int lo = 0, hi = nq - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (pstart[mid] <= g) lo = mid;
-        else hi = mid - 1;
-    }
-    int qb = lo;
-    int tbox = boxes[qb];
-    int ns_eval = n_src_eval ? src_count[tbox] : 0;
-    int b0 = lstart[qb], b1 = lstart[qb + 1];
-    int ntri = ntri_q[qb];
-    const double *S = store + sbase[qb];
-    int k = g - pstart[qb];
-    double acc[RB][NF];
-#pragma unroll
-    for (int r = 0; r < RB; r++)
-#pragma unroll
-        for (int q = 0; q < NF; q++) acc[r][q] = 0.0;
-    near_walk(b0, b1, litems, src_start, src_count, lane, 64, [&](int i, int t) {
-        int t0 = t & ~63;
-        int tw = ntri - t0 < 64 ? ntri - t0 : 64;
-        const double *Sx = S + store_idx(k, t, 0, ntri, W);
-        double v[W];
-#pragma unroll
-        for (int w = 0; w < W; w++) v[w] = Sx[w * tw];
-#pragma unroll
-        for (int r = 0; r < RB; r++) {
-            if (r >= nr) break;
-#pragma unroll
-            for (int a = 0; a < NL; a++) {
-                const double *dd = (a ? d1 : d0) + r * dstride + 3 * (size_t)i;
-                double c0 = dd[0], c1 = dd[1], c2 = dd[2];
-#pragma unroll
-                for (int q = 0; q < NF; q++)
-                    acc[r][q] += c0 * v[(a * 3) * NF + q] + c1 * v[(a * 3 + 1) * NF + q] + c2 * v[(a * 3 + 2) * NF + q];
+                for (int q = 0; q < NF; q++) acc[r][k][q] = 0.0;
+        int done = 0;                                   // slots of the list's earlier boxes
+        for (int c0 = b0; c0 < b1; c0 += RP_LIST) {
+            const int nb = min(RP_LIST, b1 - c0);
+            __syncthreads();
+            if (wave == 0) {
+                int cum = done;
+                for (int e = 0; e < nb; e += 64) {
+                    int cnt = 0;
+                    if (e + lane < nb) {
+                        int box = litems[c0 + e + lane];
+                        start[e + lane] = src_start[box];
+                        cnt = src_count[box];
+                    }
+                    int end = cnt;
+                    for (int off = 1; off < 64; off <<= 1) {
+                        int v = __shfl_up(end, off);
+                        if (lane >= off) end += v;
+                    }
+                    if (e + lane < nb) first[e + lane] = cum + end - cnt;
+                    cum += __shfl(end, 63);
+                }
+                if (lane == 0) first[nb] = cum;
             }
+            __syncthreads();
+            const int last = first[nb];
+            // tiles that hold slots of these boxes
+            for (int t0 = (done / 64 + ((wave - done / 64) & (NWAVE - 1))) * 64; t0 < last; t0 += 64 * NWAVE) {
+                const int t = t0 + lane, tw = min(64, ntri - t0);
+                if (t < done || t >= last) continue;
+                int lo = 0, hi = nb - 1;                // first[lo] <= t < first[lo + 1]
+                while (lo < hi) {
+                    int mid = (lo + hi + 1) >> 1;
+                    if (first[mid] <= t) lo = mid;
+                    else hi = mid - 1;
+                }
+                const size_t i = start[lo] + (t - first[lo]);
+                double c[NL][3];
+                auto dens = [&](int r) {
+#pragma unroll
+                    for (int a = 0; a < NL; a++)
+#pragma unroll
+                        for (int kk = 0; kk < 3; kk++) c[a][kk] = (a ? d1 : d0)[r * dstride + 3 * i + kk];
+                };
+                if (RB == 1) dens(0);
+                const double *Sx = S + (int64_t)t0 * W + lane;   // word w at Sx[w * tw]
+#pragma unroll
+                for (int k = 0; k < PTS; k++) {
+                    if (k >= np) break;
+                    double v[W];
+#pragma unroll
+                    for (int w = 0; w < W; w++) v[w] = Sx[(int64_t)k * ntri * W + w * tw];
+#pragma unroll
+                    for (int r = 0; r < RB; r++) {
+                        if (r >= nr) break;
+                        if (RB > 1) dens(r);
+#pragma unroll
+                        for (int a = 0; a < NL; a++)
+#pragma unroll
+                            for (int kk = 0; kk < 3; kk++)
+#pragma unroll
+                                for (int q = 0; q < NF; q++) acc[r][k][q] += c[a][kk] * v[(a * 3 + kk) * NF + q];
+                    }
+                }
+            }
+            done = last;
         }
-    });
-    int gp = k < ns_eval ? src_start[tbox] + k : n + tgt_start[tbox] + (k - ns_eval);
 #pragma unroll
-    for (int r = 0; r < RB; r++) {
-        if (r >= nr) break;
+        for (int r = 0; r < RB; r++)
 #pragma unroll
-        for (int q = 0; q < NF; q++)
-            for (int off = 32; off > 0; off >>= 1) acc[r][q] += __shfl_xor(acc[r][q], off);
-        if (lane == 0) {
-            double *o = nf + r * nstride + (size_t)gp * 9;
+            for (int k = 0; k < PTS; k++)
 #pragma unroll
-            for (int q = 0; q < 9; q++) o[q] = (q >= Q0 && q < Q0 + NF) ? acc[r][q - Q0] : 0.0;
+                for (int q = 0; q < NF; q++) {
+                    double v = acc[r][k][q];
+                    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+                    if (lane == 0) red[wave][(r * PTS + k) * NF + q] = v;
+                }
+        __syncthreads();
+        const int tbox = boxes[qb], ns_eval = n_src_eval ? src_count[tbox] : 0;
+        for (int e = threadIdx.x; e < min(nr, RB) * np * 9; e += NF_THREADS) {
+            int r = e / (np * 9), k = e / 9 % np, q = e % 9;
+            double v = 0.0;
+            if (q >= Q0 && q < Q0 + NF)
+                for (int w = 0; w < NWAVE; w++) v += red[w][(r * PTS + k) * NF + q - Q0];
+            int kp = k0 + k, gp = kp < ns_eval ? src_start[tbox] + kp : n + tgt_start[tbox] + (kp - ns_eval);
+            nf[r * nstride + (size_t)gp * 9 + q] = v;
         }
     }
 }
@@ -1872,6 +1866,7 @@ constexpr int NPHASE = 12;
 // an OpsCache is immutable once built).
 struct DeviceState {
     bool tables = false;
+    int cus = 256;                                   // compute units
     bool p2x_wide = false;                           // 16-wave P2M/P2L for orders above 26
     bool p2t = false;                                // P2M/P2L through triangle moments (156 KB of LDS per CU)
     std::map<int, std::unique_ptr<OpsCache>> ops;   // by iprec
@@ -1922,6 +1917,7 @@ DeviceState &device_state()
                    hipFuncSetAttribute((const void *)k_p2l_tri<Z>, hipFuncAttributeMaxDynamicSharedMemorySize, b) ==
                        hipSuccess;
         };
+        HIPOK(hipDeviceGetAttribute(&ds->cus, hipDeviceAttributeMultiprocessorCount, dev));
         ds->p2t = lds_ok(P2TShape0{}) && lds_ok(P2TShape1{}) && lds_ok(P2TShape2{}) && lds_ok(P2TShape3{});
         (void)hipGetLastError();                     // a refused size leaves the narrow shape, or the node products, in use
         ds->tables = true;
@@ -2798,46 +2794,39 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
     // fields stored); with SL.W == 0 nothing is stored and the near field
     // stays zero
     auto run_replay = [&](hipStream_t rs) -> hipError_t {
-        auto rk = SL.ifsl + SL.ifdl == 2
-                      ? (SL.fd && SL.fs ? k_near_replay<2, true, true>
-                                        : SL.fd ? k_near_replay<2, true, false> : k_near_replay<2, false, true>)
-                      : (SL.fd && SL.fs ? k_near_replay<1, true, true>
-                                        : SL.fd ? k_near_replay<1, true, false> : k_near_replay<1, false, true>);
-        const double *d0 = SL.ifsl ? ssl_s : sdl_s;
-        int nqb = (int)nf_boxes.size(), wpb = NF_THREADS / 64;
-        if (SL.W > 0 && nf_pstart.back() > 0)
-            hipLaunchKernelGGL(rk, dim3((nf_pstart.back() + wpb - 1) / wpb), dim3(NF_THREADS), 0, rs, n, src_eval,
-                               I(o_nfb), I(o_nfs), I(o_nfi), I(o_ss), I(o_sc), I(o_ts),
-                               (const int64_t *)(P + o_sbase), I(o_ntri), I(o_pst), nqb, d0, sdl_s,
-                               store->data.get<double>(), W.nf.get<double>());
-        return hipGetLastError();
-    };
-    // the same for all density sets, RB sets per pass over the store
-    auto run_replay_multi = [&](hipStream_t rs) -> hipError_t {
-        const double *d0 = SL.ifsl ? dm0 : dm1;
-        int nqb = (int)nf_boxes.size(), wpb = NF_THREADS / 64;
-        if (!(SL.W > 0 && nf_pstart.back() > 0)) return hipSuccess;
+        if (!(SL.W > 0 && !nf_chunk.empty())) return hipSuccess;
+        const double *d0 = nrhs > 1 ? (SL.ifsl ? dm0 : dm1) : (SL.ifsl ? ssl_s : sdl_s), *d1 = nrhs > 1 ? dm1 : sdl_s;
+        double *out = nrhs > 1 ? W.nfm.get<double>() : W.nf.get<double>();
         size_t dstr = (size_t)n * 3, nstr = (size_t)np * 9;
-        constexpr int RB2 = 4, RB1 = 8;
-        int rb = SL.ifsl + SL.ifdl == 2 ? RB2 : RB1;
-        for (int r0 = 0; r0 < nrhs; r0 += rb) {
-            int nr = std::min(rb, nrhs - r0);
-            auto rk = SL.ifsl + SL.ifdl == 2
-                          ? (SL.fd && SL.fs ? k_near_replay_multi<2, true, true, RB2>
-                                            : SL.fd ? k_near_replay_multi<2, true, false, RB2>
-                                                    : k_near_replay_multi<2, false, true, RB2>)
-                          : (SL.fd && SL.fs ? k_near_replay_multi<1, true, true, RB1>
-                                            : SL.fd ? k_near_replay_multi<1, true, false, RB1>
-                                                    : k_near_replay_multi<1, false, true, RB1>);
-            hipLaunchKernelGGL(rk, dim3((nf_pstart.back() + wpb - 1) / wpb), dim3(NF_THREADS), 0, rs, n, src_eval,
-                               I(o_nfb), I(o_nfs), I(o_nfi), I(o_ss), I(o_sc), I(o_ts),
-                               (const int64_t *)(P + o_sbase), I(o_ntri), I(o_pst), nqb, d0 + r0 * dstr,
-                               dm1 + r0 * dstr, dstr, nr, store->data.get<double>(),
-                               W.nfm.get<double>() + r0 * nstr, nstr);
-            hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
-        }
-        return hipSuccess;
+        // One set beside its far field: a workgroup per CU, each taking every
+        // grid-th task. That reads at 4.3 TB/s and leaves the registers of
+        // three quarters of a SIMD to the far field, which else waits for the
+        // whole replay: a product of 46,080 triangles at order 26 takes 3.85 ms
+        // (4.44 unlimited, 4.2 with two per CU), of 15,680 at order 14 1.00
+        // (1.16). Unlimited: order 39, where a workgroup of P2M takes a whole
+        // CU (2.15, limited 2.31), several sets, whose far fields outweigh the
+        // replay (16 sets of 32,000 triangles: 16.0, limited 18.4), and no far
+        // field.
+        const bool limit = nrhs == 1 && oc && !near_only && T.nlev >= 2 && p <= 30;
+        auto run = [&](auto rk, int rb) {
+            int ntask = (int)nf_chunk.size() / 2 * (ST_CHUNK / replay_pts(SL.ifsl + SL.ifdl, SL.fd, SL.fs, rb));
+            for (int r0 = 0; r0 < nrhs; r0 += rb)
+                hipLaunchKernelGGL(rk, dim3(limit ? std::min(ntask, ds.cus) : ntask), dim3(NF_THREADS), 0, rs, n, src_eval, I(o_nfb), I(o_nfs),
+                                   I(o_nfi), I(o_ss), I(o_sc), I(o_ts), (const int64_t *)(P + o_sbase), I(o_ntri),
+                                   I(o_pst), I(o_nfc), ntask, d0 + r0 * dstr, d1 + r0 * dstr, dstr, std::min(rb, nrhs - r0),
+                                   store->data.get<double>(), out + r0 * nstr, nstr);
+        };
+        auto layers = [&](auto nl) {
+            constexpr int NL = decltype(nl)::value, RB = NL == 2 ? 4 : 8;   // sets per pass over the store
+            if (nrhs > 1)
+                SL.fd && SL.fs ? run(k_near_replay<NL, true, true, RB>, RB)
+                               : SL.fd ? run(k_near_replay<NL, true, false, RB>, RB) : run(k_near_replay<NL, false, true, RB>, RB);
+            else
+                SL.fd && SL.fs ? run(k_near_replay<NL, true, true, 1>, 1)
+                               : SL.fd ? run(k_near_replay<NL, true, false, 1>, 1) : run(k_near_replay<NL, false, true, 1>, 1);
+        };
+        SL.ifsl + SL.ifdl == 2 ? layers(std::integral_constant<int, 2>{}) : layers(std::integral_constant<int, 1>{});
+        return hipGetLastError();
     };
     if (nrhs > 1 && !(store && icomp == 3)) return it->status == 64 ? 64 : 16;   // several sets: replays only
     HIPOK(hipEventRecord(W.ev_fork, stream));
@@ -2865,7 +2854,7 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
                 HIPOK(launch_hnear(ha, ntask, W.hq.p, store->data.get<double>(), ns));
                 HIPOK(run_replay(ns));
             } else if (store && icomp == 3) {
-                HIPOK(nrhs > 1 ? run_replay_multi(ns) : run_replay(ns));
+                HIPOK(run_replay(ns));
             } else {
                 W.htmp.ensure((size_t)h_tbase.back() * 8);
                 ha.sbase = (const int64_t *)(P + o_htbase);
@@ -2882,7 +2871,7 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
                            W.rec.get<double>(), ssl_s, sdl_s, rlam, rmu, c1, SL, store->data.get<double>(),
                            W.nf.get<double>());
     } else if (!nf_boxes.empty() && store && icomp == 3) {
-        HIPOK(nrhs > 1 ? run_replay_multi(ns) : run_replay(ns));
+        HIPOK(run_replay(ns));
     } else if (!PL.nf_tasks.empty() && (ifsl || ifdl)) {   // no layer: the near field stays zero
         hipLaunchKernelGGL(near_kernel(ifsl, ifdl, ifst || ifstt), dim3(PL.nf_tasks.size() / 3), dim3(64), 0, ns, n,
                            src_eval, I(o_nfb), I(o_nfs), I(o_nfi), I(o_ss), I(o_sc), I(o_ts), I(o_tc), I(o_nfw),
