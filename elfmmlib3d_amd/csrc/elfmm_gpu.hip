@@ -559,16 +559,14 @@ __global__ __launch_bounds__(Z::NT, 2) void k_p2l_tri(
 }
 
 // ------------------------------------------------------------------------
-// Translations (M2L, M2M, L2L): gather columns, multiply, scatter-add
+// Translations (M2L, M2M, L2L) on the matrix cores
 // ------------------------------------------------------------------------
 
-// Translations on the matrix cores with the translation rotated into the
-// xz-plane: per pair, x' = e^{i m phi} x (coefficient-wise), y'_re = R x'_re,
+// M2L of the lower orders (tiles with h < h_turned), with the translation
+// rotated into the xz-plane: per pair, x' = e^{i m phi} x (coefficient-wise), y'_re = R x'_re,
 // y'_im = I x'_im with the operator's two real h x h matrices, then
-// y = e^{-i k phi} y', scaled (1/s of the target box for M2L, 1 for M2M and
-// L2L) and added to the destination expansion. M2L has one operator per
-// list-2 offset, M2M and L2L one per child octant. A tile is ML_M = 64
-// output coefficients for ML_P = 32
+// y = e^{-i k phi} y', scaled (1/s of the target box) and added to the
+// destination expansion. A tile is ML_M = 64 output coefficients for ML_P = 32
 // pairs x NRHS right-hand sides (128 columns). Wave w owns coefficients
 // 16*(w/2) .. +16 and columns 64*(w%2) .. +64: 4 column blocks of 16 x 16
 // accumulators for the real parts and 4 for the imaginary parts, so the
@@ -584,7 +582,7 @@ constexpr int ML_APER = ML_M * ML_K / ML_THREADS;    // operator entries per thr
 constexpr int ML_BPER = ML_P * NRHS * ML_K / ML_THREADS;   // source entries per thread
 static_assert(ML_APER >= 1 && ML_BPER >= 1 && ML_K % 4 == 0, "loader shapes");
 
-__device__ __forceinline__ void trans_tile(const M2LTile *__restrict__ tiles, int ntiles,
+__global__ __launch_bounds__(ML_THREADS, 4) void k_m2l(const M2LTile *__restrict__ tiles, int ntiles, int h_turned,
                                                     const double *__restrict__ A_all,
                                                     const int *__restrict__ psrc,
                                                     const int *__restrict__ pdst,
@@ -605,7 +603,7 @@ __device__ __forceinline__ void trans_tile(const M2LTile *__restrict__ tiles, in
     int tix = blockIdx.x;
     if (tix >= ntiles) return;
     M2LTile t = tiles[tix];
-    if (t.npair <= 0) return;
+    if (t.npair <= 0 || t.h >= h_turned) return;
     const double *Rm = A_all + t.a_off, *Im = Rm + (size_t)t.h * t.h;
     int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int wr = (wave >> 1) * 16, wc = (wave & 1) * 64;
@@ -745,7 +743,234 @@ __device__ __forceinline__ void trans_tile(const M2LTile *__restrict__ tiles, in
     }
 }
 
-__global__ __launch_bounds__(ML_THREADS, 4) void k_m2l(const M2LTile *__restrict__ tiles, int ntiles,
+// M2M, L2L and M2L of the higher orders: a translation is rotated about z (e^{i m
+// phi} per coefficient), then about y so that it points along z, applied there,
+// and rotated back: the rotations mix
+// the orders of one degree, the shift the degrees of one order, and real and
+// imaginary parts stay apart, so a part goes through three block-diagonal
+// products of (p+1)^3 / 3 multiplications each instead of one dense product of
+// (p+1)^4 / 4 (order 26: 0.08 M to 0.29 M a pair and right-hand side, both
+// parts). M2M and L2L of 16,400 pairs at order 26: 0.89 ms, dense 1.49; the
+// M2L orders of 22 and more of 303,000 pairs 2.9 ms, dense 4.2; what is left is
+// the address arithmetic, the barriers and the adds, not the matrix cores. The
+// result is scaled (1/s of the target box for M2L, 1 for M2M and L2L) and added
+// to the destination expansion (FP64 atomics: several sources feed one).
+//
+// A workgroup takes TR_P = 4 pairs x NRHS right-hand sides, the 16 columns of a
+// matrix-core tile: the tile list is that of the dense products, the 8 parts
+// of a tile's 32 pairs are dealt to the group's row blocks (grid: tiles x
+// most parts of a row block). One part's coefficients stay in LDS, [coefficient][column],
+// through its three products, the other part's in registers. A unit of work is
+// 16 rows of one block: its operand comes from L2 as the matrix cores read it
+// (build_operators), the next unit's in flight during the products of this
+// one; the units, longest first, go to the W waves to and fro, and a product is
+// written back once all waves have read its operands. U units a wave, EJ
+// coefficients a lane and column, KM steps a unit at most.
+constexpr int TR_P = 4, TR_LD = TR_P * NRHS + 1;
+static_assert(TR_P * NRHS == 16, "columns of a matrix-core tile");
+struct TransTab {
+    int v[PMAX + 3];
+};
+constexpr TransTab make_trans_tab()
+{
+    TransTab t{};
+    for (int n = 0; n < PMAX + 3; n++) t.v[n] = (int)trans_blocks(n);
+    return t;
+}
+__constant__ const TransTab c_trans = make_trans_tab();
+
+// rows of LDS at order p: three degrees of zeros past the last
+__host__ __device__ constexpr int tr_rows(int p) { return (p + 4) * (p + 5) / 2; }
+inline size_t trans_lds(int p) { return (size_t)tr_rows(p) * TR_LD * 8; }
+
+template <int W, int U, int EJ, int KM>
+__device__ __forceinline__ void trans_tile(const M2LTile *__restrict__ tiles, int ntiles, int h_turned,
+                                           const double *__restrict__ A_all, const int *__restrict__ psrc,
+                                           const int *__restrict__ pdst, const double *__restrict__ pscale,
+                                           const double *__restrict__ X, double *__restrict__ Y, int nc, double *S)
+{
+    constexpr int C = 16 / W;                         // columns of a wave
+    __shared__ double2 cs[PMAX + 1];                  // (cos m phi, sin m phi)
+    // the tiles come in launch order (workgroup b on XCD b % 8); empty
+    // tiles fill the slots past an XCD's last one
+    if ((int)blockIdx.x >= ntiles) return;
+    const M2LTile t = tiles[blockIdx.x];
+    if (t.npair <= 0 || t.h < h_turned) return;
+    const int nrb = (t.h + ML_M - 1) / ML_M, rb = t.row0 / ML_M, parts = ML_P / TR_P;
+    const int sub = (parts * rb + nrb - 1) / nrb + (int)blockIdx.y;
+    if (sub >= (parts * (rb + 1) + nrb - 1) / nrb || sub * TR_P >= t.npair) return;
+    const int pair0 = t.pair0 + sub * TR_P, npair = min(TR_P, t.npair - sub * TR_P);
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = t.h, N = (int)((sqrtf(8.0f * h + 1.0f) - 1.0f) * 0.5f + 0.5f);   // p + 1
+    if (tid < N) {
+        double sn, c;
+        sincos(tid * t.phi, &sn, &c);
+        cs[tid] = double2{c, sn};
+    }
+    // the wave's columns, lane = coefficient
+    double2 x[C][EJ];
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int col = wave + W * c, pair = col / NRHS;
+        const bool on = pair < npair;
+        const double2 *Xc =
+            reinterpret_cast<const double2 *>(X + ((size_t)(on ? psrc[pair0 + pair] : 0) * NRHS + col % NRHS) * nc);
+#pragma unroll
+        for (int j = 0; j < EJ; j++) x[c][j] = on && lane + 64 * j < h ? Xc[lane + 64 * j] : double2{0.0, 0.0};
+    }
+    __syncthreads();
+    auto phase = [&](int k) {                         // and the signs (-1)^(l+m) of a z-mirrored operator
+        int l, m;
+        coef_nk(k, l, m);
+        double2 e = cs[m];
+        return t.refl && ((l + m) & 1) ? double2{-e.x, -e.y} : e;
+    };
+    for (int k = h * TR_LD + tid; k < tr_rows(N - 1) * TR_LD; k += 64 * W) S[k] = 0.0;
+    double keep[C][EJ];
+#pragma unroll
+    for (int j = 0; j < EJ; j++) {
+        const int k = lane + 64 * j;
+        if (k >= h) continue;
+        const double2 e = phase(k);
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            S[k * TR_LD + wave + W * c] = e.x * x[c][j].x - e.y * x[c][j].y;
+            keep[c][j] = e.y * x[c][j].x + e.x * x[c][j].y;
+        }
+    }
+    // unit s of the wave: size n of its block (0: none) and row tile rt
+    auto unit = [&](int s, int &n, int &rt) {
+        int u = W * s + (s & 1 ? W - 1 - wave : wave), c3 = max(N - 32, 0) * 3;
+        if (u < c3) {
+            n = N - u / 3;
+            rt = u % 3;
+            return;
+        }
+        u -= c3;
+        int top = min(N, 32), c2 = max(top - 16, 0) * 2;
+        if (u < c2) {
+            n = top - u / 2;
+            rt = u & 1;
+            return;
+        }
+        n = max(min(top, 16) - (u - c2), 0);
+        rt = 0;
+    };
+    const double *rec = A_all + t.a_off + lane;
+    const int Z = c_trans.v[N + 1];
+    // One product of a part. SHIFT: blocks of an order, whose coefficients lie j
+    // apart at degree j; else of a degree, one after the other. Columns past a
+    // block meet zeros of the operand: they read what follows (the rows past the
+    // last coefficient are zero).
+    auto product = [&](auto shift, const double *B) {
+        constexpr bool SHIFT = decltype(shift)::value;
+        double a[KM];
+        auto load = [&](int s) {
+            int n, rt;
+            unit(s, n, rt);
+            const int ks = (n + 3) >> 2;
+            const double *Ap = B + c_trans.v[n] + rt * ks * 64;
+#pragma unroll
+            for (int q = 0; q < KM; q++) a[q] = q < ks ? Ap[q * 64] : 0.0;
+        };
+        // coefficient of row k of a block of size n
+        auto coef = [&](int n, int k) {
+            return SHIFT ? (N - n + k) * (N - n + k + 1) / 2 + N - n : n * (n - 1) / 2 + k;
+        };
+        gemm_d4 acc[U];
+        load(0);
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < U; s++) {
+            int n, rt;
+            unit(s, n, rt);
+            acc[s] = gemm_d4{0.0, 0.0, 0.0, 0.0};
+            const int ks = (n + 3) >> 2;
+            const double *row = S + coef(n, lq) * TR_LD + li;
+            int step = (4 * (N - n + lq) + 10) * TR_LD;
+#pragma unroll
+            for (int q = 0; q < KM; q++)
+                if (q < ks) {
+                    double b = SHIFT ? *row : row[4 * q * TR_LD];
+                    acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], b, acc[s], 0, 0, 0);
+                    if (SHIFT) {
+                        row += step;
+                        step += 16 * TR_LD;
+                    }
+                }
+            if (s + 1 < U) load(s + 1);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < U; s++) {
+            int n, rt;
+            unit(s, n, rt);
+            const int k0 = 16 * rt + lq;              // lane holds rows lane/16 + 4 i of the tile, column lane % 16
+            double *row = S + coef(n, k0) * TR_LD + li;
+            int step = (4 * (N - n + k0) + 10) * TR_LD;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                if (k0 + 4 * i < n) *(SHIFT ? row : row + 4 * i * TR_LD) = acc[s][i];
+                if (SHIFT) {
+                    row += step;
+                    step += 16 * TR_LD;
+                }
+            }
+        }
+    };
+#pragma unroll 1
+    for (int part = 0; part < 2; part++) {
+        product(std::false_type{}, rec + (size_t)Z * part);
+        product(std::true_type{}, rec + (size_t)Z * 2);
+        product(std::false_type{}, rec + (size_t)Z * (3 + part));
+        __syncthreads();
+        if (part == 0)
+#pragma unroll
+            for (int j = 0; j < EJ; j++) {
+                const int k = lane + 64 * j;
+                if (k >= h) continue;
+#pragma unroll
+                for (int c = 0; c < C; c++) {
+                    double v = S[k * TR_LD + wave + W * c];
+                    S[k * TR_LD + wave + W * c] = keep[c][j];
+                    keep[c][j] = v;
+                }
+            }
+    }
+    // rotated back about z, scaled and added: 64 consecutive doubles of the
+    // destination per step
+    double sc[C];
+    double *y[C];
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int col = wave + W * c, pair = col / NRHS;
+        const bool on = pair < npair;
+        sc[c] = on ? pscale[pair0 + pair] : 0.0;
+        y[c] = on ? Y + ((size_t)pdst[pair0 + pair] * NRHS + col % NRHS) * nc : nullptr;
+    }
+#pragma unroll
+    for (int j = 0; j < EJ; j++) {
+        if (64 * j >= h) break;
+        const int k = lane + 64 * j;
+        const double2 e = k < h ? phase(k) : double2{0.0, 0.0};
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            if (!y[c]) continue;
+            double yr = k < h ? keep[c][j] : 0.0, yi = k < h ? S[k * TR_LD + wave + W * c] : 0.0;
+            double re = (e.x * yr + e.y * yi) * sc[c], im = (e.x * yi - e.y * yr) * sc[c];
+#pragma unroll
+            for (int half = 0; half < 2; half++) {
+                int src = 32 * half + (lane >> 1);
+                double vr = __shfl(re, src), vi = __shfl(im, src);
+                if (64 * j + src < h) unsafeAtomicAdd(y[c] + 128 * j + 64 * half + lane, lane & 1 ? vi : vr);
+            }
+        }
+    }
+}
+
+template <int W, int U, int EJ, int KM>
+__global__ __launch_bounds__(64 * W, 4) void k_m2l_turned(const M2LTile *__restrict__ tiles, int ntiles, int h_turned,
                                                     const double *__restrict__ A_all,
                                                     const int *__restrict__ psrc,
                                                     const int *__restrict__ pdst,
@@ -753,11 +978,13 @@ __global__ __launch_bounds__(ML_THREADS, 4) void k_m2l(const M2LTile *__restrict
                                                     const double *__restrict__ X, double *__restrict__ Y,
                                                     int nc)
 {
-    trans_tile(tiles, ntiles, A_all, psrc, pdst, pscale, X, Y, nc);
+    extern __shared__ double lds[];
+    trans_tile<W, U, EJ, KM>(tiles, ntiles, h_turned, A_all, psrc, pdst, pscale, X, Y, nc, lds);
 }
 
 // M2M / L2L of one level: the same body with the octants' operators
-__global__ __launch_bounds__(ML_THREADS, 4) void k_m2m_l2l(const M2LTile *__restrict__ tiles, int ntiles,
+template <int W, int U, int EJ, int KM>
+__global__ __launch_bounds__(64 * W, 4) void k_m2m_l2l(const M2LTile *__restrict__ tiles, int ntiles, int h_turned,
                                                     const double *__restrict__ A_all,
                                                     const int *__restrict__ psrc,
                                                     const int *__restrict__ pdst,
@@ -765,7 +992,24 @@ __global__ __launch_bounds__(ML_THREADS, 4) void k_m2m_l2l(const M2LTile *__rest
                                                     const double *__restrict__ X, double *__restrict__ Y,
                                                     int nc)
 {
-    trans_tile(tiles, ntiles, A_all, psrc, pdst, pscale, X, Y, nc);
+    extern __shared__ double lds[];
+    trans_tile<W, U, EJ, KM>(tiles, ntiles, h_turned, A_all, psrc, pdst, pscale, X, Y, nc, lds);
+}
+
+// The kernels: 8 waves to order 26 (38 units, 378 coefficients: two workgroups
+// a CU), 16 to PMAX (87 and 1035).
+static_assert(PMAX <= 44, "units and coefficients of the largest order");
+// (Order 39, M2M and L2L: 0.71 ms with 16 waves, 0.83 with 8, dense 1.20.)
+constexpr auto k_m2l_turned_26 = k_m2l_turned<8, 5, 6, 7>, k_m2l_turned_max = k_m2l_turned<16, 6, 17, 12>;
+constexpr auto k_m2m_l2l_26 = k_m2m_l2l<8, 5, 6, 7>, k_m2m_l2l_max = k_m2m_l2l<16, 6, 17, 12>;
+static_assert(tr_rows(PMAX) * TR_LD * 8 + (PMAX + 1) * 16 <= 160 * 1024, "LDS of a CU");
+inline auto m2m_l2l_kernel(int p) { return p <= 26 ? k_m2m_l2l_26 : k_m2m_l2l_max; }
+inline int trans_threads(int p) { return p <= 26 ? 512 : 1024; }
+// h: the fewest coefficients among the tiles (a row block then has most parts)
+inline dim3 trans_grid(int ntiles, int h)
+{
+    int nrb = (h + ML_M - 1) / ML_M;
+    return dim3(ntiles, (ML_P / TR_P + nrb - 1) / nrb);
 }
 
 
@@ -1899,6 +2143,10 @@ DeviceState &device_state()
         // M2T stages the four expansions of a slot (order up to PMAX) in LDS
         int mf = NRHS * (PMAX + 1) * (PMAX + 2) * 8;
         HIPOK(hipFuncSetAttribute((const void *)k_m2t, hipFuncAttributeMaxDynamicSharedMemorySize, mf));
+        for (auto *k : {k_m2l_turned_max, k_m2m_l2l_max})
+            HIPOK(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)trans_lds(PMAX)));
+        for (auto *k : {k_m2l_turned_26, k_m2m_l2l_26})
+            HIPOK(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)trans_lds(26)));
         int wide = 8 * P2X_WIDE_STRIDE * 8;
         ds->p2x_wide =
             hipFuncSetAttribute((const void *)k_p2m<16, 7, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, wide) ==
@@ -2223,15 +2471,36 @@ void far_scratch(int iprec, int n, int np, int nb, int p, size_t &nodes, size_t 
 // memsets, copies or host waits), so that it can be captured into a graph.
 // mark(k, begin), when given, brackets phase k (2 nodes and P2M, 3 M2M, 4
 // M2L, 5 P2L, 6 L2L, 7 L2T, 8 M2T) for the caller's timing events.
-// M2M / L2L of one level: rotated translations, the kernel of M2L (unit scale)
+// M2M / L2L of one level (unit scale)
 void enqueue_trans(const GemmLaunch &g, const LaunchOff &l, const char *P, const DevBuf &A, const double *X, double *Y,
                    int nc, Lane &ln)
 {
     if (g.tiles.empty()) return;
-    int ntiles = (int)g.tiles.size();
-    ln.launch(k_m2m_l2l, dim3(ntiles), dim3(ML_THREADS), 0, (const M2LTile *)(P + l.tiles), ntiles,
-              (const double *)A.p, (const int *)(P + l.src), (const int *)(P + l.dst), (const double *)(P + l.sc), X,
-              Y, nc);
+    int ntiles = (int)g.tiles.size(), p = (int)(std::sqrt(nc + 0.25) - 1.0);   // nc = (p + 1)(p + 2)
+    ln.launch(m2m_l2l_kernel(p), trans_grid(ntiles, nc / 2), dim3(trans_threads(p)), trans_lds(p), (const M2LTile *)(P + l.tiles),
+              ntiles, 0, (const double *)A.p, (const int *)(P + l.src), (const int *)(P + l.dst),
+              (const double *)(P + l.sc), X, Y, nc);
+}
+
+// M2L: the turned orders (the list's first tiles, xcd_order), then the others
+void enqueue_m2l_tiles(const std::vector<M2LTile> &list, size_t at, const LaunchOff &l, const char *P, const double *A,
+                       int p, const double *X, double *Y, Lane &ln)
+{
+    const int nc = ncoef(p), ht = m2l_turned_h(p);
+    auto turned = [&](const M2LTile &t) { return t.npair > 0 && t.h >= ht; };
+    int n1 = (int)list.size(), n0 = 0;
+    while (n1 && !turned(list[n1 - 1])) n1--;
+    while (n0 < (int)list.size() && (turned(list[n0]) || list[n0].npair <= 0)) n0++;
+    n0 = n0 / 8 * 8;                                  // XCD of a workgroup: index % 8
+    const M2LTile *tiles = (const M2LTile *)(P + at);
+    const int *src = (const int *)(P + l.src), *dst = (const int *)(P + l.dst);
+    const double *sc = (const double *)(P + l.sc);
+    if (n1)
+        ln.launch(p <= 26 ? k_m2l_turned_26 : k_m2l_turned_max, trans_grid(n1, ht), dim3(trans_threads(p)), trans_lds(p), tiles, n1, ht, A, src, dst, sc, X, Y,
+                  nc);
+    const int nd = (int)list.size() - n0;
+    if (nd > 0)
+        ln.launch(k_m2l, dim3(nd), dim3(ML_THREADS), 0, tiles + n0, nd, ht, A, src, dst, sc, X, Y, nc);
 }
 
 // P2M, M2M and P2L (build_plan_up)
@@ -2318,12 +2587,8 @@ void enqueue_m2l(const FarLaunch &a, Lane &ln, Mark mark)
     const int nc = ncoef(oc.p);
     double *mp = a.exps, *lo = mp + (size_t)a.nb * NRHS * nc;
     mark(4, true);
-    if (!PL.m2l_tiles.empty()) {
-        int ntiles = (int)PL.m2l_tiles.size();
-        ln.launch(k_m2l, dim3(ntiles), dim3(ML_THREADS), 0, (const M2LTile *)(P + o.m2lt), ntiles,
-                  (const double *)oc.m2l.p, (const int *)(P + o.m2l.src), (const int *)(P + o.m2l.dst),
-                  (const double *)(P + o.m2l.sc), (const double *)mp, lo, nc);
-    }
+    enqueue_m2l_tiles(PL.m2l_tiles, o.m2lt, o.m2l, P, (const double *)oc.m2l.p, oc.p, mp,
+                      lo, ln);
     mark(4, false);
     mark(6, true);
     for (size_t k = 0; k < PL.l2l_l.size(); k++) enqueue_trans(PL.l2l_l[k], o.l2l[k], P, oc.l2l, lo, lo, nc, ln);
@@ -3536,34 +3801,23 @@ int mindlin_far_dev(int iprec, double rlam, double rmu, int n, const double *d_t
     } else {
         HIPOK(launch_mind_p2m(md, I(M.o_p2m), nbx, stream));
     }
-    auto run_trans = [&](const GemmLaunch &g, const LaunchOff &o, const double *A, const double *X, double *Y,
-                         bool m2l) {
-        if (g.tiles.empty()) return;
-        int ntiles = (int)g.tiles.size();
-        if (m2l)
-            hipLaunchKernelGGL(k_m2l, dim3(ntiles), dim3(ML_THREADS), 0, stream, (const M2LTile *)(P + o.tiles),
-                               ntiles, A, (const int *)(P + o.src), (const int *)(P + o.dst),
-                               (const double *)(P + o.sc), X, Y, nc);
-        else
-            hipLaunchKernelGGL(k_m2m_l2l, dim3(ntiles), dim3(ML_THREADS), 0, stream, (const M2LTile *)(P + o.tiles),
-                               ntiles, A, (const int *)(P + o.src), (const int *)(P + o.dst),
-                               (const double *)(P + o.sc), X, Y, nc);
-        HIPOK(hipGetLastError());
-    };
+    Lane ln;
+    ln.stream = stream;
     for (size_t k = 0; k < PL.m2m_l.size(); k++) {
-        run_trans(PL.m2m_l[k], M.off_m2m[k], oc->m2m.get<double>(), mp, mp, false);
+        enqueue_trans(PL.m2m_l[k], M.off_m2m[k], P, oc->m2m, mp, mp, nc, ln);
         HIPOK(launch_mind_bscale(md, I(M.o_bsc[k]), (int)M.bsc[k].size(), stream));
     }
     // plane waves, proxy rings and B's remainder of every sourced box
     HIPOK(launch_mind_bmod(md, I(M.o_src), (int)MP.src_boxes.size(), stream));
     // list 2: near pairs (exact M2L of the remainder of B, and of C1, C2;
     // the proxies' field), far pairs (plane waves)
-    run_trans(MP.m2l, M.off_m2l, oc->mind_m2l.get<double>(), mp, lo, true);
+    enqueue_m2l_tiles(MP.m2l.tiles, M.off_m2l.tiles, M.off_m2l, P,
+                      oc->mind_m2l.get<double>(), p, mp, lo, ln);
     HIPOK(launch_mind_proxy(md, I(M.o_px), (int)MP.px_tasks.size() / 3, I(M.off_m2l.src), I(M.off_m2l.dst), stream));
     HIPOK(launch_mind_far(md, I(M.o_fb), I(M.o_fs), I(M.o_fi), (int)MP.far_boxes.size(), stream));
     // downward pass and evaluation
     for (size_t k = 0; k < PL.l2l_l.size(); k++)
-        run_trans(PL.l2l_l[k], M.off_l2l[k], oc->l2l.get<double>(), lo, lo, false);
+        enqueue_trans(PL.l2l_l[k], M.off_l2l[k], P, oc->l2l, lo, lo, nc, ln);
     S.lap.ensure((size_t)np * 40 * 8);
     HIPOK(hipMemsetAsync(S.lap.p, 0, (size_t)np * 40 * 8, stream));
     if (!PL.l2t_tpt.empty()) {

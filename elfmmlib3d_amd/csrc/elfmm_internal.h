@@ -63,19 +63,42 @@ int build_tree(const double *src, int n, const double *targ, int nt, int nbox,
 // coefficient (re, im) sits at 2*(l*(l+1)/2 + m); ncoef(p) doubles total.
 inline int ncoef(int p) { return (p + 1) * (p + 2); }
 
-// Dense translation operators on packed, box-size-scaled expansions.
+// Doubles of the blocks of sizes 1 .. n - 1 in a translation's record: a block,
+// n x n, is stored as the matrix cores read it, 64 doubles (lane 16 c + r: row r,
+// column c of a 16 x 4 part) per row tile of 16 and step of 4 columns.
+constexpr size_t trans_blocks(int n)
+{
+    size_t z = 0;
+    for (int k = 1; k < n; k++) z += (size_t)((k + 15) / 16) * ((k + 3) / 4) * 64;
+    return z;
+}
+// Record of a translation of order p: the rotation to the z axis of the real
+// parts and of the imaginary parts (blocks of degree n - 1), the shift along z
+// (blocks of order p + 1 - n), and the rotation back of both.
+constexpr size_t trans_doubles(int p) { return 5 * trans_blocks(p + 2); }
+
+// M2L offsets whose order has at least this many coefficients are applied by
+// their records at expansion order p, the others by dense products, 32 pairs to
+// an operator read: below, the adds to the destinations bound either way, and a
+// record's six products with their barriers cost more than the dense ones
+// (order 26, 303,000 pairs: 4.5 ms split between the orders 16 and 22,
+// all dense 5.3, all by records 5.8; order 39, 53,000 pairs, split between 23
+// and 24: 3.3 ms, all dense 3.7).
+inline int m2l_turned_h(int p) { return p <= 26 ? 260 : 310; }
+
+// Translation operators on packed, box-size-scaled expansions.
 struct Operators {
     int p = 0;
     int nc = 0;                          // ncoef(p)
-    // M2M / L2L per octant, rotated into the xz-plane (as M2L): two real
-    // (nc/2)^2 matrices each, real-part then imaginary-part, and the azimuth
+    // M2M / L2L per octant: its record and the azimuth
     std::vector<double> m2m;
     std::vector<double> l2l;
     double oct_phi[8];
     // M2L per offset (i,j,k) in [-3,3]^3 with max|.|>=2: truncation order
-    // pt, azimuth phi of the translation, and at m2l_off[o] the two real
-    // (ncoef(pt)/2)^2 matrices of the translation rotated into the xz-plane
-    // (real parts, then imaginary parts; see build_operators).
+    // pt, azimuth phi of the translation, and at m2l_off[o] its record where
+    // ncoef(pt)/2 >= m2l_turned_h(p), else the two real (ncoef(pt)/2)^2
+    // matrices of the translation rotated into the xz-plane (real parts, then
+    // imaginary parts).
     int m2l_pt[343];
     int64_t m2l_off[343];
     // 1 when offset o uses the stored operator of its mirror image in z:
@@ -101,11 +124,11 @@ struct alignas(16) FieldTerm {   // 48 bytes; the device reads idx and c[0..1] a
 };
 void build_field_table(int p, bool irr, std::vector<FieldTerm> &tab);
 
-// One tile of a rotated translation (M2L, M2M, L2L): ML_M coefficients
-// (real and imaginary parts) of one operator for up to ML_P (source,
-// destination) pairs.
+// One tile of a translation (M2L, M2M, L2L): ML_M coefficients (real and
+// imaginary parts) of one operator for up to ML_P (source, destination)
+// pairs; where the operator is a record, the group's tiles share its pairs.
 struct M2LTile {
-    int64_t a_off;   // offset of the real-part matrix (h x h, row-major); imaginary part follows
+    int64_t a_off;   // offset of the operator
     int h;           // coefficients = ncoef(pt) / 2
     int row0;        // first output coefficient of this tile
     int pair0;       // first pair of this tile

@@ -1,4 +1,4 @@
-// Host planner, part 2: dense translation operators.
+// Host planner, part 2: translation operators.
 //
 // Expansions use Racah-normalised solid harmonics with the Condon-Shortley
 // phase,
@@ -127,76 +127,113 @@ void add_entry(std::vector<double> &A, size_t base, int ncol, int jo, int ko, in
     }
 }
 
+// Wigner's d^l of the rotation that takes the direction (sin t, 0, cos t) to the
+// z axis, on harmonics with the Condon-Shortley phase: R_l^k(Q x) =
+// sum_m d(k, m) R_l^m(x). By Jacobi polynomials (Varshalovich et al., Quantum
+// theory of angular momentum, 4.3.4): with a = |k - m|, b = |k + m|, s = l -
+// max(|k|, |m|),
+//   d(k, m) = sg sqrt(s! (s+a+b)! / ((s+a)! (s+b)!)) sin^a cos^b P_s^(a,b)(cos t)
+// (sin, cos of t / 2), sg = (-1)^(m-k) for k < m, else 1.
+long double wigner(int l, int k, int m, long double c, long double sh, long double ch)
+{
+    int a = std::abs(k - m), b = std::abs(k + m), s = l - std::max(std::abs(k), std::abs(m));
+    long double p0 = 1, p1 = s ? (a + 1) + (a + b + 2) * (c - 1) / 2 : 1;
+    for (int n = 2; n <= s; n++) {
+        long double q = 2.0L * n + a + b;
+        long double p2 = ((q - 1) * (q * (q - 2) * c + (long double)a * a - (long double)b * b) * p1 -
+                          2 * (n + a - 1.0L) * (n + b - 1.0L) * q * p0) /
+                         (2.0L * n * (n + a + b) * (q - 2));
+        p0 = p1;
+        p1 = p2;
+    }
+    long double f = 1;                                // s! (s+a+b)! / ((s+a)! (s+b)!)
+    for (int i = 1; i <= a; i++) f *= (long double)(s + b + i) / (s + i);
+    return ((k < m && ((m - k) & 1)) ? -1 : 1) * std::sqrt(f) * std::pow(sh, a) * std::pow(ch, b) * p1;
+}
+
+// The record of one translation by (rho, 0, z) at order p (see trans_doubles):
+// T(j, l, m) the coefficient from degree l to degree j of order m of the
+// translation by its length along z.
+template <class F>
+void pack_translation(int p, double rho, double z, F &&T, double *o)
+{
+    const long double r = std::sqrt((long double)rho * rho + (long double)z * z), c = z / r;
+    const long double sh = std::sqrt((1 - c) / 2), ch = std::sqrt((1 + c) / 2);
+    const size_t Z = trans_blocks(p + 2);
+    std::vector<double> M;
+    auto put = [&](double *dst, int n) {              // n x n matrix M: row tiles of 16, steps of 4 columns, lane order
+        int ks = (n + 3) / 4;
+        for (int rt = 0; rt < (n + 15) / 16; rt++)
+            for (int k = 0; k < ks; k++)
+                for (int lane = 0; lane < 64; lane++) {
+                    int row = 16 * rt + lane % 16, col = 4 * k + lane / 16;
+                    *dst++ = row < n && col < n ? M[(size_t)row * n + col] : 0.0;
+                }
+    };
+    for (int n = 1; n <= p + 1; n++) {
+        // rotations of degree l = n - 1: into the frame with the translation
+        // along z (d) and back (d transposed); orders m < 0 of a real field folded,
+        // c^{-m} = (-1)^m conj(c^m): sums for the real parts, differences for the imaginary
+        int l = n - 1;
+        size_t off = trans_blocks(n);
+        for (int back = 0; back < 2; back++)
+            for (int im = 0; im < 2; im++) {
+                M.assign((size_t)n * n, 0.0);
+                for (int k = im; k <= l; k++)
+                    for (int m = im; m <= l; m++) {
+                        auto d = [&](int mm) { return back ? wigner(l, mm, k, c, sh, ch) : wigner(l, k, mm, c, sh, ch); };
+                        long double v = d(m);
+                        if (m) v += ((m & 1) != im ? -1 : 1) * d(-m);
+                        M[(size_t)k * n + m] = (double)v;
+                    }
+                put(o + (back ? 3 + im : im) * Z + off, n);
+            }
+        // shift of order m = p + 1 - n: degrees m .. p
+        int m = p + 1 - n;
+        M.assign((size_t)n * n, 0.0);
+        for (int j = 0; j < n; j++)
+            for (int k = 0; k < n; k++) M[(size_t)j * n + k] = (double)T(m + j, m + k, m, r);
+        put(o + 2 * Z + off, n);
+    }
+}
+
 }  // namespace
 
+// A translation by t = Rz(phi) (rho, 0, z) is applied as a rotation about z
+// (e^{i m phi}, in the kernel), one about y that takes (rho, 0, z) to the z axis,
+// the translation along z, where orders do not mix, and both rotations back. In
+// the turned frame all coefficients are real: real parts map to real parts,
+// imaginary to imaginary.
 void build_operators(int p, const int *itable, Operators &ops)
 {
     ops.p = p;
-    int nc = ncoef(p), h = nc / 2;
-    ops.nc = nc;
-    // M2M / L2L per octant, rotated like M2L below: the child-centre offset
-    // t = Rz(phi) t' with t' = (rho, 0, tz) in the xz-plane, where the
-    // regular harmonics R_n^q(t') are real, so on coefficients rotated by
-    // e^{i m phi} the translation is real: real parts to real parts and
-    // imaginary parts to imaginary parts, two h x h matrices per octant
-    // (real-part matrix, then imaginary-part matrix).
-    ops.m2m.assign((size_t)8 * 2 * h * h, 0.0);
-    ops.l2l.assign((size_t)8 * 2 * h * h, 0.0);
-    std::vector<double> pw(p + 1);
-    for (int l = 0; l <= p; l++) pw[l] = std::ldexp(1.0, -l);
-    std::vector<double> Dm((size_t)nc * nc), Dl((size_t)nc * nc);
+    ops.nc = ncoef(p);
+    // M2M / L2L per octant; t = child centre minus parent centre, in units of
+    // the parent side
+    const size_t sz = trans_doubles(p);
+    ops.m2m.assign(8 * sz, 0.0);
+    ops.l2l.assign(8 * sz, 0.0);
+    std::vector<long double> half(p + 1);
+    for (int l = 0; l <= p; l++) half[l] = std::ldexp(1.0L, -l);
     for (int o = 0; o < 8; o++) {
-        // child centre minus parent centre, in units of the parent side
         double t[3] = {(o & 1) ? 0.25 : -0.25, (o & 2) ? 0.25 : -0.25, (o & 4) ? 0.25 : -0.25};
+        double rho = std::sqrt(t[0] * t[0] + t[1] * t[1]);
         ops.oct_phi[o] = std::atan2(t[1], t[0]);
-        Harm R = regular(p, std::sqrt(t[0] * t[0] + t[1] * t[1]), 0.0, t[2]);
-        std::fill(Dm.begin(), Dm.end(), 0.0);
-        std::fill(Dl.begin(), Dl.end(), 0.0);
-        for (int l = 0; l <= p; l++)
-            for (int m = 0; m <= l; m++)
-                for (int j = 0; j <= l; j++)
-                    for (int k = -j; k <= j; k++) {
-                        if (std::abs(m - k) > l - j) continue;
-                        double c = std::sqrt(binom(l + m, j + k) * binom(l - m, j - k));
-                        // M2M: Mp_l^m += c 2^-j Mc_j^k conj(R_{l-j}^{m-k}(t))
-                        add_entry(Dm, 0, nc, l, m, j, k, c * pw[j] * std::conj(R.get(l - j, m - k)));
-                        // L2L: Lc_j^k += c 2^-j Lp_l^m R_{l-j}^{m-k}(t)
-                        if (k >= 0) add_entry(Dl, 0, nc, j, k, l, m, c * pw[j] * R.get(l - j, m - k));
-                    }
-        // L2L needs inputs of negative order too
-        for (int l = 0; l <= p; l++)
-            for (int m = -l; m < 0; m++)
-                for (int j = 0; j <= l; j++)
-                    for (int k = 0; k <= j; k++) {
-                        if (std::abs(m - k) > l - j) continue;
-                        double c = std::sqrt(binom(l + m, j + k) * binom(l - m, j - k));
-                        add_entry(Dl, 0, nc, j, k, l, m, c * pw[j] * R.get(l - j, m - k));
-                    }
-        for (int which = 0; which < 2; which++) {
-            const std::vector<double> &D = which ? Dl : Dm;
-            double *Rm = (which ? ops.l2l : ops.m2m).data() + (size_t)o * 2 * h * h, *Im = Rm + (size_t)h * h;
-            double big = 0, cross = 0;
-            for (int r = 0; r < h; r++)
-                for (int c = 0; c < h; c++) {
-                    Rm[(size_t)r * h + c] = D[(size_t)(2 * r) * nc + 2 * c];
-                    Im[(size_t)r * h + c] = D[(size_t)(2 * r + 1) * nc + 2 * c + 1];
-                    big = std::max(big, std::max(std::abs(Rm[(size_t)r * h + c]), std::abs(Im[(size_t)r * h + c])));
-                    cross = std::max(cross, std::max(std::abs(D[(size_t)(2 * r) * nc + 2 * c + 1]),
-                                                     std::abs(D[(size_t)(2 * r + 1) * nc + 2 * c])));
-                }
-            if (cross > 1e-13 * big) throw std::runtime_error("rotated M2M/L2L operator is not real");
-        }
+        // Mp_l^m += sqrt(C(l+m,j+m) C(l-m,j-m)) 2^-j Mc_j^m r^(l-j)
+        auto up = [&](int l, int j, int m, long double r) {
+            return j > l ? 0 : std::sqrt(binom(l + m, j + m) * binom(l - m, j - m)) * half[j] * std::pow(r, l - j);
+        };
+        // Lc_j^m += sqrt(C(l+m,j+m) C(l-m,j-m)) 2^-j Lp_l^m r^(l-j)
+        auto down = [&](int j, int l, int m, long double r) {
+            return j > l ? 0 : std::sqrt(binom(l + m, j + m) * binom(l - m, j - m)) * half[j] * std::pow(r, l - j);
+        };
+        pack_translation(p, rho, t[2], up, &ops.m2m[o * sz]);
+        pack_translation(p, rho, t[2], down, &ops.l2l[o * sz]);
     }
     // M2L per offset; offsets are source ijk minus target ijk, so the
-    // translation vector (target centre minus source centre) is -offset.
-    // With t = Rz(phi) t', t' = (rho, 0, tz) in the xz-plane,
-    // I_n^q(t) = e^{i q phi} I_n^q(t') and I_n^q(t') is real, so
-    //   L_j^k = e^{-i k phi} sum_{l,m} a_{jklm}(t') (e^{i m phi} M_l^m)
-    // with real a: on the rotated coefficients the real parts map to real
-    // parts and the imaginary parts to imaginary parts, each by a real
-    // ncoef(pt)/2 square matrix (rows j,k; columns l,m >= 0). Stored per
-    // offset: the real-part matrix, then the imaginary-part matrix.
-    // The rotated operator depends on the offset only through rho^2 =
+    // translation vector (target centre minus source centre) is -offset:
+    //   L_j^m = sum_l (-1)^(j+m) sqrt(C(l+j,j+m) C(l+j,j-m)) M_l^m / r^(l+j+1)
+    // along z. The operator depends on the offset only through rho^2 =
     // i^2 + j^2, k and pt: offsets that share them (up to eight, mirror
     // images in x, y and the diagonal) share one stored copy. The mirror
     // image in z shares it too: the irregular harmonics of the translation
@@ -224,13 +261,24 @@ void build_operators(int p, const int *itable, Operators &ops)
                 break;
             }
         }
-        if (owner[o] < 0) tot += (size_t)2 * (ncoef(pt) / 2) * (ncoef(pt) / 2);
+        const size_t h = ncoef(pt) / 2;
+        if (owner[o] < 0) tot += (int)h >= m2l_turned_h(p) ? trans_doubles(pt) : 2 * h * h;
     }
     ops.m2l.assign(tot, 0.0);
     for (int o = 0; o < 343; o++) {
         int pt = ops.m2l_pt[o];
         if (pt < 0 || owner[o] >= 0) continue;
         int i = o / 49 - 3, j = (o / 7) % 7 - 3, k = o % 7 - 3;
+        if (ncoef(pt) / 2 >= m2l_turned_h(p)) {
+            auto far = [](int jo, int l, int m, long double r) {
+                return (((jo + m) & 1) ? -1 : 1) * std::sqrt((long double)binom(l + jo, jo + m) * binom(l + jo, jo - m)) /
+                       std::pow(r, l + jo + 1);
+            };
+            pack_translation(pt, std::sqrt((double)(i * i + j * j)), -(double)k, far, &ops.m2l[(size_t)ops.m2l_off[o]]);
+            continue;
+        }
+        // in the xz-plane I_n^q(t') is real: L_j^k = e^{-i k phi} sum_{l,m}
+        // a_{jklm}(t') (e^{i m phi} M_l^m) with real a
         int n = ncoef(pt), h = n / 2;
         double rho = std::sqrt((double)(i * i + j * j));
         Harm I = irregular(2 * pt, rho, 0.0, -(double)k);

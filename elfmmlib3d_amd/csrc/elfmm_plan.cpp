@@ -97,11 +97,12 @@ inline int offset_index(const Tree &T, int j, int b)
            (T.ijk[3 * j + 2] - T.ijk[3 * b + 2] + 3);
 }
 
-// M2M (up) or L2L (down) launch for one level: pairs grouped by octant,
-// each octant's rotated operator (two h x h matrices, h = nc / 2).
+// M2M (up) or L2L (down) launch for one level: pairs grouped by octant.
 GemmLaunch tree_pass(const Tree &T, int lev, int nc, const double *oct_phi, bool up)
 {
-    int h = nc / 2;
+    int h = nc / 2, p = 0;
+    while (ncoef(p) < nc) p++;
+    const int64_t oper = (int64_t)trans_doubles(p);
     GemmLaunch g;
     std::vector<int> s[8], d[8];
     for (int b = T.laddr[2 * lev]; b < T.laddr[2 * lev] + T.laddr[2 * lev + 1]; b++) {
@@ -117,7 +118,7 @@ GemmLaunch tree_pass(const Tree &T, int lev, int nc, const double *oct_phi, bool
     for (int o = 0; o < 8; o++)
         if (!s[o].empty()) {
             std::vector<double> one(s[o].size(), 1.0);
-            add_pairs(g, (int64_t)o * 2 * h * h, h, oct_phi[o], s[o].data(), d[o].data(), one.data(),
+            add_pairs(g, o * oper, h, oct_phi[o], s[o].data(), d[o].data(), one.data(),
                       (int)s[o].size());
         }
     xcd_order(g.tiles);
