@@ -3064,20 +3064,24 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
         const double *d0 = nrhs > 1 ? (SL.ifsl ? dm0 : dm1) : (SL.ifsl ? ssl_s : sdl_s), *d1 = nrhs > 1 ? dm1 : sdl_s;
         double *out = nrhs > 1 ? W.nfm.get<double>() : W.nf.get<double>();
         size_t dstr = (size_t)n * 3, nstr = (size_t)np * 9;
-        // One set beside its far field: a workgroup per CU, each taking every
-        // grid-th task. That reads at 4.3 TB/s and leaves the registers of
-        // three quarters of a SIMD to the far field, which else waits for the
-        // whole replay: a product of 46,080 triangles at order 26 takes 3.85 ms
-        // (4.44 unlimited, 4.2 with two per CU), of 15,680 at order 14 1.00
-        // (1.16). Unlimited: order 39, where a workgroup of P2M takes a whole
-        // CU (2.15, limited 2.31), several sets, whose far fields outweigh the
-        // replay (16 sets of 32,000 triangles: 16.0, limited 18.4), and no far
-        // field.
-        const bool limit = nrhs == 1 && oc && !near_only && T.nlev >= 2 && p <= 30;
+        // One set beside its far field: a few workgroups per CU, each taking
+        // every grid-th task, which leaves registers to the far field; launched
+        // whole, the replay holds every CU and P2M, half a CU's registers a
+        // workgroup, waits for its end. One per CU where the replay is short
+        // (order 26, 14.5 GB: 3.59 ms a product, 3.98 with three, 4.12 whole; 9.8
+        // GB: 2.12, 2.42, 2.41); three where it outlasts the far field, which
+        // one would slow (21 GB: 6.22 ms, 6.90 with one, 6.34 whole; 109 GB:
+        // 27.6, 39.3, 27.4); two at order 14 and below (8 GB: 2.93, 3.37 with
+        // one, 3.14 whole). Whole: order 39, where a workgroup of P2M takes
+        // a whole CU (2.15, limited 2.31), several sets, whose far fields
+        // outweigh the replay (16 sets of 32,000 triangles: 16.0, limited
+        // 18.4), and no far field.
+        const bool beside = nrhs == 1 && oc && !near_only && T.nlev >= 2 && p <= 30;
+        const int per_cu = !beside ? 0 : p <= 14 ? 2 : store_words <= 2000000000 ? 1 : 3;
         auto run = [&](auto rk, int rb) {
             int ntask = (int)nf_chunk.size() / 2 * (ST_CHUNK / replay_pts(SL.ifsl + SL.ifdl, SL.fd, SL.fs, rb));
             for (int r0 = 0; r0 < nrhs; r0 += rb)
-                hipLaunchKernelGGL(rk, dim3(limit ? std::min(ntask, ds.cus) : ntask), dim3(NF_THREADS), 0, rs, n, src_eval, I(o_nfb), I(o_nfs),
+                hipLaunchKernelGGL(rk, dim3(per_cu ? std::min(ntask, per_cu * ds.cus) : ntask), dim3(NF_THREADS), 0, rs, n, src_eval, I(o_nfb), I(o_nfs),
                                    I(o_nfi), I(o_ss), I(o_sc), I(o_ts), (const int64_t *)(P + o_sbase), I(o_ntri),
                                    I(o_pst), I(o_nfc), ntask, d0 + r0 * dstr, d1 + r0 * dstr, dstr, std::min(rb, nrhs - r0),
                                    store->data.get<double>(), out + r0 * nstr, nstr);
