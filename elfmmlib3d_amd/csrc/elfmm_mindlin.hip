@@ -530,9 +530,7 @@ __global__ __launch_bounds__(MW) void k_mind_bmod(MindArgs a, MindPw pw, const i
     harm_regular(p, radius * st, 0.0, -radius * ct, A[1]);
     __syncthreads();
     // remainder of B (scaled proxies' multipole subtracted), dz^-2, scale
-    for (int k = 0; k < 2; k++) {
-        int idx = threadIdx.x + k * MW;
-        if (idx >= nown) break;
+    for (int idx = threadIdx.x; idx < nown; idx += MW) {
         int l = 0;
         while ((l + 1) * (l + 2) / 2 <= idx) l++;
         int m = idx - l * (l + 1) / 2;
@@ -547,9 +545,7 @@ __global__ __launch_bounds__(MW) void k_mind_bmod(MindArgs a, MindPw pw, const i
         H[idx] = make_double2(Mb[2 * idx] - mp.x * sc, Mb[2 * idx + 1] - mp.y * sc);
     }
     __syncthreads();
-    for (int k = 0; k < 2; k++) {
-        int idx = threadIdx.x + k * MW;
-        if (idx >= nown) break;
+    for (int idx = threadIdx.x; idx < nown; idx += MW) {
         int l = 0;
         while ((l + 1) * (l + 2) / 2 <= idx) l++;
         int m = idx - l * (l + 1) / 2;
