@@ -2277,6 +2277,7 @@ struct Workspace {
     std::unique_ptr<OctreeWork> oct;                 // device octree buffers
     Plan planh;
     Tree treeh;
+    std::vector<int> near_waves;
     PinnedBuf stage, part_stage[3];   // plan staging; the call that filled them has completed before reuse
     hipStream_t near_stream = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_done = nullptr;
@@ -2365,7 +2366,8 @@ int max_lds()
 // buffer of its part (FarLaunch), which may be one and the same.
 struct PlanOffsets {
     size_t iz, izt, cen, side, ss, sc, ts, tc, p2m, p2mp, p2lb, p2ls, p2li, l2t, l2tp, m2tsb, m2tp, l2tw, m2tw, m2tbt;
-    size_t nfb, nfs, nfi, nfw, m2lt;
+    size_t nfb, nfs, nfi, m2lt;
+    size_t nfw, near_waves = 0;                      // near_tasks, where the near field is integrated
     std::vector<LaunchOff> m2m, l2l;
     LaunchOff m2l;
 };
@@ -2383,7 +2385,12 @@ void pack_near(Packer &pk, const Tree &T, const Plan &PL, PlanOffsets &o)
     o.nfb = pk.add(PL.nf_boxes);
     o.nfs = pk.add(PL.nf_start);
     o.nfi = pk.add(PL.nf_items);
-    o.nfw = pk.add(PL.nf_tasks);
+}
+
+void pack_near_tasks(Packer &pk, const std::vector<int> &tasks, PlanOffsets &o)
+{
+    o.nfw = pk.add(tasks);
+    o.near_waves = tasks.size() / 3;
 }
 
 LaunchOff pack_launch(Packer &pk, const GemmLaunch &g)
@@ -2995,8 +3002,13 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
     } else {
         pack_plan(pk, T, PL, po);
     }
+    // no store, no half space, a layer: the near field is integrated (k_near)
+    if (!direct_only && !half && !store && (ifsl || ifdl)) {
+        near_tasks(T, PL, src_eval, W.near_waves);
+        pack_near_tasks(pk, W.near_waves, po);
+    }
     const size_t o_iz = po.iz, o_izt = po.izt, o_ss = po.ss, o_sc = po.sc, o_ts = po.ts, o_tc = po.tc;
-    const size_t o_nfb = po.nfb, o_nfs = po.nfs, o_nfi = po.nfi, o_nfw = po.nfw;
+    const size_t o_nfb = po.nfb, o_nfs = po.nfs, o_nfi = po.nfi;
     size_t o_sbase = pk.add(nf_sbase), o_ntri = pk.add(nf_ntri), o_pst = pk.add(nf_pstart);
     size_t o_nfc = pk.add(nf_chunk);
     size_t o_htb = pk.add(h_tb), o_htbase = pk.add(h_tbase);
@@ -3142,9 +3154,9 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
                            W.nf.get<double>());
     } else if (!nf_boxes.empty() && store && icomp == 3) {
         HIPOK(run_replay(ns));
-    } else if (!PL.nf_tasks.empty() && (ifsl || ifdl)) {   // no layer: the near field stays zero
-        hipLaunchKernelGGL(near_kernel(ifsl, ifdl, ifst || ifstt), dim3(PL.nf_tasks.size() / 3), dim3(64), 0, ns, n,
-                           src_eval, I(o_nfb), I(o_nfs), I(o_nfi), I(o_ss), I(o_sc), I(o_ts), I(o_tc), I(o_nfw),
+    } else if (po.near_waves) {                      // no layer: the near field stays zero
+        hipLaunchKernelGGL(near_kernel(ifsl, ifdl, ifst || ifstt), dim3(po.near_waves), dim3(64), 0, ns, n,
+                           src_eval, I(o_nfb), I(o_nfs), I(o_nfi), I(o_ss), I(o_sc), I(o_ts), I(o_tc), I(po.nfw),
                            W.pts.get<double>(), W.rec.get<double>(), rlam, rmu, c1, W.nf.get<double>());
     }
     HIPOK(hipGetLastError());
@@ -4116,10 +4128,10 @@ void batch_enqueue_view(Batch &B, const BatchView &V, Lane &f, Lane &q)
              B.ifdl, B.ifdl ? (const double *)(B.sdl + 3 * V.off) : none,
              nt ? (const double *)(B.tgt + 3 * V.offt) : none, tri_s, nrm_s, ssl_s, sdl_s, V.pts, V.rec);
     f.fill0(V.nf, (size_t)np * 9);
-    bool near = !V.PL->nf_tasks.empty() && (B.ifsl || B.ifdl);
+    bool near = po.near_waves && (B.ifsl || B.ifdl);
     if (near) {
         q.after(f);
-        q.launch(near_kernel(B.ifsl, B.ifdl, B.ifst || B.ifstt), dim3(V.PL->nf_tasks.size() / 3), dim3(64), 0, n,
+        q.launch(near_kernel(B.ifsl, B.ifdl, B.ifst || B.ifstt), dim3(po.near_waves), dim3(64), 0, n,
                  B.src_eval, I(po.nfb), I(po.nfs), I(po.nfi), I(po.ss), I(po.sc), I(po.ts), I(po.tc), I(po.nfw),
                  (const double *)V.pts, (const double *)V.rec, B.rlam, B.rmu, c1, V.nf);
     }
@@ -4386,6 +4398,7 @@ int batch_create(int iprec, double rlam, double rmu, int nmesh, const int *npart
     if (nG) HIPOK(hipMemcpy(ht.data(), d_tgt, 3 * nG * 8, hipMemcpyDeviceToHost));
     // per mesh: octree, task lists, the packed plan and the tree-order buffers
     const OpsCache &oc = *B->oc;
+    std::vector<int> waves;
     for (int m = 0; m < nmesh; m++) {
         auto M = std::make_unique<BatchMesh>();
         M->n = nparts[m];
@@ -4407,6 +4420,8 @@ int batch_create(int iprec, double rlam, double rmu, int nmesh, const int *npart
         M->cost = 2400.0 * st[6] + (M->usefar ? st[4] : 0.0) + 2.0e4 * np + 1.0e9;
         Packer pk;
         pack_plan(pk, M->T, M->PL, M->po);
+        near_tasks(M->T, M->PL, B->src_eval != 0, waves);
+        pack_near_tasks(pk, waves, M->po);
         std::vector<char> stage(pk.size);
         pk.pack(stage.data());
         M->plan.ensure(pk.size);
@@ -4435,6 +4450,8 @@ int batch_create(int iprec, double rlam, double rmu, int nmesh, const int *npart
         F.usefar = F.T.nlev >= 2;
         Packer pk;
         pack_plan(pk, F.T, F.PL, F.po);
+        near_tasks(F.T, F.PL, B->src_eval != 0, waves);
+        pack_near_tasks(pk, waves, F.po);
         std::vector<char> stage(pk.size);
         pk.pack(stage.data());
         F.plan.ensure(pk.size);

@@ -163,7 +163,7 @@ struct Plan {
     std::vector<int> p2l_boxes, p2l_start, p2l_items;   // box <- sources of its list-4 boxes
     std::vector<int> m2t_items;                      // boxes taking the multipole of each m2t slot, slot after slot
     std::vector<int> l2t_boxes, nf_boxes, nf_start, nf_items;
-    std::vector<int> nf_tasks;                       // near-field waves: (near box, first lane, lanes per point)
+    std::vector<int> nf_ntri;                        // triangles of each near box's list
     std::vector<int> l2t_tpt;                        // points of each l2t slot, slot after slot
     std::vector<int> m2t_slot_box, m2t_tpt;          // points of each m2t slot, slot after slot
     // evaluation wave tasks: (slot, first task, task count <= EW_PTS) triples
@@ -192,6 +192,10 @@ void build_plan(const Tree &T, int n, const Operators *ops, bool src_eval, bool 
 // build_plan_eval L2T and M2T. None clears what another fills (P starts from
 // plan_reset).
 void build_plan_near(const Tree &T, bool src_eval, bool direct_only, bool iter, Plan &P);
+// The waves of the near field of triangles over P's near lists: (near box,
+// first (point, lane) pair, lanes per point). Only for calls that integrate
+// the near field as they go: stored products and points have tasks of their own.
+void near_tasks(const Tree &T, const Plan &P, bool src_eval, std::vector<int> &tasks);
 // Empties P for a new plan (zero stats), keeping its arrays' memory; the M2L
 // pair arrays keep their length too, which the next build_plan_m2l resizes and
 // overwrites (no clearing of the largest arrays per apply).

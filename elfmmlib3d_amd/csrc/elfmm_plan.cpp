@@ -141,40 +141,6 @@ void wave_tasks(const std::vector<I> &off, std::vector<int> &wt)
         }
 }
 
-// Waves of the near field: lanes per point of each near box, the power of two
-// that costs the box the least time, waves x (steps per wave + 1): the last
-// step and the last wave of a box run partly idle, and setting a wave up and
-// adding its lanes costs about a step (20 points, 135 triangles: 2 waves x 35
-// at 4 lanes, 3 x 18 at 8, 5 x 10 at 16, 10 x 6 at 32). A call too small to
-// give the device NF_WAVES waves that way starts from more lanes per point:
-// 217 points against 180 triangles took 205 us as one workgroup per leaf.
-template <class NP>
-void near_tasks(Plan &P, const std::vector<int> &ntri, NP &&npts, double npt)
-{
-    constexpr int NF_WAVES = 2048;                   // 256 CUs x 4 SIMDs x 2
-    int low = 0;                                     // log2 of the lanes per point
-    while (low < 6 && npt * (1 << low) < NF_WAVES * 64.0) low++;
-    int nq = (int)P.nf_boxes.size();
-    std::vector<int> start(nq + 1, 0);
-    std::vector<unsigned char> lanes(nq);
-    for (int q = 0; q < nq; q++) {
-        int64_t np = npts(P.nf_boxes[q]), cost = 0;
-        for (int k = low; k <= 6; k++) {
-            int64_t c = (((np << k) + 63) >> 6) * (((ntri[q] + (1 << k) - 1) >> k) + 1);
-            if (!cost || c < cost) lanes[q] = (unsigned char)k, cost = c;
-        }
-        start[q + 1] = start[q] + (int)(((np << lanes[q]) + 63) >> 6);
-    }
-    P.nf_tasks.resize(3 * (size_t)start[nq]);
-    for (int q = 0; q < nq; q++)
-        for (int k = 0; k < start[q + 1] - start[q]; k++) {
-            int *t = &P.nf_tasks[3 * (size_t)(start[q] + k)];
-            t[0] = q;
-            t[1] = 64 * k;
-            t[2] = 1 << lanes[q];
-        }
-}
-
 // P2M workgroups: a box's triangles are a chain of chunks of 8 to 12, so where
 // the boxes are too few to fill the device (iter leaves hold up to 240
 // triangles) they are cut into equal parts, about P2M_WG of them, none under
@@ -216,7 +182,7 @@ void build_plan_near(const Tree &T, bool src_eval, bool direct_only, bool iter, 
     P.nf_boxes.clear();
     P.nf_start.assign(1, 0);
     P.nf_items.clear();
-    P.nf_tasks.clear();
+    P.nf_ntri.clear();
     P.stats[6] = 0;
     if (direct_only) return;
     // leaves: near field over self + list 1. With iter, lists 3 and 4 join
@@ -257,14 +223,13 @@ void build_plan_near(const Tree &T, bool src_eval, bool direct_only, bool iter, 
     int nq = (int)box.size();
     P.nf_boxes.resize(nq);
     P.nf_start.resize(nq + 1);
-    std::vector<int> ntri(nq);
-    double npair_near = 0, npt_near = 0;
+    P.nf_ntri.resize(nq);
+    double npair_near = 0;
     for (int q = 0; q < nq; q++) {
         int b = P.nf_boxes[q] = box[ord[q]];
         P.nf_start[q + 1] = P.nf_start[q] + items[b];
-        ntri[q] = tris[b];
+        P.nf_ntri[q] = tris[b];
         npair_near += w[ord[q]];
-        npt_near += npts(b);
     }
     P.nf_items.resize(P.nf_start[nq]);
     parallel_chunks((nq + CHUNK - 1) / CHUNK, [&](int ch, int) {
@@ -274,13 +239,48 @@ void build_plan_near(const Tree &T, bool src_eval, bool direct_only, bool iter, 
         }
     });
     P.stats[6] = npair_near;
-    near_tasks(P, ntri, npts, npt_near);
+}
+
+// Lanes per point of each near box: the power of two that costs the box the
+// least time, waves x (steps per wave + 1): the last step and the last wave
+// of a box run partly idle, and setting a wave up and adding its lanes costs
+// about a step (20 points, 135 triangles: 2 waves x 35 at 4 lanes, 3 x 18 at
+// 8, 5 x 10 at 16, 10 x 6 at 32). A call too small to give the device
+// NF_WAVES waves that way starts from more lanes per point: 217 points
+// against 180 triangles took 205 us as one workgroup per leaf.
+void near_tasks(const Tree &T, const Plan &P, bool src_eval, std::vector<int> &tasks)
+{
+    constexpr int NF_WAVES = 2048;                   // 256 CUs x 4 SIMDs x 2
+    auto npts = [&](int b) { return (src_eval ? T.src_count[b] : 0) + T.tgt_count[b]; };
+    int nq = (int)P.nf_boxes.size();
+    double total = 0;
+    for (int b : P.nf_boxes) total += npts(b);
+    int low = 0;                                     // log2 of the lanes per point
+    while (low < 6 && total * (1 << low) < NF_WAVES * 64.0) low++;
+    std::vector<int> start(nq + 1, 0);
+    std::vector<unsigned char> lanes(nq);
+    for (int q = 0; q < nq; q++) {
+        int64_t np = npts(P.nf_boxes[q]), cost = 0;
+        for (int k = low; k <= 6; k++) {
+            int64_t c = (((np << k) + 63) >> 6) * (((P.nf_ntri[q] + (1 << k) - 1) >> k) + 1);
+            if (!cost || c < cost) lanes[q] = (unsigned char)k, cost = c;
+        }
+        start[q + 1] = start[q] + (int)(((np << lanes[q]) + 63) >> 6);
+    }
+    tasks.resize(3 * (size_t)start[nq]);
+    for (int q = 0; q < nq; q++)
+        for (int k = 0; k < start[q + 1] - start[q]; k++) {
+            int *t = &tasks[3 * (size_t)(start[q] + k)];
+            t[0] = q;
+            t[1] = 64 * k;
+            t[2] = 1 << lanes[q];
+        }
 }
 
 void plan_reset(Plan &P)
 {
     for (std::vector<int> *v : {&P.p2m_boxes, &P.p2m_parts, &P.p2l_boxes, &P.p2l_start, &P.p2l_items, &P.m2t_items, &P.l2t_boxes,
-                                &P.nf_boxes, &P.nf_start, &P.nf_items, &P.nf_tasks, &P.l2t_tpt, &P.m2t_slot_box,
+                                &P.nf_boxes, &P.nf_start, &P.nf_items, &P.nf_ntri, &P.l2t_tpt, &P.m2t_slot_box,
                                 &P.m2t_tpt, &P.l2t_wt, &P.m2t_wt, &P.m2t_bt})
         v->clear();
     P.sides.clear();
