@@ -113,9 +113,6 @@ typedef double gemm_d4 __attribute__((ext_vector_type(4)));
 
 #include "elfmm_moments.h"
 
-__device__ __forceinline__ int hidx(int l, int m) { return l * (l + 1) / 2 + m; }
-
-
 // order m of packed coefficient index c = l*(l+1)/2 + m (c < 2^20), from
 // a float square root and one correction each way: no table load
 __device__ __forceinline__ int coef_m(int c)
@@ -2113,7 +2110,6 @@ struct DeviceState {
     bool tables = false;
     int cus = 256;                                   // compute units
     bool p2x_wide = false;                           // 16-wave P2M/P2L for orders above 26
-    bool p2t = false;                                // P2M/P2L through triangle moments (156 KB of LDS per CU)
     std::map<int, std::unique_ptr<OpsCache>> ops;   // by iprec
 };
 
@@ -2154,21 +2150,20 @@ DeviceState &device_state()
                 hipSuccess &&
             hipFuncSetAttribute((const void *)k_p2l<16, 7, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, wide) ==
                 hipSuccess;
-        auto lds_ok = [](auto z) {
+        (void)hipGetLastError();                     // a refused size leaves the narrow shape in use
+        auto tri_lds = [](auto z) {                  // 154 KB for the largest shape
             using Z = decltype(z);
             int ph = 0;
             while (Z::fits(ph + 1)) ph++;
             int b = Z::lds(ph) * 8;
-            return hipFuncSetAttribute((const void *)k_p2m_tri<Z, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       b) == hipSuccess &&
-                   hipFuncSetAttribute((const void *)k_p2m_tri<Z, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       b) == hipSuccess &&
-                   hipFuncSetAttribute((const void *)k_p2l_tri<Z>, hipFuncAttributeMaxDynamicSharedMemorySize, b) ==
-                       hipSuccess;
+            for (const void *k : {(const void *)k_p2m_tri<Z, false>, (const void *)k_p2m_tri<Z, true>, (const void *)k_p2l_tri<Z>})
+                HIPOK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, b));
         };
+        tri_lds(P2TShape0{});
+        tri_lds(P2TShape1{});
+        tri_lds(P2TShape2{});
+        tri_lds(P2TShape3{});
         HIPOK(hipDeviceGetAttribute(&ds->cus, hipDeviceAttributeMultiprocessorCount, dev));
-        ds->p2t = lds_ok(P2TShape0{}) && lds_ok(P2TShape1{}) && lds_ok(P2TShape2{}) && lds_ok(P2TShape3{});
-        (void)hipGetLastError();                     // a refused size leaves the narrow shape, or the node products, in use
         ds->tables = true;
     }
     return *ds;
@@ -2529,10 +2524,9 @@ void enqueue_up(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
     mark(2, true);
     ln.fill0(a.exps, (size_t)2 * a.nb * NRHS * nc);
     ln.fill0(a.lap, np * 40);
-    // triangles with 6 or 12 nodes go through three moments each, where the
-    // device gives the LDS that takes; rules of 1 and 3 nodes and point sources
-    // through one product per node
-    const bool tri = !a.points && a.ds->p2t && p2t_shape(p, nq) >= 0 && p2t_shape(p + 1, nq) >= 0;
+    // triangles with 6 or 12 nodes go through three moments each; rules of 1 and
+    // 3 nodes and point sources through one product per node
+    const bool tri = !a.points && nq >= 6;
     if (tri)
         ln.launch(k_tcoef, dim3((n + 255) / 256), dim3(256), 0, n, a.tri_s, a.nrm_s, a.ssl, a.sdl, a.ifsl, a.ifdl,
                   a.mu, a.c1, a.c2, a.dls, a.nodes);
@@ -2566,12 +2560,13 @@ void enqueue_up(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
                   sc, (const double *)a.nodes, nc, out);
     };
     auto p2 = [&](bool irr, size_t nbx, const int *bx, const int *ls, const int *li, double *out) {
-        switch (tri ? p2t_shape(irr ? p + 1 : p, nq) : -1) {
+        if (!tri) return p2x(irr, nbx, bx, ls, li, out);
+        switch (p2t_shape(irr ? p + 1 : p, nq)) {
         case 0: return p2t(P2TShape0{}, irr, nbx, bx, ls, li, out);
         case 1: return p2t(P2TShape1{}, irr, nbx, bx, ls, li, out);
         case 2: return p2t(P2TShape2{}, irr, nbx, bx, ls, li, out);
         case 3: return p2t(P2TShape3{}, irr, nbx, bx, ls, li, out);
-        default: return p2x(irr, nbx, bx, ls, li, out);
+        default: HIPOK(hipErrorInvalidValue);
         }
     };
     if (!PL.p2m_boxes.empty()) p2(false, PL.p2m_boxes.size(), I(o.p2m), nullptr, nullptr, mp);
@@ -3777,7 +3772,7 @@ int mindlin_far_dev(int iprec, double rlam, double rmu, int n, const double *d_t
     char *tb = oc->mind_tab.get<char>();
     MindDev md;
     md.args = MindArgs{p, ifsl, ifdl, rlam, rmu, T.size, I(M.o_lev), I(M.o_ss), I(M.o_sc), D(M.o_cen), tri_s, nrm_s,
-                       ssl_s, sdl_s, nc, mp, lo, iprec >= 1 ? 6 : iprec == 0 ? 4 : 2};
+                       ssl_s, sdl_s, nc, mp, lo};
     md.pw = oc->mind_pw;
     md.slot = I(M.o_slot);
     md.ycst = (const double *)(tb + oc->mind_off[0]);
@@ -3791,8 +3786,9 @@ int mindlin_far_dev(int iprec, double rlam, double rmu, int n, const double *d_t
     md.gmom = S.gm.get<double>();
     // upward pass
     const int nbx = (int)PL.p2m_boxes.size(), nown = nc / 2;
-    const int nqn = iprec >= 1 ? 12 : iprec == 0 ? 6 : 3, shape = dsp->p2t ? p2t_shape(p, nqn) : -1;
-    if (nbx && shape >= 0) {
+    if (nbx && iprec >= 0) {
+        const int shape = p2t_shape(p, iprec >= 1 ? 12 : 6);
+        if (shape < 0) HIPOK(hipErrorInvalidValue);
         // triangle moments (elfmm_moments.h), one layer at a time: 6 or 12 columns
         HIPOK(launch_fill0(S.gm.get<double>(), (size_t)2 * nbx * MindMoments::MCOLS * nown, stream));
         S.tcoef.ensure((size_t)48 * n * 8);

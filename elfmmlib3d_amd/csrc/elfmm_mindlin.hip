@@ -19,11 +19,9 @@ constexpr int MW = 256;                      // threads per workgroup
 constexpr int MP_MAX = 39;                   // largest supported order (iprec 3)
 constexpr int MH = (MP_MAX + 1) * (MP_MAX + 2) / 2;
 constexpr int MPW_FOUR = 544;                // Fourier modes of the largest plane-wave table (525)
-constexpr size_t MIND_P2M_LDS = 100 * 1024;   // LDS and threads of the P2M moment pass
-constexpr int MIND_P2M_NT = 512;
+constexpr int MIND_P2M_NT = 512, MIND_P2M_NODES = 32;   // threads and nodes at a time of the P2M moment pass
 
-// rows 0-2: order 2, rows 3-8: order 4, rows 9-20: order 6
-__constant__ double c_mrule[21][3] = {ELFMM_RULE2, ELFMM_RULE4, ELFMM_RULE6};
+__constant__ double c_mrule[3][3] = {ELFMM_RULE2};
 
 // Regular harmonics R_l^m(x) (Racah normalisation, Condon-Shortley phase)
 // of one point for l <= L, 0 <= m <= l, into H[pk(l, m)] (re, im): thread m
@@ -91,10 +89,9 @@ __device__ __forceinline__ double lmn(int l, int m)
 // P2M of B, C1, C2 (l3dtriaformmp_mindlinb_trunc / _mindlinc_trunc,
 // src/mindlinformmptri.f:305, :449 with formmp_mindlinb_trunc
 // src/mindlinbformmp.f and formmp_mindlinc_trunc src/mindlincformmp.f) from
-// the nodes of the order-nqtri rule on a leaf's (mirrored) triangles (order
-// 6 from iprec 1 up, 4 at iprec 0, 2 below,
-// src/lfmm3dtriamindlin_iter_1.f:679-693), densities times weight * 2 *
-// area. Every charge, dipole and quadrupole strength the three expansions
+// the nodes of a rule on a leaf's (mirrored) triangles (order 6 from iprec 1
+// up, 4 at iprec 0, 2 below, src/lfmm3dtriamindlin_iter_1.f:679-693),
+// densities times weight * 2 * area. Every charge, dipole and quadrupole strength the three expansions
 // take at a node is a fixed combination of 18 real columns:
 //   0-2 sigma_sl, 3-5 y3 sigma_sl, 6-11 q, 12-17 y3 q,
 // q = (b1 n1, b2 n2, b3 n3, b1 n2 + b2 n1, b1 n3 + b3 n1, b2 n3 + b3 n2)
@@ -109,13 +106,14 @@ constexpr int MCOLS = 18;
 // elfmm_moments.h): one workgroup per box, thread = coefficient (l, m). The columns
 // are per-triangle values times per-node factors: a triangle's moments are
 // its 9 values (sigma_sl, q) times U = sum_nodes w R(x) and U' = sum_nodes
-// w y3 R(x), w = rule weight * 2 * area. Nodes go through LDS nch at a time
+// w y3 R(x), w = rule weight * 2 * area. Nodes go through LDS 32 at a time
 // (their harmonics by column recurrences with the constants tabulated in
 // LDS); each thread folds a finished triangle into its 18 moments.
 // MIND_P2M_NT >= (p+1)(p+2)/2.
-__global__ __launch_bounds__(MIND_P2M_NT) void k_mind_moments(MindArgs a, const int *__restrict__ boxes, int nch,
+__global__ __launch_bounds__(MIND_P2M_NT) void k_mind_moments(MindArgs a, const int *__restrict__ boxes,
                                                      double2 *__restrict__ G)
 {
+    constexpr int nch = MIND_P2M_NODES;
     extern __shared__ double smem[];
     int p = a.p, nown = (p + 1) * (p + 2) / 2;
     double2 *Hs = (double2 *)smem;                          // [nch][nown] harmonics
@@ -143,10 +141,8 @@ __global__ __launch_bounds__(MIND_P2M_NT) void k_mind_moments(MindArgs a, const 
     for (int k = tid; k <= p; k += MIND_P2M_NT) Dg[k] = k ? sqrt((2.0 * k - 1) / (2.0 * k)) : 1.0;
     int b = boxes[blockIdx.x];
     const double *c = a.centers + 3 * (size_t)b;
-    int q0 = a.nqtri == 2 ? 0 : a.nqtri == 4 ? 3 : 9, q1 = a.nqtri == 2 ? 3 : a.nqtri == 4 ? 9 : 21;
-    int nqn = q1 - q0;
     int s0 = a.src_start[b];
-    int K = a.src_count[b] * nqn;
+    int K = a.src_count[b] * 3;
     double2 g[MCOLS];
 #pragma unroll
     for (int j = 0; j < MCOLS; j++) g[j] = make_double2(0.0, 0.0);
@@ -175,7 +171,7 @@ __global__ __launch_bounds__(MIND_P2M_NT) void k_mind_moments(MindArgs a, const 
         int nk = min(nch, K - k0);
         __syncthreads();
         if (tid < nk) {
-            int tl = (k0 + tid) / nqn, qn = q0 + (k0 + tid) % nqn, ti = s0 + tl;
+            int tl = (k0 + tid) / 3, qn = (k0 + tid) % 3, ti = s0 + tl;
             const double *t = a.tri + 9 * (size_t)ti;
             double ax = t[3] - t[0], ay = t[4] - t[1], az = t[5] - t[2];
             double bx = t[6] - t[0], by = t[7] - t[1], bz = t[8] - t[2];
@@ -814,21 +810,6 @@ __global__ void k_mind_assemble(int n, int nt, const int *__restrict__ izt, cons
 
 // ---- launchers ----
 
-// LDS of the moment pass: nch nodes of (harmonics, 2 weights, 9 triangle
-// values, 3 coordinates, triangle index) and the recurrence tables
-size_t mind_p2m_lds(int p, int nch)
-{
-    size_t nown = (size_t)(p + 1) * (p + 2) / 2;
-    return (size_t)nch * (nown * 16 + (2 + 9 + 3) * 8 + 4) + nown * 16 + (size_t)(p + 1) * 8;
-}
-
-size_t mind_p2m_nch(int p)
-{
-    size_t nown = (size_t)(p + 1) * (p + 2) / 2, per = nown * 16 + (2 + 9 + 3) * 8 + 4;
-    size_t fixed = nown * 16 + (size_t)(p + 1) * 8;
-    return std::min<size_t>(32, (MIND_P2M_LDS - fixed) / per);
-}
-
 size_t mind_p2m_scratch_bytes(int p, int nbx)
 {
     return (size_t)nbx * MCOLS * ((size_t)(p + 1) * (p + 2) / 2) * 16;
@@ -839,10 +820,11 @@ hipError_t launch_mind_p2m(const MindDev &d, const int *boxes, int nbx, hipStrea
     if (nbx <= 0) return hipSuccess;
     const MindArgs &a = d.args;
     int nown = (a.p + 1) * (a.p + 2) / 2;
-    int nch = (int)mind_p2m_nch(a.p);
-    size_t sh = mind_p2m_lds(a.p, nch);
-    if (nown > MIND_P2M_NT) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_mind_moments, dim3(nbx), dim3(MIND_P2M_NT), sh, st, a, boxes, nch, (double2 *)d.gmom);
+    // the nodes' harmonics, 2 weights, 9 triangle values, 3 coordinates and
+    // triangle index, and the recurrence tables
+    size_t sh = (size_t)MIND_P2M_NODES * (nown * 16 + (2 + 9 + 3) * 8 + 4) + nown * 16 + (size_t)(a.p + 1) * 8;
+    if (nown > MIND_P2M_NT || sh > 64 * 1024) return hipErrorInvalidValue;   // order 9 and below
+    hipLaunchKernelGGL(k_mind_moments, dim3(nbx), dim3(MIND_P2M_NT), sh, st, a, boxes, (double2 *)d.gmom);
     hipError_t e = hipGetLastError();
     return e != hipSuccess ? e : launch_mind_combine(d, boxes, nbx, st);
 }
@@ -920,8 +902,6 @@ size_t mind_far_lds(int nexptotp, int nexptot) { return (size_t)3 * (nexptotp + 
 void mind_set_lds_limits(size_t far)
 {
     (void)hipFuncSetAttribute((const void *)k_mind_far, hipFuncAttributeMaxDynamicSharedMemorySize, (int)far);
-    (void)hipFuncSetAttribute((const void *)k_mind_moments, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)MIND_P2M_LDS);
     (void)hipGetLastError();
 }
 

@@ -171,6 +171,7 @@ using P2TShape0 = P2TShape<2, 4, 4, 6, 3>;
 using P2TShape1 = P2TShape<2, 4, 5, 8, 6>;
 using P2TShape2 = P2TShape<4, 4, 8, 14, 6>;
 using P2TShape3 = P2TShape<8, 3, 14, 21, 6>;
+static_assert(P2TShape0::fits(10) && P2TShape1::fits(15) && P2TShape2::fits(27) && P2TShape3::fits(40), "P2L's degrees");
 // The shape for degree ph and nq nodes, -1 if none fits.
 inline int p2t_shape(int ph, int nq)
 {

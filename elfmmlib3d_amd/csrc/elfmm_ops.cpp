@@ -46,30 +46,6 @@ struct Harm {
     }
 };
 
-Harm regular(int p, double x, double y, double z)
-{
-    Harm h{p, std::vector<cd>((p + 1) * (p + 2) / 2)};
-    double r2 = x * x + y * y + z * z;
-    cd diag = 1.0;
-    for (int m = 0; m <= p; m++) {
-        if (m > 0) diag = -cd(x, y) * std::sqrt((2.0 * m - 1) / (2.0 * m)) * diag;
-        cd a = diag, b = 0.0;
-        h.v[m * (m + 1) / 2 + m] = a;
-        if (m + 1 <= p) {
-            b = std::sqrt(2.0 * m + 1) * z * a;
-            h.v[(m + 1) * (m + 2) / 2 + m] = b;
-        }
-        for (int l = m + 2; l <= p; l++) {
-            cd c = ((2.0 * l - 1) * z * b - std::sqrt((l - 1.0 + m) * (l - 1.0 - m)) * r2 * a) /
-                   std::sqrt((l + m) * (double)(l - m));
-            h.v[l * (l + 1) / 2 + m] = c;
-            a = b;
-            b = c;
-        }
-    }
-    return h;
-}
-
 Harm irregular(int p, double x, double y, double z)
 {
     Harm h{p, std::vector<cd>((p + 1) * (p + 2) / 2)};
