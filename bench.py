@@ -163,7 +163,7 @@ def measure_traffic(args):
                 return None, f"no device copy in the {counter} pass"
             factors[counter] = (CALIB_MIB << 20) / (max(copies) * 1024.0)
             for name, vs in per.items():
-                short = name.split("(")[0].split("::")[-1].split("<")[0]
+                short = name.split("(")[0].split("<")[0].split("::")[-1]
                 kib.setdefault(short, {})[counter] = float(np.mean(vs))
     traffic = {k: v.get("FETCH_SIZE", 0.0) * 1024 * factors["FETCH_SIZE"] +
                v.get("WRITE_SIZE", 0.0) * 1024 * factors["WRITE_SIZE"] for k, v in kib.items()
@@ -769,14 +769,13 @@ def main():
     #    count 2 R(p_t) + Z(p_t) (elfmm_gfx950_last_stats()[5])
     kernels = {k: kph[k] for k in ("p2m", "m2m", "m2l", "p2l", "l2l", "l2t", "m2t", "near")}
     work = {"near": (stats["near_pairs"] * NEAR_OPS_PER_PAIR, "k_near"),
-            "m2l": (stats["m2l_flops_alg"], "k_m2l")}
+            "m2l": (stats["m2l_flops_alg"], "k_m2l_turned + k_m2l")}   # higher and lower orders, a launch each
     rooflines = {}
     for k, (alg, name) in work.items():
         t = kernels[k] / 1e3
         rooflines[k] = {"kernel": name, "bound": "fp64", "achieved": alg / t / 1e12, "peak": PEAK_FP64 / 1e12,
                         "unit": "TFLOP/s", "frac": alg / t / PEAK_FP64, "traffic": None,
                         "algorithmic_flop_per_launch": alg, "ms_per_launch": kernels[k]}
-    rooflines["m2l"]["executed_tflops"] = stats["m2l_flops_dense"] / (kernels["m2l"] / 1e3) / 1e12
     dom = max(kernels, key=kernels.get)
     roof = rooflines.get(dom, {"kernel": dom, "bound": "fp64", "achieved": None, "peak": PEAK_FP64 / 1e12,
                                "unit": "TFLOP/s", "frac": None, "traffic": None,
@@ -784,8 +783,9 @@ def main():
     traffic, factors = measure_traffic(args) if args.traffic else (None, "not measured (--no-traffic)")
     if traffic:
         for r in list(rooflines.values()) + [roof]:
-            if r.get("kernel") in traffic:
-                r["traffic"] = traffic[r["kernel"]]
+            parts = r.get("kernel", "").split(" + ")
+            if all(k in traffic for k in parts):
+                r["traffic"] = sum(traffic[k] for k in parts)
 
     c3 = c3_half(args) if args.c3 else None
     c4 = c4_batched(args) if args.c4 else None
