@@ -1315,7 +1315,7 @@ constexpr int NF_THREADS = 256;
 // code: elfmm_near.h). 81,920 triangles + 100,000 targets, iprec 2 (25.0e6
 // pairs, both layers, strain): 4.25 ms with two passes over the edges
 // and a 256-thread workgroup per leaf whose lanes idled in boxes of fewer
-// triangles than lanes per point, 1.23 ms in this form; 217 points against 180
+// triangles than lanes per point, 1.32 ms in this form; 217 points against 180
 // triangles: 0.23 and 0.014 ms.
 template <bool SL, bool DL, bool ST>
 __global__ __launch_bounds__(64) void k_near(
@@ -2470,10 +2470,6 @@ void far_scratch(int iprec, int n, int np, int nb, int p, size_t &nodes, size_t 
     lap = (size_t)np * 40;
 }
 
-// Enqueues the far field on one stream with kernel launches only (no
-// memsets, copies or host waits), so that it can be captured into a graph.
-// mark(k, begin), when given, brackets phase k (2 nodes and P2M, 3 M2M, 4
-// M2L, 5 P2L, 6 L2L, 7 L2T, 8 M2T) for the caller's timing events.
 // M2M / L2L of one level (unit scale)
 void enqueue_trans(const GemmLaunch &g, const LaunchOff &l, const char *P, const DevBuf &A, const double *X, double *Y,
                    int nc, Lane &ln)
@@ -2631,6 +2627,10 @@ void enqueue_eval(const FarLaunch &a, Lane &ln, Mark mark)
     mark(8, false);
 }
 
+// Enqueues the far field on one stream with kernel launches only (no
+// memsets, copies or host waits), so that it can be captured into a graph.
+// mark(k, begin) brackets phase k (2 nodes and P2M, 3 M2M, 4 M2L, 5 P2L, 6
+// L2L, 7 L2T, 8 M2T) for the caller's timing events.
 template <class Mark>
 void enqueue_far(const FarLaunch &a, size_t np, Lane &ln, Mark mark)
 {
@@ -2676,8 +2676,10 @@ void run_far_parts(FarLaunch a, const Tree &T, Plan &PL, PlanOffsets &o, bool sr
 // the device is free: the device build is a chain of about 20 launches and a
 // round trip per level (0.34 ms for 217 points, 0.69 for 3,880, 0.82 for 9,200),
 // the host's costs about 0.02 us a point and 1 us a box (0.005, 0.43 and 1.0
-// ms for the same points at 40 to a leaf; 0.24 against 0.43 ms for 12,000 at 400
-// to a leaf).
+// ms for the same points at 40 to a leaf). With larger leaves the boxes are
+// fewer (host and device, ms: 12,000 points at 400 to a leaf 0.26 and 0.46,
+// 20,000 0.36 and 0.51; 20,000 in a cluster of many levels 1.29 and 1.69; 14,580
+// at 240 0.42 and 0.60).
 bool small_tree(int np, int nbox) { return np <= 6000 || (np <= 20000 && np / 64 <= nbox); }
 
 // The apply: device pointers in, device pointers out.
@@ -3074,12 +3076,15 @@ int triatarg_dev(int iprec, double rlam, double rmu, int n, const double *d_tri,
         // One set beside its far field: a few workgroups per CU, each taking
         // every grid-th task, which leaves registers to the far field; launched
         // whole, the replay holds every CU and P2M, half a CU's registers a
-        // workgroup, waits for its end. One per CU where the replay is short
-        // (order 26, 14.5 GB: 3.59 ms a product, 3.98 with three, 4.12 whole; 9.8
-        // GB: 2.12, 2.42, 2.41); three where it outlasts the far field, which
-        // one would slow (21 GB: 6.22 ms, 6.90 with one, 6.34 whole; 109 GB:
-        // 27.6, 39.3, 27.4); two at order 14 and below (8 GB: 2.93, 3.37 with
-        // one, 3.14 whole). Whole: order 39, where a workgroup of P2M takes
+        // workgroup, waits for its end. By the bytes to read, at order 26 one per
+        // CU up to 16 GB (15.1 GB of both layers' displacements, 46,080 triangles:
+        // 3.71 ms a product, 4.04 with three, 4.24 whole; 9.7 GB of both layers
+        // with strain, 11,520 triangles: 2.20, 2.40, 2.46) and three above, where
+        // one reads too slowly (21 GB: 6.22 ms, 6.90 with one, 6.34 whole; 109 GB:
+        // 27.6, 39.3, 27.4; between 16 and 21 GB not measured). Two at order 14
+        // and below, whose far field is short (8 GB: 2.93, 3.37 with one, 3.14
+        // whole; 14.6 GB: 3.53, 3.62, 3.93; 44 GB: 8.81, 9.51, 8.62). Whole:
+        // order 39, where a workgroup of P2M takes
         // a whole CU (2.15, limited 2.31), several sets, whose far fields
         // outweigh the replay (16 sets of 32,000 triangles: 16.0, limited
         // 18.4), and no far field.

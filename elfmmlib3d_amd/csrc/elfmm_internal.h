@@ -83,7 +83,8 @@ constexpr size_t trans_doubles(int p) { return 5 * trans_blocks(p + 2); }
 // record's six products with their barriers cost more than the dense ones
 // (order 26, 303,000 pairs: 4.5 ms split between the orders 16 and 22,
 // all dense 5.3, all by records 5.8; order 39, 53,000 pairs, split between 23
-// and 24: 3.3 ms, all dense 3.7).
+// and 24: 3.5 ms, all dense 3.7). One line for each of the two orders that use M2L
+// orders above it (iprec 2 and 3): where the two measured equal.
 inline int m2l_turned_h(int p) { return p <= 26 ? 260 : 310; }
 
 // Translation operators on packed, box-size-scaled expansions.
@@ -138,8 +139,8 @@ struct M2LTile {
 };
 constexpr int ML_M = 64, ML_P = 32;
 
-// One launch of rotated translations (M2M or L2L of one level): pairs and
-// their tiles, run by the same kernel as M2L.
+// One launch of translations by records (M2M or L2L of one level): pairs and
+// their tiles. A record's workgroups deal a group's pairs among its row tiles.
 struct GemmLaunch {
     std::vector<M2LTile> tiles;
     std::vector<int> src, dst;
@@ -159,7 +160,7 @@ struct Plan {
     std::vector<int> p2m_parts;                      // P2M workgroups of triangles: (box of the list, first, triangles)
     std::vector<GemmLaunch> m2m_l, l2l_l;            // one launch per level
     GemmLaunch m2l;                                  // all list-2 pairs, grouped by offset (src/dst/scale)
-    std::vector<M2LTile> m2l_tiles;                  // rotated-M2L tiles over those pairs
+    std::vector<M2LTile> m2l_tiles;                  // M2L tiles over those pairs
     std::vector<int> p2l_boxes, p2l_start, p2l_items;   // box <- sources of its list-4 boxes
     std::vector<int> m2t_items;                      // boxes taking the multipole of each m2t slot, slot after slot
     std::vector<int> l2t_boxes, nf_boxes, nf_start, nf_items;

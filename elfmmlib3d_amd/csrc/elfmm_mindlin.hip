@@ -567,7 +567,8 @@ __global__ __launch_bounds__(MW) void k_mind_bmod(MindArgs a, MindPw pw, const i
 // kernel per pair instead (nquad^2 points x 2 nq charges, a square root and a
 // logarithm each, 281,000 at order 26) took 5.1 ms of the 20,020-triangle
 // fault mesh's product; the matrices take 0.11 ms there, and 1.3 ms
-// once per precision to build.
+// once per precision to build (120 offsets x 4p charges x (p+1)(p+2) doubles:
+// 75 MB at order 26, 246 MB at 39, kept with the precision's operators).
 
 // Matrix of one charge (blockIdx.x) and offset (blockIdx.y, source box minus
 // target box, in sides): op[offset][charge][2 coefficient + part].

@@ -429,8 +429,9 @@ void build_plan_m2l(const Tree &T, const Operators *ops, bool src_eval, int nrhs
                 }
             }
         });
-        // work counts: dense operator flops as executed and the reference's
-        // point-and-shoot count per pair and right-hand side, two rotations
+        // work counts: the flops of dense operators (what orders below
+        // m2l_turned_h execute) and the reference's point-and-shoot count per
+        // pair and right-hand side, two rotations
         // R(p) = 4 sum (2n+1)^2 and a z-shift Z(p) = 6 sum_j sum_k (p+1-|k|)
         std::vector<double> alg_m2l(p + 1, 0.0);
         for (int pt = 0; pt <= p; pt++) {

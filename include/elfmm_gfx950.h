@@ -355,9 +355,9 @@ void elfmm_gfx950_octree_get(int *boxes, double *centers, int *iz, int *iztarg, 
 void elfmm_gfx950_last_timings(double *ms16);
 
 /* Work counts of the last call on this thread: [0] boxes, [1] levels,
- * [2] expansion order p, [3] M2L pairs, [4] M2L flops as executed (dense
- * operators, four right-hand sides), [5] M2L flops of the reference's
- * rotate/shift/rotate scheme for the same pairs, [6] near-field (point,
+ * [2] expansion order p, [3] M2L pairs, [4] M2L flops of dense
+ * operators (four right-hand sides; the higher orders run fewer), [5] M2L
+ * flops of the reference's rotate/shift/rotate scheme for the same pairs, [6] near-field (point,
  * triangle) pairs, [7] M2L tiles, [8] M2M pairs, [9] L2L pairs, [10] P2M
  * boxes, [11] P2L (box, source box) pairs, [12] M2T (box, source box) pairs,
  * [13] L2T boxes, [14] iter: near-field store size in the reference's
